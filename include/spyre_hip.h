@@ -233,13 +233,19 @@ int sph_gemm_swiglu(sph_dtype dtype, int64_t m, int64_t n, int64_t k, const void
                     void* workspace, int64_t workspace_bytes, sph_stream_t stream);
 int64_t sph_gemm_swiglu_workspace_bytes(int64_t m, int64_t n, int64_t k);
 
+/* sph_gemm_swiglu for any m >= 1 and n >= 1 with k % 8 == 0 (16-byte aligned
+ * rows of A and W; D rows of any alignment): decode batches above 8 rows and
+ * ragged prompts.  The same workspace. */
+int sph_gemm_swiglu_any(sph_dtype dtype, int64_t m, int64_t n, int64_t k, const void* a,
+                        int64_t lda, const void* w, int64_t ldw, void* d, int64_t ldd,
+                        void* workspace, int64_t workspace_bytes, sph_stream_t stream);
+
 /* sph_gemm_strided_batched with a workspace (device memory, may be NULL):
  * with at least sph_gemm_workspace_bytes(batch, m, n, k) bytes, a product
- * on whole 256 x 256 tiles whose tile count leaves a partial last round on
- * the 256 CUs may split that round's tiles along K into fp32 partial tiles
- * (summed and finished with the epilogue by a second kernel) instead of
- * running it on a few CUs; the size is 0 for shapes where the library's
- * time model prefers whole rounds of 256- or 128-wide tiles.  Same results up to fp32 summation order.  No
+ * whose tiles would leave CUs idle (few rows, or a partial last round of 256
+ * x 256 tiles) may split its K range into fp32 partial tiles, summed and
+ * finished with the epilogue by a second kernel; the size is 0 for shapes
+ * where the library's time model prefers whole tiles.  Same results up to fp32 summation order.  No
  * counterpart in the reference (its GEMM is one device call,
  * spyre_torch_ops.cpp:214-293); calls sharing a workspace must be ordered
  * on a stream. */

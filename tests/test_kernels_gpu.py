@@ -634,6 +634,79 @@ def test_gemm_swiglu(m, n, k, pad, dtype):
         assert bool((d[:, n:] == 7.0).all()), "padding columns written"
 
 
+@pytest.mark.parametrize("batch,m,n,k,tb,pad,epi,dtype", [
+    (1, 9, 1024, 4096, 1, 0, 0, torch.float16),      # smallest ring rows, K split
+    (1, 33, 4096, 1032, 1, 8, 3, torch.bfloat16),    # last K tile one chunk deep, split
+    (1, 31, 65, 8, 1, 0, 2, torch.float16),          # one chunk of K, odd N
+    (1, 64, 300, 520, 0, 8, 0, torch.bfloat16),      # row-major B, partial K tile (padded rows)
+    (1, 65, 264, 1544, 0, 0, 3, torch.float16),      # row-major B, split, N % 128 != 0
+    (1, 129, 1001, 2048, 1, 0, 2, torch.bfloat16),   # odd N: element stores, no split
+    (1, 200, 4100, 4096, 1, 8, 0, torch.float16),    # N % 128 != 0 through the reduce
+    (1, 193, 512, 96, 1, 0, 0, torch.bfloat16),      # 32-deep K tiles
+    (3, 300, 136, 776, 0, 0, 0, torch.float16),      # batched, ragged M, N and K
+    (1, 2100, 4104, 576, 1, 0, 3, torch.float16),    # ragged rows and columns of 256-row tiles
+    (1, 2100, 4104, 576, 0, 8, 0, torch.bfloat16),   # the same, row-major B
+    (1, 1100, 3000, 4096, 1, 0, 2, torch.float16)])  # ragged, K-split tail of 256-row tiles
+def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype):
+    # rows that do not fill 256-row tiles, K down to one 16-byte chunk: every
+    # element against the oracle, with and without the K-split workspace, and
+    # nothing written outside D
+    if tb == 0 and (n + pad) % 8:
+        n += 8 - (n + pad) % 8
+    _log(f"gemm ragged {batch}x{m}x{n}x{k} tb={tb} pad={pad} epi={epi} {dtype}")
+    A = uniform((batch, m, k), k=51, dtype=dtype)
+    W = (uniform((batch, n, k) if tb else (batch, k, n), k=52, dtype=dtype).float() * 0.05).to(dtype)
+    bias = uniform((n,), k=53, dtype=dtype)
+    # what lies between rows must not enter the product
+    a_buf = torch.full((batch, m, k + pad), float("nan"), dtype=dtype)
+    a_buf[:, :, :k] = A
+    w_buf = torch.full((*W.shape[:2], W.shape[2] + pad), float("nan"), dtype=dtype)
+    w_buf[:, :, :W.shape[2]] = W
+    ad, wd, bd = a_buf.to(DEV), w_buf.to(DEV), bias.to(DEV)
+    wf = W.float().numpy()
+    want = O.gemm(A.float().numpy(), np.swapaxes(wf, 1, 2) if tb else wf, alpha=0.75, beta=0.5,
+                  c=bias.float().numpy()[None, None, :],
+                  epilogue={0: "none", 2: "gelu", 3: "silu"}[epi])
+    tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    nws = _capi.lib().sph_gemm_workspace_bytes(batch, m, n, k)
+    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
+    for w_ptr, w_n in ((None, 0), (_p(ws), nws)):
+        d = torch.full((batch, m + 1, n), 7.0, dtype=dtype, device=DEV)
+        _capi.call("sph_gemm_ex", DT[dtype], 0, tb, batch, m, n, k, 0.75, _p(ad), k + pad,
+                   a_buf[0].numel(), _p(wd), w_buf.shape[2], w_buf[0].numel(), 0.5, _p(bd), 0, 1,
+                   0, _p(d), n, (m + 1) * n, epi, w_ptr if w_n else None, w_n, _stream())
+        _sync()
+        assert_close_fp(d[:, :m], want, out_dtype=dtype, what="ragged gemm", **tol)
+        assert bool((d[:, m] == 7.0).all()), "rows past M written"
+
+
+@pytest.mark.parametrize("m,n,k,pad", [(9, 512, 4096, 0), (24, 1000, 520, 8), (100, 513, 512, 0),
+                                       (333, 1280, 1024, 0), (1100, 1280, 2048, 8),
+                                       (2, 64, 40, 0)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gemm_swiglu_any_rows(m, n, k, pad, dtype):
+    # the row counts, widths and depths that sph_gemm_swiglu refuses
+    _log(f"gemm swiglu any {m}x{n}x{k} pad={pad} {dtype}")
+    X = uniform((m, k), k=54, dtype=dtype)
+    W = (uniform((2 * n, k), k=55) * 0.05).to(dtype)
+    xd = torch.full((m, k + pad), float("nan"), dtype=dtype, device=DEV)
+    xd[:, :k] = X.to(DEV)
+    wd = torch.full((2 * n, k + pad), float("nan"), dtype=dtype, device=DEV)
+    wd[:, :k] = W.to(DEV)
+    xf, wf = X.float().numpy(), W.float().numpy()
+    want = O.silu(O.gemm(xf, wf[:n].T)) * O.gemm(xf, wf[n:].T)
+    tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    nws = _capi.lib().sph_gemm_swiglu_workspace_bytes(m, n, k)
+    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
+    for w_n in (0, nws):
+        d = torch.full((m + 1, n + pad), 7.0, dtype=dtype, device=DEV)
+        _capi.call("sph_gemm_swiglu_any", DT[dtype], m, n, k, _p(xd), k + pad, _p(wd), k + pad,
+                   _p(d), n + pad, _p(ws) if w_n else None, w_n, _stream())
+        _sync()
+        assert_close_fp(d[:m, :n], want, out_dtype=dtype, what=f"swiglu any {dtype}", **tol)
+        assert bool((d[m] == 7.0).all()) and bool((d[:, n:] == 7.0).all()), "outside D written"
+
+
 @pytest.mark.parametrize("m,n,k,tb,epi,dtype", [
     (2048, 4096, 12800, True, 0, torch.float16),   # 128 tiles, 2 K slices (c4 down shape)
     (1024, 4096, 8192, False, 3, torch.bfloat16),  # row-major B, bf16: 64 tiles, 4 slices

@@ -39,7 +39,7 @@ HIP_FLAGS = [
     "-std=c++17",
     # Packed-fp32 VALU forms are kept out of every kernel.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wno-unused-command-line-argument",
+    "-Wno-unused-command-line-argument", "-Wno-inline-asm",
     f"-I{INCLUDE}",
     f"-I{HIP_SRC}",
 ]

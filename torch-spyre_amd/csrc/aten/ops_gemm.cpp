@@ -207,9 +207,8 @@ at::Tensor gemm_swiglu(const at::Tensor& x_in, const at::Tensor& w_in) {
   at::Tensor x = x_in.stride(1) == 1 ? x_in : contiguous_on_device(x_in);
   at::Tensor w = w_in.stride(1) == 1 ? w_in : contiguous_on_device(w_in);
   c10::DeviceGuard guard(out.device());
-  const bool fits = ((m % 256 == 0 && n % 128 == 0 && k % 64 == 0) ||
-                     (m <= 8 && k >= 64 && k % 8 == 0 && k <= 8192)) && k > 0 &&
-                    x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 &&
+  const bool fits = k > 0 && k % 8 == 0 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 &&
+                    x.stride(0) >= k && w.stride(0) >= k &&
                     reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
   if (fits) {
@@ -217,7 +216,7 @@ at::Tensor gemm_swiglu(const at::Tensor& x_in, const at::Tensor& w_in) {
     check_matrix_extent(w, w.data_ptr(), 2 * n, k, w.stride(0), 0, 1, 0, "swiglu_mm w");
     const int64_t nws = sph_gemm_swiglu_workspace_bytes(m, n, k);
     at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, out.device()) : at::Tensor();
-    const int rc = sph_gemm_swiglu(to_sph(out.scalar_type()), m, n, k, x.data_ptr(), x.stride(0),
+    const int rc = sph_gemm_swiglu_any(to_sph(out.scalar_type()), m, n, k, x.data_ptr(), x.stride(0),
                                    w.data_ptr(), w.stride(0), out.data_ptr(), n,
                                    ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? nws : 0,
                                    stream(out.get_device()));

@@ -57,6 +57,8 @@ _SIGS = {
                                   c_i64, vp, c_i64, c_i64, c_int, vp], c_int),
     "sph_gemm_swiglu": ([c_int, c_i64, c_i64, c_i64, vp, c_i64, vp, c_i64, vp, c_i64, vp, c_i64,
                          vp], c_int),
+    "sph_gemm_swiglu_any": ([c_int, c_i64, c_i64, c_i64, vp, c_i64, vp, c_i64, vp, c_i64, vp, c_i64,
+                         vp], c_int),
     "sph_gemm_swiglu_workspace_bytes": ([c_i64, c_i64, c_i64], c_i64),
     "sph_gemm_ex": ([c_int, c_int, c_int, c_i64, c_i64, c_i64, c_i64, c_f32, vp, c_i64, c_i64, vp,
                      c_i64, c_i64, c_f32, vp, c_i64, c_i64, c_i64, vp, c_i64, c_i64, c_int, vp,

@@ -14,8 +14,10 @@ Here, on spyre graphs, the chain
 
 is replaced by swiglu_mm(x, w) (reshaped like y) when a fused kernel takes
 the shape (fp16 / bf16; M % 256 == 0, n % 128 == 0, K % 64 == 0 for the
-tiled GEMM of prefill, or M <= 8 with K % 8 == 0 and 64 <= K <= 8192 for
-the weight-stream kernel of decode) and no intermediate is used elsewhere:
+tiled GEMM of prefill, M <= 8 with K % 8 == 0 and 64 <= K <= 8192 for
+the weight-stream kernel of decode, or any other M with K % 8 == 0 and a
+weight of at least 512 x 512 per half for the ring kernel of ragged row
+counts: below that the call is launch-bound) and no intermediate is used elsewhere:
 the [M, 2n] projection is then never written to HBM.
 """
 
@@ -32,6 +34,7 @@ prims = torch.ops.prims
 
 ROW_BLOCK, COL_BLOCK, K_BLOCK = 256, 128, 64  # tiled GEMM (prefill)
 STREAM_ROWS, STREAM_K = 8, 8192               # weight-stream kernel (decode)
+RING_MIN = 512                                # n and K of a ragged-row product
 _BIG = 2 ** 62
 
 
@@ -106,7 +109,8 @@ def _match(y: torch.fx.Node) -> Optional[tuple]:
             continue
         tiles = M % ROW_BLOCK == 0 and n % COL_BLOCK == 0 and K % K_BLOCK == 0
         stream = M <= STREAM_ROWS and K % 8 == 0 and 64 <= K <= STREAM_K
-        if not (tiles or stream):
+        ring = M > STREAM_ROWS and K % 8 == 0 and K >= RING_MIN and n >= RING_MIN
+        if not (tiles or stream or ring):
             continue
         return x, w, chain
     return None
