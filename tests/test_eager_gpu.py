@@ -537,3 +537,22 @@ def test_out_of_range_indices_raise_index_error():
         f(table, torch.tensor([0, 11]).to("spyre")).cpu()
     torch.testing.assert_close(f(table, torch.tensor([0, 9]).to("spyre")).cpu(),
                                table.cpu()[[0, 9]] * 2)
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_single_row_projections_take_any_row_stride(swiglu):
+    """A one-row activation's row stride is arbitrary (a view of a decode
+    batch of one may report 1); an expanded activation has stride 0."""
+    K, n = 512, 320
+    w = (randn((2 * n, K), k=1) * 0.1).to(DEV)
+    nw = randn((K,), k=2, scale=0.1, mean=1.0).to(DEV)
+    x = randn((1, K), k=3).to(DEV)
+    want = torch.ops.spyre.rms_norm_mm(x, nw, 1e-5, w, swiglu)
+    odd = torch.as_strided(x, (1, K), (1, 1))
+    assert torch.equal(torch.ops.spyre.rms_norm_mm(odd, nw, 1e-5, w, swiglu).cpu(), want.cpu())
+    if swiglu:
+        a = torch.ops.spyre.swiglu_mm(x, w)
+        assert torch.equal(torch.ops.spyre.swiglu_mm(odd, w).cpu(), a.cpu())
+        wide = torch.ops.spyre.swiglu_mm(x.expand(20, K), w).cpu()
+        torch.testing.assert_close(wide.float(), a.cpu().expand(20, n).float(), rtol=1e-2,
+                                   atol=1e-2)

@@ -192,6 +192,11 @@ at::Tensor& baddbmm_out(const at::Tensor& self, const at::Tensor& b1, const at::
 
 }  // namespace
 
+// Leading dim of a row-major view: a single row's stride is arbitrary.
+int64_t row_ld(const at::Tensor& t) {
+  return t.size(0) == 1 ? (t.size(1) + 7) / 8 * 8 : t.stride(0);
+}
+
 // silu(x w[:n]^T) * (x w[n:]^T) for x [M, K], w [2n, K] on spyre: one fused
 // GEMM (sph_gemm_swiglu) when the shape fits it, else the three device ops
 // (mm, silu, mul) with the rounding the unfused program has.
@@ -207,17 +212,17 @@ at::Tensor gemm_swiglu(const at::Tensor& x_in, const at::Tensor& w_in) {
   at::Tensor x = x_in.stride(1) == 1 ? x_in : contiguous_on_device(x_in);
   at::Tensor w = w_in.stride(1) == 1 ? w_in : contiguous_on_device(w_in);
   c10::DeviceGuard guard(out.device());
-  const bool fits = k > 0 && k % 8 == 0 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 &&
-                    x.stride(0) >= k && w.stride(0) >= k &&
+  const int64_t ldx = row_ld(x), ldw = row_ld(w);
+  const bool fits = k > 0 && k % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= k && ldw >= k &&
                     reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
   if (fits) {
-    check_matrix_extent(x, x.data_ptr(), m, k, x.stride(0), 0, 1, 0, "swiglu_mm x");
-    check_matrix_extent(w, w.data_ptr(), 2 * n, k, w.stride(0), 0, 1, 0, "swiglu_mm w");
+    check_matrix_extent(x, x.data_ptr(), m, k, ldx, 0, 1, 0, "swiglu_mm x");
+    check_matrix_extent(w, w.data_ptr(), 2 * n, k, ldw, 0, 1, 0, "swiglu_mm w");
     const int64_t nws = sph_gemm_swiglu_workspace_bytes(m, n, k);
     at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, out.device()) : at::Tensor();
-    const int rc = sph_gemm_swiglu_any(to_sph(out.scalar_type()), m, n, k, x.data_ptr(), x.stride(0),
-                                   w.data_ptr(), w.stride(0), out.data_ptr(), n,
+    const int rc = sph_gemm_swiglu_any(to_sph(out.scalar_type()), m, n, k, x.data_ptr(), ldx,
+                                   w.data_ptr(), ldw, out.data_ptr(), n,
                                    ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? nws : 0,
                                    stream(out.get_device()));
     if (rc == 0) return out;
@@ -253,16 +258,17 @@ at::Tensor gemm_rmsnorm(const at::Tensor& x_in, const at::Tensor& norm_w_in, dou
   auto al = [](const at::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  const bool fits = m <= 8 && k >= 64 && k % 8 == 0 && k <= 8192 && x.stride(0) % 8 == 0 &&
-                    w.stride(0) % 8 == 0 && al(x) && al(w) && al(nw);
+  const int64_t ldx = row_ld(x), ldw = row_ld(w);
+  const bool fits = m <= 8 && k >= 64 && k % 8 == 0 && k <= 8192 && ldx % 8 == 0 && ldw % 8 == 0 &&
+                    ldx >= k && ldw >= k && al(x) && al(w) && al(nw);
   c10::DeviceGuard guard(out.device());
   if (fits) {
-    check_matrix_extent(x, x.data_ptr(), m, k, x.stride(0), 0, 1, 0, "rms_norm_mm x");
-    check_matrix_extent(w, w.data_ptr(), swiglu ? 2 * n : n, k, w.stride(0), 0, 1, 0,
+    check_matrix_extent(x, x.data_ptr(), m, k, ldx, 0, 1, 0, "rms_norm_mm x");
+    check_matrix_extent(w, w.data_ptr(), swiglu ? 2 * n : n, k, ldw, 0, 1, 0,
                         "rms_norm_mm w");
     SPYRE_SPH_CHECK(sph_gemm_rmsnorm(to_sph(out.scalar_type()), m, n, k, x.data_ptr(),
-                                     x.stride(0), nw.data_ptr(), static_cast<float>(eps),
-                                     w.data_ptr(), w.stride(0), out.data_ptr(), n, swiglu ? 1 : 0,
+                                     ldx, nw.data_ptr(), static_cast<float>(eps),
+                                     w.data_ptr(), ldw, out.data_ptr(), n, swiglu ? 1 : 0,
                                      stream(out.get_device())));
     return out;
   }
