@@ -237,3 +237,41 @@ def test_fused_masked_attention_any_key_count(sk):
     # and the op itself, called directly with the unpadded mask
     direct = torch.ops.spyre.attention(q.to(DEV), k.to(DEV), v.to(DEV), mask.to(DEV), scale)
     assert_close_fp(direct, want, what=f"spyre.attention sk={sk}")
+
+
+def test_bf16_conversion_bits():
+    # float32 -> bf16 in the generated and in the eager kernels: ties to even,
+    # subnormals, overflow to infinity and NaN as torch's CPU cast has them
+    _log("float32 -> bf16 conversion")
+    g = torch.Generator().manual_seed(0xAFFE)
+    bits = torch.randint(-2 ** 31, 2 ** 31, (4096, 8), generator=g, dtype=torch.int64)
+    edge = torch.tensor([0, 0x80000000, 1, 0x7fff, 0x8000, 0x8001, 0x18000, 0x007fffff, 0x3f808000,
+                         0x3f818000, 0x3f80ffff, 0x7f7f7fff, 0x7f7f8000, 0x7f7fffff, 0x7f800000,
+                         0xff800000, 0x7fc00000, 0x7f800001, 0xffc12345, 0xff7fffff, 0x00800000,
+                         0x807f8000, 0x33800000, 0x477fe000])
+    bits = torch.cat([edge.view(-1, 8), bits])
+    x = (bits & 0xffffffff).to(torch.int64)
+    x = torch.where(x >= 2 ** 31, x - 2 ** 32, x).to(torch.int32).view(torch.float32)
+    want = x.to(torch.bfloat16)
+    eager = x.to(DEV).to(torch.bfloat16).cpu()
+    compiled = torch.compile(lambda t: t.to(torch.bfloat16))(x.to(DEV)).cpu()
+    nan = torch.isnan(want)
+    for got in (eager, compiled):
+        assert torch.equal(torch.isnan(got), nan)
+        assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
+def test_c3_gelu_chain_bf16_matches_cpu():
+    # bf16 rows of the fused chain, widths with and without 16-byte rows
+    for cols in (4096, 1000, 513):
+        x, s, b = randn((64, cols), k=0).bfloat16(), randn((cols,), k=1).bfloat16(), \
+            randn((cols,), k=2).bfloat16()
+        fn = torch.compile(lambda a, s, c: (lambda t: (t, t.sum(-1)))(F.gelu(a * s + c)),
+                           dynamic=False)
+        y, r = fn(x.to(DEV), s.to(DEV), b.to(DEV))
+        want = F.gelu(x.float() * s.float() + b.float())
+        torch.testing.assert_close(y.cpu().float(), want, rtol=1e-2, atol=1e-2)
+        # the sum of `cols` values rounded to bf16: 2^-8 of the rounded total
+        # plus half a bf16 step of each addend
+        bound = want.sum(-1).abs() * 2 ** -7 + want.abs().sum(-1) * 2 ** -9 + 1e-2
+        assert ((r.cpu().float() - want.sum(-1)).abs() <= bound).all()

@@ -77,6 +77,12 @@ __device__ __host__ inline float bf16_to_float(bf16_t v) {
 }
 
 __device__ __host__ inline bf16_t float_to_bf16(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // gfx950's conversion: the same result in one instruction, branch-free
+  bf16_t d;
+  d.bits = __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+  return d;
+#else
   uint32_t u;
   __builtin_memcpy(&u, &f, 4);
   bf16_t r;
@@ -88,6 +94,7 @@ __device__ __host__ inline bf16_t float_to_bf16(float f) {
   u += 0x7fffu + lsb;
   r.bits = static_cast<uint16_t>(u >> 16);
   return r;
+#endif
 }
 
 template <typename T>

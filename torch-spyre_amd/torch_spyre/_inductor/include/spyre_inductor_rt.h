@@ -55,14 +55,12 @@ template <>
 struct Cvt<bfloat16> {
   template <typename V>
   __device__ static inline bfloat16 from(V v) {
-    uint32_t u = __float_as_uint(static_cast<float>(v));
+    // gfx950's own conversion (round to nearest even, NaN stays quiet): no
+    // branch, so a group's stores merge into 16-byte ones.  (With the NaN case
+    // as a branch the 8192 x 4096 bf16 GELU chain wrote 2 bytes a store: 213 us
+    // against 24 us.)
     bfloat16 r;
-    if ((u & 0x7fffffffu) > 0x7f800000u) {  // NaN stays quiet
-      r.bits = static_cast<uint16_t>((u >> 16) | 0x40u);
-      return r;
-    }
-    u += 0x7fffu + ((u >> 16) & 1u);
-    r.bits = static_cast<uint16_t>(u >> 16);
+    r.bits = __builtin_bit_cast(uint16_t, static_cast<__bf16>(static_cast<float>(v)));
     return r;
   }
 };
