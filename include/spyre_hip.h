@@ -298,6 +298,15 @@ int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
                       int64_t stride_m, int64_t causal_q, int64_t causal_off, float scale,
                       void* o, int64_t ldo, int64_t stride_o, void* workspace,
                       int64_t workspace_bytes, sph_stream_t stream);
+/* sph_attention_fwd for any number of query rows (ragged prompts): the last
+ * block of rows may be partial.  Same arguments, workspace and results. */
+int sph_attention_fwd_rows(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
+                      int64_t head_dim, const void* q, int64_t ldq, int64_t stride_q,
+                      const void* k, int64_t ldk, int64_t stride_k, const void* v,
+                      int64_t ldv, int64_t stride_v, const void* mask, int64_t ldm,
+                      int64_t stride_m, int64_t causal_q, int64_t causal_off, float scale,
+                      void* o, int64_t ldo, int64_t stride_o, void* workspace,
+                      int64_t workspace_bytes, sph_stream_t stream);
 /* Bytes of mask-block classes sph_attention_fwd uses for this shape: one
  * per (mask batch, 128-row block, 64-key block); 0 for an empty shape.
  * For mq <= 16 (the decode path below) the split workspace of

@@ -187,3 +187,14 @@ def test_nonpositive_or_infinite_scales_stay_unfused(form):
         ref = _chain(q, k, v, mask, scale=scale, div=form == "neg_div")
     assert n == 0
     torch.testing.assert_close(out, ref, rtol=1e-2, atol=1e-2, equal_nan=True)
+
+
+@pytest.mark.parametrize("mq,sk", [(300, 130), (4 * 77, 77)])
+def test_ragged_rows_fuse(mq, sk):
+    # row counts off the 128-row block, from 2^16 scores on
+    q, k, v = _qkv(4, mq, sk, seed=6)
+    mask = torch.zeros(mq, sk, dtype=torch.float16)
+    mask[:, sk - 5:] = float("-inf")
+    out, n = _run(lambda q, k, v, m: _chain(q, k, v, m), q, k, v, mask)
+    assert n == 1
+    torch.testing.assert_close(out, _chain(q, k, v, mask), rtol=2e-3, atol=2e-3)

@@ -983,6 +983,51 @@ def test_attention_causal_mask_matches_causal_positions():
     assert torch.equal(by_mask, by_pos)
 
 
+@pytest.mark.parametrize("kind,b,mq,sk,causal_q", [
+    ("none", 2, 17, 64, 0), ("none", 1, 129, 70, 0), ("positions", 2, 3 * 77, 77, 77),
+    ("positions", 1, 255, 255, 255), ("causal", 2, 4 * 77, 80, 77), ("window", 2, 300, 328, 0),
+    ("holes", 3, 200, 320, 0), ("row", 2, 140, 72, 0)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
+    # row counts off the 128-row block: the oracle's rows, the same bits as
+    # the padded call's, and nothing written past the last row
+    _log(f"attention ragged {kind} b={b} mq={mq} sk={sk} {dtype}")
+    q = randn((b, mq, 128), k=58, dtype=dtype)
+    k = randn((b, sk, 128), k=59, dtype=dtype)
+    v = randn((b, sk, 128), k=60, dtype=dtype)
+    scale = 1 / math.sqrt(128)
+    mask, ldm, sm = None, 0, 0
+    if kind == "row":
+        mask = torch.where(torch.arange(sk) < sk - 9, 0.0, float("-inf")).to(dtype).expand(mq, sk)
+        md = mask[0].contiguous().to(DEV)
+    elif kind not in ("none", "positions"):
+        mask = _block_mask(kind, b, mq, sk, causal_q).to(dtype)
+        md, ldm, sm = mask.to(DEV), sk, mq * sk if mask.dim() == 3 else 0
+    cq = causal_q if kind == "positions" else 0
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    nws = _capi.lib().sph_attention_workspace_bytes(b, mq, sk, sm) if mask is not None else 0
+    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
+    want = O.attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), scale,
+                       mask=None if mask is None else mask.float().numpy(), causal_q_len=cq,
+                       causal_offset=sk - cq if cq else 0)
+    tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    for w_n in ((0, nws) if mask is not None else (0,)):
+        o = torch.full((b, mq + 1, 128), 7.0, dtype=dtype, device=DEV)
+        _capi.call("sph_attention_fwd_rows", DT[dtype], b, mq, sk, 128, _p(qd), 128, mq * 128,
+                   _p(kd), 128, sk * 128, _p(vd), 128, sk * 128, _p(md) if mask is not None else None,
+                   ldm, sm, cq, sk - cq if cq else 0, scale, _p(o), 128, (mq + 1) * 128,
+                   _p(ws) if w_n else None, w_n, _stream())
+        _sync()
+        assert_close_fp(o[:, :mq], want, out_dtype=dtype, what="ragged attention", **tol)
+        assert bool((o[:, mq] == 7.0).all()), "rows past mq written"
+    # sph_attention_fwd keeps refusing these rows
+    rc = _capi.lib().sph_attention_fwd(DT[dtype], b, mq, sk, 128, _p(qd), 128, mq * 128, _p(kd), 128,
+                                       sk * 128, _p(vd), 128, sk * 128, None, 0, 0, 0, 0,
+                                       ctypes.c_float(scale), _p(o), 128, (mq + 1) * 128, None, 0,
+                                       _stream())
+    assert rc == 1002
+
+
 def test_attention_fused_c4_shape():
     # the c4 layer's attention: 8 KV heads, 4 query heads stacked per KV
     # head (mq = 4 * 2048), causal over 2048 keys; one batch element

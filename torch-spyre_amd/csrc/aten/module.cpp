@@ -31,7 +31,7 @@ at::Tensor gemm_rmsnorm(const at::Tensor& x, const at::Tensor& norm_w, double ep
 // Fused attention (ops_attention.cpp).
 at::Tensor attention_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                          const c10::optional<at::Tensor>& mask, double scale, int64_t causal_q,
-                         int64_t causal_off);
+                         int64_t causal_off, bool any_rows);
 at::Tensor decode_attention_step(const at::Tensor& qkv, const at::Tensor& cos,
                                  const at::Tensor& sin, const at::Tensor& pos,
                                  at::Tensor& k_cache, at::Tensor& v_cache, int64_t n_heads,
@@ -68,8 +68,10 @@ PYBIND11_MODULE(_C, m) {
 
   m.def("attention_fwd", &spyre::attention_fwd, py::arg("q"), py::arg("k"), py::arg("v"),
         py::arg("mask"), py::arg("scale"), py::arg("causal_q") = 0, py::arg("causal_off") = 0,
+        py::arg("any_rows") = false,
         "softmax(scale * q k^T + mask) v on the spyre stream (q [B, mq, 128], k / v "
-        "[B, sk, 128], mask [mq, sk] / [B or 1, mq, sk] or None; fp16 / bf16).");
+        "[B, sk, 128], mask [mq, sk] / [B or 1, mq, sk] or None; fp16 / bf16; mq % 128 == 0 or "
+        "mq <= 16, with any_rows any mq).");
   m.def("decode_attention_step", &spyre::decode_attention_step, py::arg("qkv"), py::arg("cos"),
         py::arg("sin"), py::arg("pos"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("n_heads"), py::arg("n_kv_heads"), py::arg("scale"),

@@ -8,7 +8,8 @@
 // substitutes this entry for that chain when its shapes fit (head dim 128,
 // query rows a multiple of 128, or at most 16 per batch entry for a decode
 // step (sph_attention_decode), fp16/bf16); called directly it accepts the
-// same shapes and raises otherwise.
+// same shapes and raises otherwise.  With any_rows the row count is free
+// (sph_attention_fwd_rows).
 #include <torch/extension.h>
 
 #include "spyre_ops_common.h"
@@ -32,7 +33,7 @@ at::Tensor rows_aligned(const at::Tensor& t) {
 
 at::Tensor attention_fwd(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& v_in,
                          const c10::optional<at::Tensor>& mask_in, double scale,
-                         int64_t causal_q, int64_t causal_off) {
+                         int64_t causal_q, int64_t causal_off, bool any_rows) {
   TORCH_CHECK(is_spyre(q_in) && is_spyre(k_in) && is_spyre(v_in),
               "spyre attention: q, k, v must be spyre tensors");
   TORCH_CHECK(q_in.dim() == 3 && k_in.dim() == 3 && v_in.dim() == 3,
@@ -109,7 +110,8 @@ at::Tensor attention_fwd(const at::Tensor& q_in, const at::Tensor& k_in, const a
         stream(q.get_device())));
     return out;
   }
-  SPYRE_SPH_CHECK(sph_attention_fwd(
+  const auto fwd = any_rows ? sph_attention_fwd_rows : sph_attention_fwd;
+  SPYRE_SPH_CHECK(fwd(
       to_sph(dt), B, mq, sk, d, q.data_ptr(), q.stride(1), qst[0], k.data_ptr(), k.stride(1),
       kst[0], v.data_ptr(), v.stride(1), vst[0], mp, ldm, sm, causal_q, causal_off,
       static_cast<float>(scale), out.data_ptr(), d, mq * d, ws.defined() ? ws.data_ptr() : nullptr,

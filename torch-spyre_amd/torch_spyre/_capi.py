@@ -71,6 +71,9 @@ _SIGS = {
     "sph_attention_fwd": ([c_int, c_i64, c_i64, c_i64, c_i64, vp, c_i64, c_i64, vp, c_i64,
                            c_i64, vp, c_i64, c_i64, vp, c_i64, c_i64, c_i64, c_i64, c_f32, vp,
                            c_i64, c_i64, vp, c_i64, vp], c_int),
+    "sph_attention_fwd_rows": ([c_int, c_i64, c_i64, c_i64, c_i64, vp, c_i64, c_i64, vp, c_i64,
+                           c_i64, vp, c_i64, c_i64, vp, c_i64, c_i64, c_i64, c_i64, c_f32, vp,
+                           c_i64, c_i64, vp, c_i64, vp], c_int),
     "sph_attention_workspace_bytes": ([c_i64, c_i64, c_i64, c_i64], c_i64),
     "sph_attention_decode": ([c_int, c_i64, c_i64, c_i64, c_i64, vp, c_i64, c_i64, vp, c_i64,
                               c_i64, vp, c_i64, c_i64, c_i64, vp, c_i64, c_i64, c_i64, c_i64,

@@ -230,6 +230,14 @@ def _(x, mean, norm_mean, weight, bias):
 
 # ---- fused attention --------------------------------------------------------
 
+def _attention_chain(q, k, v, mask, scale):
+    s = torch.bmm(q, k.transpose(1, 2)) * scale
+    if mask is not None:
+        s = s + mask
+    p = torch.softmax(s.float(), dim=-1).to(q.dtype)
+    return torch.bmm(p, v)
+
+
 @torch.library.custom_op("spyre::attention", mutates_args=())
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor],
               scale: float) -> torch.Tensor:
@@ -240,11 +248,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[
     (codegen/inputs/spyre_torch_ops.cpp:297-377), add + _softmax
     (codegen/inputs/Metadata.yaml:275-277) and bmm again; on other devices
     it runs as that chain, on spyre as one fused kernel."""
-    s = torch.bmm(q, k.transpose(1, 2)) * scale
-    if mask is not None:
-        s = s + mask
-    p = torch.softmax(s.float(), dim=-1).to(q.dtype)
-    return torch.bmm(p, v)
+    return _attention_chain(q, k, v, mask, scale)
 
 
 @attention.register_kernel("spyre")
@@ -255,6 +259,25 @@ def _(q, k, v, mask, scale):
 
 
 @attention.register_fake
+def _(q, k, v, mask, scale):
+    return q.new_empty((q.shape[0], q.shape[1], v.shape[2]))
+
+
+@torch.library.custom_op("spyre::attention_rows", mutates_args=())
+def attention_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                   mask: Optional[torch.Tensor], scale: float) -> torch.Tensor:
+    """spyre::attention for any number of query rows (ragged prompts)."""
+    return _attention_chain(q, k, v, mask, scale)
+
+
+@attention_rows.register_kernel("spyre")
+def _(q, k, v, mask, scale):
+    from torch_spyre import _C
+
+    return _C.attention_fwd(q, k, v, mask, float(scale), any_rows=True)
+
+
+@attention_rows.register_fake
 def _(q, k, v, mask, scale):
     return q.new_empty((q.shape[0], q.shape[1], v.shape[2]))
 

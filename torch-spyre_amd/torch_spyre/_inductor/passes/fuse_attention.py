@@ -6,8 +6,9 @@ separate ops (spyre__bmm_default, codegen/inputs/spyre_torch_ops.cpp:297-377;
 add and _softmax, codegen/inputs/Metadata.yaml:275-277) and forbids fusion
 in its scheduler (torch_spyre/_inductor/choices.py:58-83).  Here the chain
 is replaced, on spyre graphs only, when the fused kernel takes its shapes:
-fp16 / bf16, head dim 128, query rows a multiple of 128, and a mask (if
-any) of the same dtype shaped [mq, sk] or [B or 1, mq, sk], or one mask row
+fp16 / bf16, head dim 128, query rows a multiple of 128 (or, from 2^16
+scores on, any number above 16: `torch.ops.spyre.attention_rows`), and a
+mask (if any) of the same dtype shaped [mq, sk] or [B or 1, mq, sk], or one mask row
 [sk] / [1, sk] broadcast over the rows (expanded to [mq, sk] as a view).  The fused op
 computes the same function (fp32 scores and softmax, probabilities rounded
 to the input dtype before the second product).
@@ -38,6 +39,9 @@ prims = torch.ops.prims
 
 HEAD_DIM = 128
 ROW_BLOCK = 128
+# Ragged row counts: below this many scores the chain's products and softmax
+# are one small launch each, which a last, mostly empty row block does not beat.
+RAGGED_SCORES = 1 << 16
 
 
 def _val(n):
@@ -178,8 +182,9 @@ def _finish(bmm2, bmm1, chain, v, mask, scale) -> Optional[tuple]:
     # Decode shapes (a few rows per KV head) stay on the unfused chain: the
     # fused decode kernel (sph_attention_decode) measured slower than it in
     # the c5 decode step (4.77 against 4.65 ms per step).
-    if d != HEAD_DIM or mq % ROW_BLOCK or tuple(kv.shape) != (B, sk, d) or \
-            tuple(vv.shape) != (B, sk, d):
+    if d != HEAD_DIM or tuple(kv.shape) != (B, sk, d) or tuple(vv.shape) != (B, sk, d):
+        return None
+    if mq % ROW_BLOCK and (mq <= 16 or B * mq * sk < RAGGED_SCORES):
         return None
     expand = None
     if mask is not None:
@@ -209,7 +214,9 @@ def fuse_attention(gm: torch.fx.GraphModule) -> int:
             if expand is not None:  # one mask row for every query row
                 mask = g.call_function(aten.expand.default, (mask, expand))
                 mask.meta["val"] = _val(m[3]).expand(expand)
-            new = g.call_function(torch.ops.spyre.attention.default, (q, k, v, mask, scale))
+            ragged = _val(q).shape[1] % ROW_BLOCK != 0
+            op = torch.ops.spyre.attention_rows if ragged else torch.ops.spyre.attention
+            new = g.call_function(op.default, (q, k, v, mask, scale))
         new.meta.update(node.meta)
         node.replace_all_uses_with(new)
         g.erase_node(node)
