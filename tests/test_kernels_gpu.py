@@ -61,6 +61,45 @@ def test_softmax_shapes(rows, cols):
     np.testing.assert_allclose(np32(yd).sum(-1), 1.0, rtol=2e-2)
 
 
+@pytest.mark.parametrize("rows,cols", [(3, 8193), (2, 16384), (2, 16391), (2, 32769), (3, 49155),
+                                       (2, 65536), (1, 65537), (1, 131071), (1, 131073)])
+@pytest.mark.parametrize("log,causal,scale", [(0, 0, 1.0), (1, 0, 0.5), (0, 1, 1.0), (1, 1, 1.0),
+                                              (0, 0, -0.5)])
+def test_softmax_long_rows(rows, cols, log, causal, scale):
+    # rows held in registers as 16-bit values, at odd element offsets: infinite
+    # and fully masked entries, causal limits inside and at the row ends
+    _log(f"softmax long {rows}x{cols} log={log} causal={causal} scale={scale}")
+    for dtype in (torch.float16, torch.bfloat16):
+        x = randn((rows, cols), k=3, scale=3.0, dtype=dtype)
+        x[0, 5:4000] = float("-inf")
+        buf = torch.full((rows, cols + 3), float("nan"), dtype=dtype)
+        buf[:, 1:1 + cols] = x
+        bd = buf.to(DEV)
+        yd = torch.full((rows, cols + 3), 7.0, dtype=dtype, device=DEV)
+        off = cols - rows - 7
+        _capi.call("sph_softmax_rows", DT[dtype], DT[dtype], _p(bd) + 2, cols + 3, _p(yd) + 2,
+                   cols + 3, rows, cols, scale, log + 2 * causal, rows, off, _stream())
+        _sync()
+        xf = x.double() * scale
+        if scale < 0:
+            xf[0, 5:4000] = float("inf")
+        if causal:
+            c = torch.arange(cols)[None, :] > torch.arange(rows)[:, None] + off
+            xf = xf.masked_fill(c, float("-inf"))
+        want = torch.log_softmax(xf, -1) if log else torch.softmax(xf, -1)
+        got = yd[:, 1:1 + cols].cpu().double()
+        tol = 2e-3 if dtype == torch.float16 else 1e-2  # a rounding step of the output type
+        torch.testing.assert_close(got, want, rtol=tol, atol=1e-3 if log else 1e-7, equal_nan=True)
+        assert bool((yd[:, 0] == 7.0).all()) and bool((yd[:, cols + 1:] == 7.0).all())
+    x[:] = float("-inf")
+    xd = x.to(DEV)
+    yd = torch.zeros_like(xd)
+    _capi.call("sph_softmax_rows", DT[dtype], DT[dtype], _p(xd), cols, _p(yd), cols, rows, cols,
+               1.0, log, 0, 0, _stream())
+    _sync()
+    assert bool(torch.isnan(yd).all())
+
+
 def test_softmax_reference_kat():
     _log("softmax arange KAT")
     x = torch.arange(0, 64, dtype=torch.float16).unsqueeze(0).repeat(3, 1)

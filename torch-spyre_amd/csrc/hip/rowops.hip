@@ -36,14 +36,49 @@ constexpr int block_of() {
   return TPR < 256 ? 256 : TPR;
 }
 
+// 16 bytes at any element alignment: global memory takes 16-byte accesses off
+// their natural alignment in one instruction, so rows of odd length (a
+// vocabulary of 49155) move in whole chunks too.  (Element by element, lanes 16
+// bytes apart, the 64 x 49155 bf16 log-softmax took 35 us.)
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <typename T>
+__device__ inline void load8u(const T* __restrict__ p, float (&v)[8]) {
+  constexpr int W = 16 / sizeof(T);
+#pragma unroll
+  for (int h = 0; h < 8 / W; ++h) {
+    const u32x4 raw = *reinterpret_cast<const u32x4_any*>(p + h * W);
+    const T* e = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+    for (int i = 0; i < W; ++i) v[h * W + i] = Num<T>::to_f(e[i]);
+  }
+}
+template <typename T, bool NT = false>
+__device__ inline void store8u(T* __restrict__ p, const float (&v)[8]) {
+  constexpr int W = 16 / sizeof(T);
+#pragma unroll
+  for (int h = 0; h < 8 / W; ++h) {
+    u32x4 raw;
+    T* e = reinterpret_cast<T*>(&raw);
+#pragma unroll
+    for (int i = 0; i < W; ++i) e[i] = Num<T>::from_f(v[h * W + i]);
+    if constexpr (NT)
+      __builtin_nontemporal_store(raw, reinterpret_cast<u32x4_any*>(p + h * W));
+    else
+      *reinterpret_cast<u32x4_any*>(p + h * W) = raw;
+  }
+}
+
 // Loads one chunk of 8 elements starting at column c0 (out-of-row elements
-// get `fill`).  VEC: the row base is 16-byte aligned, so a full chunk can be
-// read with vector loads; a partial last chunk is read element-wise.
-template <typename T, bool VEC>
+// get `fill`); a partial last chunk is read element by element.  VEC: rows
+// are 16-byte aligned (the norms at 8192 x 4096: 39.3 us, 40.3 without it).
+template <typename T, bool VEC = false>
 __device__ inline void load_chunk(const T* __restrict__ row, int64_t cols,
                                   int64_t c0, float fill, float (&v)[8]) {
-  if (VEC && c0 + 8 <= cols) {
-    load8<T>(row + c0, v);
+  if (c0 + 8 <= cols) {
+    if constexpr (VEC)
+      load8<T>(row + c0, v);
+    else
+      load8u<T>(row + c0, v);
   } else {
     const int64_t n = cols - c0;
     load8_partial<T>(row + c0, n > 8 ? 8 : (n < 0 ? 0 : static_cast<int>(n)),
@@ -58,21 +93,24 @@ __device__ inline int64_t chunk_col(int i, int t) {
 }
 
 // Loads this thread's VPT chunks of a row.
-template <typename T, int TPR, int VPT, bool VEC>
+template <typename T, int TPR, int VPT, bool VEC = false>
 __device__ inline void load_row(const T* __restrict__ row, int64_t cols,
                                 int t, float fill, float (&v)[VPT][8]) {
 #pragma unroll
   for (int i = 0; i < VPT; ++i) load_chunk<T, VEC>(row, cols, chunk_col<TPR>(i, t), fill, v[i]);
 }
 
-template <typename T, int TPR, int VPT, bool VEC, bool NT = false>
+template <typename T, int TPR, int VPT, bool NT = false, bool VEC = false>
 __device__ inline void store_row(T* __restrict__ row, int64_t cols, int t,
                                  const float (&v)[VPT][8]) {
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int64_t c0 = chunk_col<TPR>(i, t);
-    if (VEC && c0 + 8 <= cols) {
-      store8<T, NT>(row + c0, v[i]);
+    if (c0 + 8 <= cols) {
+      if constexpr (VEC)
+        store8<T, NT>(row + c0, v[i]);
+      else
+        store8u<T, NT>(row + c0, v[i]);
     } else {
       const int64_t n = cols - c0;
       if (n > 0) store8_partial<T>(row + c0, n > 8 ? 8 : static_cast<int>(n), v[i]);
@@ -86,7 +124,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 // ----------------------------------------------------------------------------
 // Softmax
 // ----------------------------------------------------------------------------
-template <typename TI, typename TO, int TPR, int VPT, bool VEC>
+template <typename TI, typename TO, int TPR, int VPT>
 __global__ void __launch_bounds__(block_of<TPR>())
 softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
              int64_t ldy, int64_t rows, int64_t cols, float scale, int flags,
@@ -101,7 +139,7 @@ softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
 
   float v[VPT][8];
   if (valid) {
-    load_row<TI, TPR, VPT, VEC>(x + row * ldx, cols, t, ninf, v);
+    load_row<TI, TPR, VPT>(x + row * ldx, cols, t, ninf, v);
   } else {
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
@@ -156,7 +194,7 @@ softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[i][j] *= inv;
   }
-  store_row<TO, TPR, VPT, VEC>(y + row * ldy, cols, t, v);
+  store_row<TO, TPR, VPT>(y + row * ldy, cols, t, v);
 }
 
 // (max, sum) state of an online softmax: `s` sums exp2(x - m) over the
@@ -208,15 +246,25 @@ __device__ inline void group_ms(float& m, float& s, float* lds_m, float* lds_s) 
     }
     __syncthreads();
     const int first = (wave / NW) * NW;
-    m = lds_m[first];
-    s = lds_s[first];
+    if constexpr (NW == 16) {
+      // 16 waves: one state per lane of a 16-lane row, four butterfly steps
+      // instead of 15 merges in series
+      m = lds_m[threadIdx.x & 15];
+      s = lds_s[threadIdx.x & 15];
+      ms_merge(m, s, dpp_f<0xB1>(m), dpp_f<0xB1>(s));
+      ms_merge(m, s, dpp_f<0x4E>(m), dpp_f<0x4E>(s));
+      ms_merge(m, s, dpp_f<0x141>(m), dpp_f<0x141>(s));
+      ms_merge(m, s, dpp_f<0x140>(m), dpp_f<0x140>(s));
+    } else {
+      m = lds_m[first];
+      s = lds_s[first];
 #pragma unroll
-    for (int k = 1; k < NW; ++k) ms_merge(m, s, lds_m[first + k], lds_s[first + k]);
+      for (int k = 1; k < NW; ++k) ms_merge(m, s, lds_m[first + k], lds_s[first + k]);
+    }
   }
 }
 
-// Rows of exactly TPR * VPT * 8 columns with 16-byte aligned rows (c1's
-// [512, 4096] among them): whole chunks without per-chunk bounds tests, the
+// Rows of exactly TPR * VPT * 8 columns (c1's [512, 4096] among them): whole chunks without per-chunk bounds tests, the
 // causal mask and log form chosen once per thread rather than tested per
 // element, and one combined (max, sum) reduction per row: each thread sums
 // exp2 of its values against its own maximum, and the states merge in one
@@ -239,7 +287,7 @@ softmax_full(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t 
   if (!valid) row = rows - 1;
   float v[VPT][8];
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) load8<TI>(x + row * ldx + (i * TPR + t) * 8, v[i]);
+  for (int i = 0; i < VPT; ++i) load8u<TI>(x + row * ldx + (i * TPR + t) * 8, v[i]);
   const float sl = scale * kLog2e;
   float m = -INFINITY;
   if (flags & SPH_SOFTMAX_CAUSAL) {
@@ -303,7 +351,94 @@ softmax_full(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t 
       for (int j = 0; j < 8; ++j) v[i][j] *= f;
   }
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) store8<TO>(y + row * ldy + (i * TPR + t) * 8, v[i]);
+  for (int i = 0; i < VPT; ++i) store8u<TO>(y + row * ldy + (i * TPR + t) * 8, v[i]);
+}
+
+// Rows of 8193 to 131072 16-bit columns (token log-probabilities over a
+// vocabulary): one 1024-thread workgroup per row, the row held in registers as
+// the 16-bit values it came as (VPT chunks of 8 per thread, 4 registers each:
+// as floats, 8 chunks spilled), one combined (max, sum) reduction, the
+// exponentials of the output taken again.  With few rows a CU's own rate sets
+// the time: 64 x 49155 bf16 log-softmax 35 us -> 9.9 us.
+template <typename TI, typename TO, int VPT>
+__global__ void __launch_bounds__(1024)
+softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t ldy, int cols,
+               float scale, int flags, int64_t qlen, int64_t qoff) {
+  static_assert(sizeof(TI) == 2, "16-bit rows");
+  __shared__ float lds_m[16], lds_s[16];
+  const int64_t row = blockIdx.x;
+  const TI* xr = x + row * ldx;
+  int limit = cols;
+  if (flags & SPH_SOFTMAX_CAUSAL) {
+    const int64_t lim = (row % qlen) + qoff + 1;
+    limit = lim < 0 ? 0 : (lim < cols ? static_cast<int>(lim) : cols);
+  }
+  // columns past the limit become -inf in the registers, so the passes below
+  // test nothing (a CU's vector ALUs are as busy as its memory path here)
+  constexpr uint32_t kNegInf = __is_same(TI, bf16_t) ? 0xff80u : 0xfc00u;
+  u32x4 raw[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c0 = (i * 1024 + threadIdx.x) * 8;
+    if (c0 + 8 <= cols)
+      raw[i] = *reinterpret_cast<const u32x4_any*>(xr + c0);
+    else
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t lo = c0 + 2 * j < cols ? __builtin_bit_cast(uint16_t, xr[c0 + 2 * j]) : kNegInf;
+        const uint32_t hi = c0 + 2 * j + 1 < cols ? __builtin_bit_cast(uint16_t, xr[c0 + 2 * j + 1]) : kNegInf;
+        raw[i][j] = lo | (hi << 16);
+      }
+  }
+  if (limit < cols) {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = (i * 1024 + threadIdx.x) * 8 + 2 * j;
+        if (c >= limit) raw[i][j] = (raw[i][j] & 0xffff0000u) | kNegInf;
+        if (c + 1 >= limit) raw[i][j] = (raw[i][j] & 0xffffu) | (kNegInf << 16);
+      }
+  }
+  const float sl = scale * kLog2e;  // log2 units; scale > 0
+  auto val = [&](int i, int j) {
+    const TI* e = reinterpret_cast<const TI*>(&raw[i]);
+    return Num<TI>::to_f(e[j]);
+  };
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, val(i, j));
+  m *= sl;
+  const float bt = m == -INFINITY ? 0.f : m;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f(fmaf(val(i, j), sl, -bt));
+  group_ms<1024>(m, s, lds_m, lds_s);
+  const bool lg = flags & SPH_SOFTMAX_LOG;
+  // (a row with no finite value is NaN in both forms: -inf - -inf)
+  const float off = lg ? m + log2f(s) : m, inv = 1.0f / s;
+  TO* yr = y + row * ldy;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c0 = (i * 1024 + threadIdx.x) * 8;
+    if (c0 >= cols) continue;
+    float v[8];
+    if (lg) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = fmaf(val(i, j), sl, -off) * kLn2;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_exp2f(fmaf(val(i, j), sl, -off)) * inv;
+    }
+    if (c0 + 8 <= cols)
+      store8u<TO>(yr + c0, v);
+    else
+      store8_partial<TO>(yr + c0, cols - c0, v);
+  }
 }
 
 // Rows longer than the register-resident configs: online max/sum pass, then
@@ -374,7 +509,7 @@ norm_regs(const T* __restrict__ x, const T* __restrict__ res,
       for (int j = 0; j < 8; ++j)  // round the sum to T, as an eager add would
         v[i][j] = Num<T>::to_f(Num<T>::from_f(v[i][j] + r[j]));
     }
-    if (valid && h != nullptr) store_row<T, TPR, VPT, VEC, true>(h + rr * cols, cols, t, v);
+    if (valid && h != nullptr) store_row<T, TPR, VPT, true, VEC>(h + rr * cols, cols, t, v);
   }
   const float inv_n = 1.0f / static_cast<float>(cols);
   float mean = 0.f;
@@ -421,7 +556,7 @@ norm_regs(const T* __restrict__ x, const T* __restrict__ res,
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[i][j] = fmaf((v[i][j] - mean) * rstd, wv[j], bv[j]);
   }
-  store_row<T, TPR, VPT, VEC, true>(y + row * cols, cols, t, v);
+  store_row<T, TPR, VPT, true, VEC>(y + row * cols, cols, t, v);
 }
 
 template <typename T, typename W, bool LAYER>
@@ -468,7 +603,7 @@ norm_looped(const T* __restrict__ x, const T* __restrict__ res,
 // ----------------------------------------------------------------------------
 // y = gelu_erf(x * s + b), rowsum = sum(y)
 // ----------------------------------------------------------------------------
-template <typename T, int TPR, int VPT, bool VEC>
+template <typename T, int TPR, int VPT>
 __global__ void __launch_bounds__(block_of<TPR>())
 gelu_rowsum_regs(const T* __restrict__ x, const T* __restrict__ sv,
                  const T* __restrict__ bv, float s0, float b0,
@@ -482,20 +617,20 @@ gelu_rowsum_regs(const T* __restrict__ x, const T* __restrict__ sv,
   const bool valid = row < rows;
   const int64_t rr = valid ? row : 0;
   float v[VPT][8];
-  load_row<T, TPR, VPT, VEC>(x + rr * cols, cols, t, 0.f, v);
+  load_row<T, TPR, VPT>(x + rr * cols, cols, t, 0.f, v);
   float acc = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
     const int64_t c0 = chunk_col<TPR>(i, t);
     float s[8], b[8];
     if (sv) {
-      load_chunk<T, VEC>(sv, cols, c0, 0.f, s);
+      load_chunk<T>(sv, cols, c0, 0.f, s);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) s[j] = s0;
     }
     if (bv) {
-      load_chunk<T, VEC>(bv, cols, c0, 0.f, b);
+      load_chunk<T>(bv, cols, c0, 0.f, b);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) b[j] = b0;
@@ -509,7 +644,7 @@ gelu_rowsum_regs(const T* __restrict__ x, const T* __restrict__ sv,
   }
   if (rowsum) acc = group_reduce<SumOp, TPR>(acc, lds);
   if (!valid) return;
-  if (y) store_row<T, TPR, VPT, VEC, true>(y + row * cols, cols, t, v);
+  if (y) store_row<T, TPR, VPT, true>(y + row * cols, cols, t, v);
   if (rowsum && t == 0) rowsum[row] = Num<T>::from_f(acc);
 }
 
@@ -645,30 +780,40 @@ int softmax_impl(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
                  int64_t qoff, hipStream_t st) {
   const TI* xi = static_cast<const TI*>(x);
   TO* yo = static_cast<TO*>(y);
-  const bool vec = vec_ok<TI>(x, ldx) && vec_ok<TO>(y, ldy);
-  if (vec && cols == 4096 && rows <= 0xffffffffLL * 2) {
+  if (cols == 4096 && rows <= 0xffffffffLL * 2) {
     // 128 threads x 4 chunks per row, two rows per workgroup (measured best
     // of the register layouts at [512, 4096])
     softmax_full<TI, TO, 128, 4><<<grid_rows<128>(rows), block_of<128>(), 0, st>>>(
         xi, ldx, yo, ldy, rows, scale, flags, qlen, qoff);
     return check_launch("sph_softmax_rows");
   }
+  if constexpr (sizeof(TI) == 2) {
+    if (cols > 8192 && cols <= 131072 && scale > 0.f) {
+      const unsigned g = static_cast<unsigned>(rows);
+      const int n = static_cast<int>(cols);
+      if (cols <= 16384)
+        softmax_packed<TI, TO, 2><<<g, 1024, 0, st>>>(xi, ldx, yo, ldy, n, scale, flags, qlen, qoff);
+      else if (cols <= 32768)
+        softmax_packed<TI, TO, 4><<<g, 1024, 0, st>>>(xi, ldx, yo, ldy, n, scale, flags, qlen, qoff);
+      else if (cols <= 65536)
+        softmax_packed<TI, TO, 8><<<g, 1024, 0, st>>>(xi, ldx, yo, ldy, n, scale, flags, qlen, qoff);
+      else
+        softmax_packed<TI, TO, 16><<<g, 1024, 0, st>>>(xi, ldx, yo, ldy, n, scale, flags, qlen, qoff);
+      return check_launch("sph_softmax_rows");
+    }
+  }
   const int cfg = pick_cfg(cols);
 #define SPH_SOFTMAX_CASE(I)                                                     \
   case I: {                                                                     \
     constexpr int TPR = kCfgs[I].tpr, VPT = kCfgs[I].vpt;                       \
-    if (vec && cols == TPR * VPT * 8)                                           \
+    if (cols == TPR * VPT * 8)                                                  \
       softmax_full<TI, TO, TPR, VPT><<<grid_rows<TPR>(rows), block_of<TPR>(),   \
                                        0, st>>>(xi, ldx, yo, ldy, rows, scale,  \
                                                 flags, qlen, qoff);             \
-    else if (vec)                                                               \
-      softmax_regs<TI, TO, TPR, VPT, true><<<grid_rows<TPR>(rows),              \
-                                             block_of<TPR>(), 0, st>>>(         \
-          xi, ldx, yo, ldy, rows, cols, scale, flags, qlen, qoff);              \
     else                                                                        \
-      softmax_regs<TI, TO, TPR, VPT, false><<<grid_rows<TPR>(rows),             \
-                                              block_of<TPR>(), 0, st>>>(        \
-          xi, ldx, yo, ldy, rows, cols, scale, flags, qlen, qoff);              \
+      softmax_regs<TI, TO, TPR, VPT><<<grid_rows<TPR>(rows), block_of<TPR>(),   \
+                                       0, st>>>(xi, ldx, yo, ldy, rows, cols,   \
+                                                scale, flags, qlen, qoff);      \
     break;                                                                      \
   }
   switch (cfg) {
@@ -676,9 +821,14 @@ int softmax_impl(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
     SPH_SOFTMAX_CASE(1)
     SPH_SOFTMAX_CASE(2)
     SPH_SOFTMAX_CASE(3)
-    SPH_SOFTMAX_CASE(4)
-    SPH_SOFTMAX_CASE(5)
     default:
+      if constexpr (sizeof(TI) == 4) {  // (16-bit rows: softmax_packed; looped for scale <= 0)
+        switch (cfg) {
+          SPH_SOFTMAX_CASE(4)
+          SPH_SOFTMAX_CASE(5)
+        }
+        if (cfg >= 0) break;
+      }
       softmax_looped<TI, TO><<<static_cast<unsigned>(rows), 256, 0, st>>>(
           xi, ldx, yo, ldy, rows, cols, scale, flags, qlen, qoff);
   }
@@ -773,14 +923,9 @@ int gelu_impl(const void* x, const void* s, const void* b, float s0, float b0,
 #define SPH_GELU_CASE(I)                                                       \
   case I: {                                                                      \
     constexpr int TPR = kCfgs[I].tpr, VPT = kCfgs[I].vpt;                        \
-    if (vec)                                                                     \
-      gelu_rowsum_regs<T, TPR, VPT, true><<<grid_rows<TPR>(rows),                \
-                                            block_of<TPR>(), 0, st>>>(           \
-          xi, si, bi, s0, b0, yo, ro, rows, cols);                               \
-    else                                                                         \
-      gelu_rowsum_regs<T, TPR, VPT, false><<<grid_rows<TPR>(rows),               \
-                                             block_of<TPR>(), 0, st>>>(          \
-          xi, si, bi, s0, b0, yo, ro, rows, cols);                               \
+    gelu_rowsum_regs<T, TPR, VPT><<<grid_rows<TPR>(rows), block_of<TPR>(), 0,    \
+                                    st>>>(xi, si, bi, s0, b0, yo, ro, rows,      \
+                                          cols);                                 \
     break;                                                                       \
   }
   switch (cfg) {
