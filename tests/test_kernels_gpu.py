@@ -719,6 +719,46 @@ def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype):
         assert bool((d[:, m] == 7.0).all()), "rows past M written"
 
 
+@pytest.mark.parametrize("batch,m,n,k,tb,share,epi,dtype", [
+    (1, 300, 500, 700, 0, 0, 0, torch.float16),       # N and K off 8: both operands padded
+    (1, 301, 505, 704, 0, 0, 3, torch.bfloat16),      # K whole: only B's rows padded
+    (1, 1001, 777, 1029, 1, 0, 2, torch.float16),     # K-contiguous B, odd K
+    (1, 5, 2001, 1001, 0, 0, 0, torch.float16),       # few rows
+    (1, 1300, 1283, 515, 0, 0, 0, torch.bfloat16),    # 256-row tiles on padded operands
+    (3, 130, 777, 200, 0, 0, 0, torch.float16),       # batched, odd N
+    (3, 257, 129, 301, 0, 1, 2, torch.bfloat16)])     # one B for the batch
+def test_gemm_operands_off_16_bytes(batch, m, n, k, tb, share, epi, dtype):
+    # contiguous operands whose rows are off 16-byte chunks, with the
+    # workspace (padded copies where the model takes them) and without it
+    _log(f"gemm off 16 bytes {batch}x{m}x{n}x{k} tb={tb} share={share} epi={epi} {dtype}")
+    A = uniform((batch, m, k), k=61, dtype=dtype)
+    nb = 1 if share else batch
+    W = (uniform((nb, n, k) if tb else (nb, k, n), k=62, dtype=dtype).float() * 0.05).to(dtype)
+    bias = uniform((n,), k=63, dtype=dtype)
+    # the elements next to the operands must not enter the product
+    ad = torch.full((A.numel() + 16,), float("nan"), dtype=dtype, device=DEV)
+    ad[:A.numel()] = A.flatten().to(DEV)
+    wd = torch.full((W.numel() + 16,), float("nan"), dtype=dtype, device=DEV)
+    wd[:W.numel()] = W.flatten().to(DEV)
+    bd = bias.to(DEV)
+    wf = W.float().numpy()
+    want = O.gemm(A.float().numpy(), np.swapaxes(wf, 1, 2) if tb else wf, alpha=0.75, beta=0.5,
+                  c=bias.float().numpy()[None, None, :],
+                  epilogue={0: "none", 2: "gelu", 3: "silu"}[epi])
+    tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    nws = _capi.lib().sph_gemm_workspace_bytes(batch, m, n, k)
+    assert nws > 0
+    ws = torch.full((nws,), 255, dtype=torch.uint8, device=DEV)
+    for w_n in (0, nws, nws - 256):
+        d = torch.full((batch, m + 1, n), 7.0, dtype=dtype, device=DEV)
+        _capi.call("sph_gemm_ex", DT[dtype], 0, tb, batch, m, n, k, 0.75, _p(ad), k, m * k, _p(wd),
+                   k if tb else n, 0 if share else n * k, 0.5, _p(bd), 0, 1, 0, _p(d), n,
+                   (m + 1) * n, epi, _p(ws) if w_n else None, w_n, _stream())
+        _sync()
+        assert_close_fp(d[:, :m], want, out_dtype=dtype, what="unaligned gemm", **tol)
+        assert bool((d[:, m] == 7.0).all()), "rows past M written"
+
+
 @pytest.mark.parametrize("m,n,k,pad", [(9, 512, 4096, 0), (24, 1000, 520, 8), (100, 513, 512, 0),
                                        (333, 1280, 1024, 0), (1100, 1280, 2048, 8),
                                        (2, 64, 40, 0)])

@@ -90,7 +90,8 @@ void gemm2d(const at::Tensor& a, const at::Tensor& b, const at::Tensor& d, float
     check_extent(ce, cp, 2, cs, cst, ce.element_size(), "addmm input");
   }
   c10::DeviceGuard guard(d.device());
-  // workspace for a split-K last round of tiles, when the shape has one
+  // workspace for K slices' partial sums, or for padded copies of operands
+  // off 16-byte chunks, when the shape has either
   const int64_t nws = sph_gemm_workspace_bytes(1, m, n, k);
   at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
   SPYRE_SPH_CHECK(sph_gemm_ex(to_sph(d.scalar_type()), va.trans, vb.trans, 1, m, n, k, alpha,
@@ -142,10 +143,13 @@ void gemm3d(const at::Tensor& a_in, const at::Tensor& b_in, const at::Tensor& d,
     check_extent(ce, cp, 3, cs, cst, ce.element_size(), "baddbmm input");
   }
   c10::DeviceGuard guard(d.device());
-  SPYRE_SPH_CHECK(sph_gemm_strided_batched(
+  // workspace for padded copies of operands off 16-byte chunks
+  const int64_t nws = sph_gemm_workspace_bytes(bs, m, n, k);
+  at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
+  SPYRE_SPH_CHECK(sph_gemm_ex(
       to_sph(d.scalar_type()), va.trans, vb.trans, bs, m, n, k, alpha, va.ptr, va.ld, sa, vb.ptr,
       vb.ld, sb, cp ? beta : 0.f, cp, ldc_r, ldc_c, sc, dd.data_ptr(), n, m * n, SPH_EPI_NONE,
-      stream(d.get_device())));
+      ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? nws : 0, stream(d.get_device())));
   if (!d_ok) device_copy(d, dd);
 }
 

@@ -147,7 +147,7 @@ __global__ void __launch_bounds__((dl::Cfg<BN_, WTN_>::NT)) gemm_dl_kernel(const
   // Buffer ranges: exactly the bytes this tile's rows (columns) span, so the
   // rows of a last, partial tile that lie past M or N read zeros (and are
   // not stored).
-  const int64_t arows = min(static_cast<int64_t>(BM), p.m - m0), brows = min(static_cast<int64_t>(BN), p.n - n0);
+  const int64_t arows = min(static_cast<int64_t>(BM), p.m - m0), brows = min(static_cast<int64_t>(BN), (B_KCONT ? p.n : p.nb) - n0);
   const i32x4 ra = buffer_rsrc(A + m0 * lda, static_cast<uint32_t>(((arows - 1) * lda + p.k) * 2));
   // (SwiGLU: from gate row n0 to up row n + n0 + 127)
   const i32x4 rb = SWIGLU
@@ -444,7 +444,8 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce(const GemmArgs p) {
          (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(out[1]))) << 16);
   w[1] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(out[2]))) |
          (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(out[3]))) << 16);
-  *reinterpret_cast<u32x2*>(D + row * p.ldd + col) = w;
+  typedef u32x2 u32x2_any __attribute__((aligned(2)));
+  *reinterpret_cast<u32x2_any*>(D + row * p.ldd + col) = w;
 }
 
 // ---------------------------------------------------------------------------
@@ -995,7 +996,7 @@ inline GemmRoute gemm_route(const GemmArgs& p, int64_t batch, bool a_kcont, bool
   // kernel's single stage is ahead (64^3: 3.0 us against 3.3)
   if (p.k <= 64 && !(p.m % dl::BM == 0 && p.n % 128 == 0) &&
       ceil_div(p.m, 64) * ceil_div(p.n, 64) * batch <= kNumCUs) return r;
-  if (a_kcont && p.k % dl::BKD == 0 && p.k > 0 && p.vec_a && p.vec_b && (b_kcont || p.n % 8 == 0))
+  if (a_kcont && p.k % dl::BKD == 0 && p.k > 0 && p.vec_a && p.vec_b && (b_kcont || p.nb % 8 == 0))
     r.dc = dl_choice(p, batch, b_kcont);
   if (ring_fits(p, a_kcont, b_kcont, false)) {
     r.rp = ring_plan(batch, p.m, p.n, p.k, b_kcont, false, p.part_bytes);
@@ -1051,6 +1052,128 @@ inline bool shortk_fits(const GemmArgs& p, bool a_kcont, bool b_kcont) {
 
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Operands off 16-byte chunks (an odd K, rows of odd length): with a
+// workspace they are copied into rows of whole chunks, zero-padded (K to a
+// multiple of 64 where it is not one of 8), and the product runs on the
+// kernels above.  Taken where the time models put copy and product 10 % ahead
+// of the register-staged kernel: per K column of a round of its 64 x 64 tiles
+// 75 ns with row-major B (its transposing loader), 14 with K-contiguous B; 48
+// and 25 for 128 x 128 tiles; the copy ~3 us + its bytes at 4.5 TB/s.
+// (3001 x 3003 x 3005 row-major: 329 us register-staged, 85 padded; 1501 x 999
+// x 2003 191 / 28; 333 x 4099 x 4099 K-contiguous 69 / 44.)
+struct PackPlan {
+  bool use = false;
+  bool a = false, b = false;     // operands to copy
+  int64_t kp = 0, np = 0;        // padded K, padded columns of a row-major B
+  int64_t a_bytes = 0, bytes = 0;
+};
+constexpr int64_t kPackLimit = int64_t{256} << 20;
+
+inline GemmArgs packed_args(const GemmArgs& p, int64_t batch, bool b_kcont, const PackPlan& pp) {
+  GemmArgs q = p;
+  char* w = reinterpret_cast<char*>(p.part);
+  q.k = pp.kp;
+  if (pp.a) {
+    q.a = w;
+    q.lda = pp.kp;
+    q.stride_a = batch == 1 || p.stride_a == 0 ? 0 : p.m * pp.kp;
+    q.vec_a = 1;
+  }
+  if (pp.b) {
+    q.b = w + pp.a_bytes;
+    q.ldb = b_kcont ? pp.kp : pp.np;
+    q.stride_b = batch == 1 || p.stride_b == 0 ? 0 : (b_kcont ? p.n : pp.kp) * q.ldb;
+    q.vec_b = 1;
+    q.nb = pp.np;
+  }
+  q.part_bytes = p.part_bytes > pp.bytes ? p.part_bytes - pp.bytes : 0;
+  q.part = q.part_bytes > 0 ? reinterpret_cast<float*>(w + pp.bytes) : nullptr;
+  return q;
+}
+
+inline PackPlan pack_plan(const GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont) {
+  PackPlan pp;
+  const bool k8 = p.k % 8 == 0;
+  if (!a_kcont || p.k < 64 || p.part == nullptr) return pp;
+  pp.a = !p.vec_a || !k8;
+  pp.b = !p.vec_b || !k8 || (!b_kcont && p.nb % 8 != 0);
+  if (!pp.a && !pp.b) return pp;
+  pp.kp = k8 ? p.k : ceil_div(p.k, dl::BKD) * dl::BKD;
+  pp.np = b_kcont ? p.n : ceil_div(p.n, 8) * 8;
+  const int64_t ba = batch > 1 && p.stride_a == 0 ? 1 : batch, bb = batch > 1 && p.stride_b == 0 ? 1 : batch;
+  if (p.m > kPackLimit || p.n > kPackLimit || p.k > kPackLimit || batch > 65535) return pp;
+  if (static_cast<double>(ba) * p.m * pp.kp > kPackLimit || static_cast<double>(bb) * pp.np * pp.kp > kPackLimit)
+    return pp;
+  pp.a_bytes = pp.a ? (ba * p.m * pp.kp * 2 + 255) / 256 * 256 : 0;
+  pp.bytes = pp.a_bytes + (pp.b ? (bb * pp.np * pp.kp * 2 + 255) / 256 * 256 : 0);
+  if (pp.bytes > kPackLimit || pp.bytes > p.part_bytes) return pp;
+  const GemmRoute r = gemm_route(packed_args(p, batch, b_kcont, pp), batch, true, b_kcont);
+  const double us = 3.0 + 2.0 * static_cast<double>(pp.bytes) / 4.5e6 +
+                    (r.ring ? r.rp.us : r.dc.kind != 0 ? r.dc.us : 1e30);
+  const int64_t t128 = ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
+  const int64_t t64 = ceil_div(p.m, 64) * ceil_div(p.n, 64) * batch;
+  const double k = static_cast<double>(p.k);
+  const double staged =
+      t128 >= 128 ? 5.0 + k * (b_kcont ? 0.025 : 0.048) * std::max(1.0, static_cast<double>(t128) / kNumCUs)
+                  : 5.0 + k * (b_kcont ? 0.014 : 0.075) * std::max(1.0, static_cast<double>(t64) / (2 * kNumCUs));
+  // (short K on many tiles: the output is the cost, the copies only add to
+  // it; 8 x 1001 x 777 x 128: 14.9 us register-staged, 18.2 padded)
+  pp.use = us < 0.9 * staged && (p.k >= 256 || t128 < 128);
+  return pp;
+}
+
+// One thread per 8-element chunk of a padded operand; blockIdx.y: operand.
+struct PackOp {
+  const uint16_t* src;
+  int64_t ld, stride;
+  uint16_t* dst;
+  int rows, cols;
+  uint32_t drows, dchunks;  // padded extent (chunks of 8)
+  int batches;
+};
+__global__ void __launch_bounds__(256) gemm_pack_kernel(PackOp o0, PackOp o1) {
+  const PackOp& o = blockIdx.y == 0 ? o0 : o1;
+  const uint32_t idx = blockIdx.x * 256 + threadIdx.x;  // (at most 2^24 chunks)
+  if (idx >= static_cast<uint32_t>(o.batches) * o.drows * o.dchunks) return;
+  const uint32_t rowi = idx / o.dchunks;
+  const int c = static_cast<int>(idx - rowi * o.dchunks) * 8;
+  const int b = static_cast<int>(rowi / o.drows), r = static_cast<int>(rowi - b * o.drows);
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (r < o.rows) {
+    const uint16_t* s = o.src + b * o.stride + r * o.ld + c;
+    if (c + 8 <= o.cols) {
+      v = *reinterpret_cast<const u32x4_any*>(s);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (c + e < o.cols) v[e >> 1] |= static_cast<uint32_t>(s[e]) << (16 * (e & 1));
+    }
+  }
+  *reinterpret_cast<u32x4*>(o.dst + static_cast<int64_t>(idx) * 8) = v;
+}
+
+inline void launch_pack(const GemmArgs& p, const GemmArgs& q, int64_t batch, bool b_kcont,
+                        const PackPlan& pp, hipStream_t st) {
+  const uint32_t kc = static_cast<uint32_t>(pp.kp / 8);
+  PackOp oa{}, ob{};
+  if (pp.a)
+    oa = {static_cast<const uint16_t*>(p.a), p.lda, p.stride_a, static_cast<uint16_t*>(const_cast<void*>(q.a)),
+          static_cast<int>(p.m), static_cast<int>(p.k), static_cast<uint32_t>(p.m), kc,
+          static_cast<int>(q.stride_a == 0 ? 1 : batch)};
+  if (pp.b) {
+    const int rows = static_cast<int>(b_kcont ? p.n : p.k), cols = static_cast<int>(b_kcont ? p.k : p.n);
+    ob = {static_cast<const uint16_t*>(p.b), p.ldb, p.stride_b, static_cast<uint16_t*>(const_cast<void*>(q.b)),
+          rows, cols, static_cast<uint32_t>(b_kcont ? p.n : pp.kp),
+          b_kcont ? kc : static_cast<uint32_t>(pp.np / 8),
+          static_cast<int>(q.stride_b == 0 ? 1 : batch)};
+  }
+  if (!pp.a) oa = ob;
+  const auto chunks = [](const PackOp& o) { return static_cast<int64_t>(o.batches) * o.drows * o.dchunks; };
+  const int64_t most = std::max(chunks(oa), chunks(ob));
+  const dim3 grid(static_cast<unsigned>(ceil_div(most, 256)), pp.a && pp.b ? 2 : 1);
+  gemm_pack_kernel<<<grid, 256, 0, st>>>(oa, ob);
+}
+
 // Small row counts on the streaming kernels, short K on theirs, then the
 // direct-load and ring kernels; what neither takes (A transposed, K or rows
 // off 16-byte chunks) on the register-staged kernel: 256x256 tiles when they
@@ -1092,6 +1215,12 @@ int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont,
     }
     return check_launch("sph_gemm (short K)");
   }
+  const PackPlan pp = pack_plan(p, batch, a_kcont, b_kcont);
+  if (pp.use) {
+    GemmArgs q = packed_args(p, batch, b_kcont, pp);
+    launch_pack(p, q, batch, b_kcont, pp, st);
+    return gemm_dispatch<T>(q, batch, true, b_kcont, st);  // (aligned: packs nothing)
+  }
   const GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
   if (r.ring) return launch_ring(__is_same(T, bf16_t), p, batch, b_kcont, false, r.rp, st);
   switch (r.dc.kind) {
@@ -1131,7 +1260,7 @@ int gemm_entry(sph_dtype dtype, int trans_a, int trans_b, int64_t batch, int64_t
               "gemm: too many tiles");
   GemmArgs p{};
   p.m = m;
-  p.n = n;
+  p.n = p.nb = n;
   p.k = k;
   p.a = a;
   p.lda = lda;
@@ -1156,8 +1285,7 @@ int gemm_entry(sph_dtype dtype, int trans_a, int trans_b, int64_t batch, int64_t
   p.vec_a = al16(a) && (lda % 8 == 0) && (batch == 1 || stride_a % 8 == 0);
   p.vec_b = al16(b) && (ldb % 8 == 0) && (batch == 1 || stride_b % 8 == 0);
   p.vec_d = al16(d) && (ldd % 8 == 0) && (batch == 1 || stride_d % 8 == 0);
-  p.part = workspace != nullptr && workspace_bytes > 0 && p.vec_d ? static_cast<float*>(workspace)
-                                                                  : nullptr;
+  p.part = workspace != nullptr && workspace_bytes > 0 ? static_cast<float*>(workspace) : nullptr;
   p.part_bytes = p.part != nullptr ? workspace_bytes : 0;
   hipStream_t st = as_stream(stream);
   if (dtype == SPH_F16) return gemm_dispatch<half_t>(p, batch, a_kcont, b_kcont, st);
@@ -1177,22 +1305,29 @@ extern "C" int sph_gemm_strided_batched(
 }
 
 // A call's own layout, alignment and workspace decide its kernel; the size
-// covers each layout of B at 16-byte aligned rows.
+// covers each layout of B with contiguous operands.
 extern "C" int64_t sph_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  if (batch != 1 || m <= 0 || n <= 0 || k <= 0 || k % 8 != 0) return 0;
+  if (batch <= 0 || m <= 0 || n <= 0 || k <= 0) return 0;
+  if (batch != 1 && k % 8 == 0 && n % 8 == 0) return 0;
   int64_t bytes = 0;
   for (int b_kcont = 0; b_kcont < 2; ++b_kcont) {
     GemmArgs p{};
     p.m = m;
-    p.n = n;
-    p.k = k;
-    p.lda = k;
-    p.ldb = b_kcont ? k : (n + 7) / 8 * 8;
-    p.vec_a = p.vec_b = p.vec_d = 1;
-    p.part = reinterpret_cast<float*>(uintptr_t{16});
+    p.n = p.nb = n;
+    p.k = p.lda = k;
+    p.ldb = b_kcont ? k : n;
+    p.stride_a = m * k;
+    p.stride_b = n * k;
+    p.vec_a = k % 8 == 0;
+    p.vec_b = p.ldb % 8 == 0;
+    p.vec_d = 1;
+    p.part = reinterpret_cast<float*>(uintptr_t{256});
     p.part_bytes = INT64_MAX;
-    const GemmRoute r = gemm_route(p, 1, true, b_kcont != 0);
-    const int64_t need = r.ring ? r.rp.bytes : r.dc.split.splits > 1 ? r.dc.split.bytes : 0;
+    const PackPlan pp = pack_plan(p, batch, true, b_kcont != 0);
+    if (pp.use) p = packed_args(p, batch, b_kcont != 0, pp);
+    const GemmRoute r = gemm_route(p, batch, true, b_kcont != 0);
+    const int64_t split = r.ring ? r.rp.bytes : r.dc.split.splits > 1 ? r.dc.split.bytes : 0;
+    const int64_t need = (pp.use ? pp.bytes : 0) + split;
     bytes = bytes > need ? bytes : need;
   }
   return bytes;
@@ -1234,7 +1369,7 @@ SwigluRoute swiglu_route(const GemmArgs& p, int64_t ws_bytes) {
   constexpr int64_t kLim = 1LL << 31;
   const int64_t tiles = ceil_div(p.m, dl::BM) * (p.n / 128);
   double us = 0;
-  if (p.n % 128 == 0 && p.k > 0 && p.k % dl::BKD == 0 && p.vec_d && ((dl::BM - 1) * p.lda + p.k) * 2 < kLim &&
+  if (p.n % 128 == 0 && p.k > 0 && p.k % dl::BKD == 0 && ((dl::BM - 1) * p.lda + p.k) * 2 < kLim &&
       ((p.n + 127) * p.ldb + p.k) * 2 < kLim && tiles < kLim) {
     r.dl = true;
     us = dl_est256(tiles, p.k);
@@ -1317,7 +1452,6 @@ extern "C" int64_t sph_gemm_swiglu_workspace_bytes(int64_t m, int64_t n, int64_t
   p.n = n;
   p.k = p.lda = p.ldb = k;
   p.vec_a = p.vec_b = 1;
-  p.vec_d = n % 8 == 0;
   const SwigluRoute r = swiglu_route(p, INT64_MAX);
   return r.ring ? r.rp.bytes : r.split.bytes;
 }

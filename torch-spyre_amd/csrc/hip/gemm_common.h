@@ -42,6 +42,8 @@ struct GemmArgs {
   float norm_eps;
   // Batch entries (persistent kernels, whose grid does not carry them).
   int64_t batches;
+  // Readable columns of a row-major B's rows (n, or n padded to whole chunks).
+  int64_t nb;
 };
 
 namespace {

@@ -18,7 +18,7 @@ RingPlan ring_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool b_kcont,
                    int64_t max_bytes);
 
 // What the kernel asks of a call: K-contiguous A, whole 16-byte chunks
-// (K % 8, for row-major B N % 8), 32-bit offsets.
+// (K % 8, for row-major B nb % 8), 32-bit offsets.
 bool ring_fits(const GemmArgs& p, bool a_kcont, bool b_kcont, bool swiglu);
 
 // p.part must hold plan.bytes.

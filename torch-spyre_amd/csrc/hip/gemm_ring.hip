@@ -34,13 +34,14 @@ __device__ inline void store4(const GemmArgs& p, T* D, f32x4 v, int64_t bz, int 
       if (col + e < p.n) v[e] = epilogue_one<T>(p, v[e], bz, row, col + e);
   }
   T* dp = D + row * p.ldd + col;
-  if (p.vec_d && col + 4 <= p.n) {
+  if (col + 4 <= p.n) {
     u32x2 w;
 #pragma unroll
     for (int e = 0; e < 2; ++e)
       w[e] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e]))) |
              (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e + 1]))) << 16);
-    *reinterpret_cast<u32x2*>(dp) = w;
+    typedef u32x2 u32x2_any __attribute__((aligned(2)));
+    *reinterpret_cast<u32x2_any*>(dp) = w;
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -124,7 +125,9 @@ __global__ void __launch_bounds__(NW_ * 64) gemm_ring_kernel(const GemmArgs p) {
   const uint16_t* B = static_cast<const uint16_t*>(p.b) + bz * p.stride_b +
                       (B_KCONT ? static_cast<int64_t>(n0) * ldb : n0);
   const int arows = min(BM, m - m0);
-  const int brows = SWIGLU ? 2 * n - n0 : min(BN, n - n0);  // row-major B: columns
+  const int brows = SWIGLU    ? 2 * n - n0
+                    : B_KCONT ? min(BN, n - n0)
+                              : min(BN, static_cast<int>(p.nb) - n0);  // columns
   const i32x4 ra = buffer_rsrc(A, static_cast<uint32_t>((arows - 1) * lda + k) * 2u);
   const i32x4 rb = buffer_rsrc(B, B_KCONT ? static_cast<uint32_t>((brows - 1) * ldb + k) * 2u
                                           : static_cast<uint32_t>((k - 1) * ldb + brows) * 2u);
@@ -390,7 +393,7 @@ RingPlan ring_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool b_kcont,
 bool ring_fits(const GemmArgs& p, bool a_kcont, bool b_kcont, bool swiglu) {
   constexpr int64_t kLim = (int64_t{1} << 31) - 1;
   if (!a_kcont || !p.vec_a || !p.vec_b || p.k <= 0 || p.k % 8 != 0) return false;
-  if (!b_kcont && p.n % 8 != 0) return false;
+  if (!b_kcont && p.nb % 8 != 0) return false;
   if (p.m >= kLim / 4 || p.n >= kLim / 4 || p.k >= kLim / 4) return false;
   if (p.lda > kLim / 4 || p.ldb > kLim / 4) return false;
   const int64_t brows = swiglu ? 2 * p.n : 128;

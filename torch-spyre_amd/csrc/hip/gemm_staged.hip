@@ -73,7 +73,7 @@ struct KContLoader {
   template <bool FULL>
   __device__ inline void issue(const uint16_t* __restrict__ base, int64_t ld,
                                int64_t r0, int64_t nrows, int64_t k0,
-                               int64_t kdim, bool vec) {
+                               int64_t kdim) {
     const int t = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < PER_T; ++i) {
@@ -81,8 +81,10 @@ struct KContLoader {
       const int r = idx >> 3, c = idx & 7;
       const int64_t gr = r0 + r, gk = k0 + c * 8;
       if ((ROWS * 8) % NT != 0 && idx >= ROWS * 8) continue;
-      if (FULL || (gr < nrows && vec && gk + 8 <= kdim)) {
+      if (FULL) {
         reg[i] = *reinterpret_cast<const u32x4*>(base + gr * ld + gk);
+      } else if (gr < nrows && gk + 8 <= kdim) {
+        reg[i] = *reinterpret_cast<const u32x4_any*>(base + gr * ld + gk);
       } else if (gr < nrows && gk < kdim) {
         const int64_t n = kdim - gk;
         reg[i] = load_partial(base + gr * ld + gk, n > 8 ? 8 : static_cast<int>(n), 1);
@@ -118,7 +120,7 @@ struct KStridedLoader {
   template <bool FULL>
   __device__ inline void issue(const uint16_t* __restrict__ base, int64_t ld,
                                int64_t r0, int64_t nrows, int64_t k0,
-                               int64_t kdim, bool vec) {
+                               int64_t kdim) {
     const int t = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < PER_T; ++i) {
@@ -129,8 +131,10 @@ struct KStridedLoader {
 #pragma unroll
       for (int kr = 0; kr < 8; ++kr) {
         const int64_t gk = k0 + kb * 8 + kr;
-        if (FULL || (gk < kdim && vec && gr + 8 <= nrows)) {
+        if (FULL) {
           reg[i][kr] = *reinterpret_cast<const u32x4*>(base + gk * ld + gr);
+        } else if (gk < kdim && gr + 8 <= nrows) {
+          reg[i][kr] = *reinterpret_cast<const u32x4_any*>(base + gk * ld + gr);
         } else if (gk < kdim && gr < nrows) {
           const int64_t n = nrows - gr;
           reg[i][kr] = load_partial(base + gk * ld + gr, n > 8 ? 8 : static_cast<int>(n), 1);
@@ -250,13 +254,13 @@ gemm_kernel(const GemmArgs p) {
     // last tile are clamped, re-loading and re-writing the last tile into
     // the idle buffer, which nothing reads afterwards.
     const int64_t klast = (ksteps - 1) * BK;
-    la.template issue<true>(A, p.lda, m0, p.m, 0, p.k, true);
-    lb.template issue<true>(B, p.ldb, n0, p.n, 0, p.k, true);
+    la.template issue<true>(A, p.lda, m0, p.m, 0, p.k);
+    lb.template issue<true>(B, p.ldb, n0, p.n, 0, p.k);
     la.commit(lds);
     lb.commit(lds + BM * BK);
     const int64_t k1 = BK < klast ? BK : klast;
-    la.template issue<true>(A, p.lda, m0, p.m, k1, p.k, true);
-    lb.template issue<true>(B, p.ldb, n0, p.n, k1, p.k, true);
+    la.template issue<true>(A, p.lda, m0, p.m, k1, p.k);
+    lb.template issue<true>(B, p.ldb, n0, p.n, k1, p.k);
     __syncthreads();
     for (int64_t ks = 0; ks < ksteps; ++ks) {
       const int cur = static_cast<int>(ks & 1);
@@ -278,8 +282,8 @@ gemm_kernel(const GemmArgs p) {
       la.commit(lds + (cur ^ 1) * STAGE);
       lb.commit(lds + (cur ^ 1) * STAGE + BM * BK);
       const int64_t k2 = (ks + 2) * BK < klast ? (ks + 2) * BK : klast;
-      la.template issue<true>(A, p.lda, m0, p.m, k2, p.k, true);
-      lb.template issue<true>(B, p.ldb, n0, p.n, k2, p.k, true);
+      la.template issue<true>(A, p.lda, m0, p.m, k2, p.k);
+      lb.template issue<true>(B, p.ldb, n0, p.n, k2, p.k);
       // Instruction order for the scheduler (one wave per SIMD, so latency
       // must be hidden inside the wave): fragment reads of sub-step 0;
       // sub-steps 0-2 alternate MFMAs with the next sub-step's fragment
@@ -311,8 +315,8 @@ gemm_kernel(const GemmArgs p) {
     }
   } else {
     if (ksteps > 0) {
-      la.template issue<false>(A, p.lda, m0, p.m, 0, p.k, p.vec_a);
-      lb.template issue<false>(B, p.ldb, n0, p.n, 0, p.k, p.vec_b);
+      la.template issue<false>(A, p.lda, m0, p.m, 0, p.k);
+      lb.template issue<false>(B, p.ldb, n0, p.n, 0, p.k);
       la.commit(lds);
       lb.commit(lds + BM * BK);
       __syncthreads();
@@ -321,8 +325,8 @@ gemm_kernel(const GemmArgs p) {
       const int cur = static_cast<int>(ks & 1);
       const bool more = ks + 1 < ksteps;
       if (more) {
-        la.template issue<false>(A, p.lda, m0, p.m, (ks + 1) * BK, p.k, p.vec_a);
-        lb.template issue<false>(B, p.ldb, n0, p.n, (ks + 1) * BK, p.k, p.vec_b);
+        la.template issue<false>(A, p.lda, m0, p.m, (ks + 1) * BK, p.k);
+        lb.template issue<false>(B, p.ldb, n0, p.n, (ks + 1) * BK, p.k);
       }
       const uint16_t* sa = lds + cur * STAGE;
       const uint16_t* sb = sa + BM * BK;

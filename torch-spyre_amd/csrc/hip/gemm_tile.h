@@ -52,7 +52,7 @@ __device__ __attribute__((always_inline)) inline void store_slab_impl(const Gemm
   const int er = lane / LPR, ec = (lane % LPR) * 8;
   const int64_t col = col0 + ec;
   if (er >= RPP || col >= p.n) return;
-  const bool full_cols = p.vec_d && col + 8 <= p.n;
+  const bool full_cols = col + 8 <= p.n;
   const int ncols = p.n - col >= 8 ? 8 : static_cast<int>(p.n - col);
   // Lanes whose 8-column group has bit 3 set read the two 16-byte halves
   // in the opposite order, so each LDS read cycle touches 64 distinct banks.
@@ -99,7 +99,7 @@ __device__ __attribute__((always_inline)) inline void store_slab_impl(const Gemm
     // output leaves in one burst (4096^3: 1305-1316 -> 1335-1337 TFLOP/s,
     // alternating builds on one box; the c4 / c5 decoder unchanged)
     if (full_cols)
-      store8<T, true>(dp, v);
+      p.vec_d ? store8<T, true>(dp, v) : store8u<T, true>(dp, v);
     else
       store8_partial<T>(dp, ncols, v);
   };
