@@ -244,8 +244,9 @@ int sph_gemm_swiglu_any(sph_dtype dtype, int64_t m, int64_t n, int64_t k, const 
  * with at least sph_gemm_workspace_bytes(batch, m, n, k) bytes, a product
  * whose tiles would leave CUs idle (few rows, or a partial last round of 256
  * x 256 tiles) may split its K range into fp32 partial tiles, summed and
- * finished with the epilogue by a second kernel; the size is 0 for shapes
- * where the library's time model prefers whole tiles.  Same results up to fp32 summation order.  No
+ * finished with the epilogue by a second kernel, and operands off 16-byte
+ * chunks (k % 8, rows of odd length) may be copied into padded rows; the
+ * size is 0 for shapes where the library's time model does neither.  Same results up to fp32 summation order.  No
  * counterpart in the reference (its GEMM is one device call,
  * spyre_torch_ops.cpp:214-293); calls sharing a workspace must be ordered
  * on a stream. */
@@ -256,6 +257,9 @@ int sph_gemm_ex(sph_dtype dtype, int trans_a, int trans_b, int64_t batch, int64_
                 int64_t stride_d, int epilogue, void* workspace, int64_t workspace_bytes,
                 sph_stream_t stream);
 int64_t sph_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k);
+/* The size for one call's own layout and leading dimensions. */
+int64_t sph_gemm_workspace_bytes_ex(int trans_a, int trans_b, int64_t batch, int64_t m, int64_t n,
+                                    int64_t k, int64_t lda, int64_t ldb);
 
 /* fp16 shorthands: contiguous row-major, no transpose, no C. */
 int sph_gemm_f16(int64_t m, int64_t n, int64_t k, const void* a,

@@ -92,7 +92,7 @@ void gemm2d(const at::Tensor& a, const at::Tensor& b, const at::Tensor& d, float
   c10::DeviceGuard guard(d.device());
   // workspace for K slices' partial sums, or for padded copies of operands
   // off 16-byte chunks, when the shape has either
-  const int64_t nws = sph_gemm_workspace_bytes(1, m, n, k);
+  const int64_t nws = sph_gemm_workspace_bytes_ex(va.trans, vb.trans, 1, m, n, k, va.ld, vb.ld);
   at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
   SPYRE_SPH_CHECK(sph_gemm_ex(to_sph(d.scalar_type()), va.trans, vb.trans, 1, m, n, k, alpha,
                               va.ptr, va.ld, 0, vb.ptr, vb.ld, 0, cp ? beta : 0.f, cp, ldc_r,
@@ -144,7 +144,7 @@ void gemm3d(const at::Tensor& a_in, const at::Tensor& b_in, const at::Tensor& d,
   }
   c10::DeviceGuard guard(d.device());
   // workspace for padded copies of operands off 16-byte chunks
-  const int64_t nws = sph_gemm_workspace_bytes(bs, m, n, k);
+  const int64_t nws = sph_gemm_workspace_bytes_ex(va.trans, vb.trans, bs, m, n, k, va.ld, vb.ld);
   at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
   SPYRE_SPH_CHECK(sph_gemm_ex(
       to_sph(d.scalar_type()), va.trans, vb.trans, bs, m, n, k, alpha, va.ptr, va.ld, sa, vb.ptr,

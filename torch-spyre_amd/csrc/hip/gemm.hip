@@ -1304,33 +1304,45 @@ extern "C" int sph_gemm_strided_batched(
                     nullptr, 0, stream);
 }
 
-// A call's own layout, alignment and workspace decide its kernel; the size
-// covers each layout of B with contiguous operands.
+namespace {
+// Workspace that a call with these operands can use: padded copies and K
+// slices' partial sums.
+int64_t workspace_need(int64_t batch, int64_t m, int64_t n, int64_t k, bool b_kcont, int64_t lda,
+                       int64_t ldb) {
+  const bool al = lda % 8 == 0 && ldb % 8 == 0 && k % 8 == 0 && (b_kcont || n % 8 == 0);
+  // (host time of small calls: no copy, and K too short or rows too few to slice)
+  if (al && (batch != 1 || k < 512 || (b_kcont && m <= kSmallRows))) return 0;
+  GemmArgs p{};
+  p.m = m;
+  p.n = p.nb = n;
+  p.k = k;
+  p.lda = lda;
+  p.ldb = ldb;
+  p.stride_a = m * k;
+  p.stride_b = n * k;
+  p.vec_a = lda % 8 == 0;
+  p.vec_b = ldb % 8 == 0;
+  p.vec_d = 1;
+  p.part = reinterpret_cast<float*>(uintptr_t{256});
+  p.part_bytes = INT64_MAX;
+  const PackPlan pp = pack_plan(p, batch, true, b_kcont);
+  if (pp.use) p = packed_args(p, batch, b_kcont, pp);
+  const GemmRoute r = gemm_route(p, batch, true, b_kcont);
+  const int64_t split = r.ring ? r.rp.bytes : r.dc.split.splits > 1 ? r.dc.split.bytes : 0;
+  return (pp.use ? pp.bytes : 0) + split;
+}
+}  // namespace
+
+// (for contiguous operands, either layout of B)
 extern "C" int64_t sph_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k) {
   if (batch <= 0 || m <= 0 || n <= 0 || k <= 0) return 0;
-  if (batch != 1 && k % 8 == 0 && n % 8 == 0) return 0;
-  int64_t bytes = 0;
-  for (int b_kcont = 0; b_kcont < 2; ++b_kcont) {
-    GemmArgs p{};
-    p.m = m;
-    p.n = p.nb = n;
-    p.k = p.lda = k;
-    p.ldb = b_kcont ? k : n;
-    p.stride_a = m * k;
-    p.stride_b = n * k;
-    p.vec_a = k % 8 == 0;
-    p.vec_b = p.ldb % 8 == 0;
-    p.vec_d = 1;
-    p.part = reinterpret_cast<float*>(uintptr_t{256});
-    p.part_bytes = INT64_MAX;
-    const PackPlan pp = pack_plan(p, batch, true, b_kcont != 0);
-    if (pp.use) p = packed_args(p, batch, b_kcont != 0, pp);
-    const GemmRoute r = gemm_route(p, batch, true, b_kcont != 0);
-    const int64_t split = r.ring ? r.rp.bytes : r.dc.split.splits > 1 ? r.dc.split.bytes : 0;
-    const int64_t need = (pp.use ? pp.bytes : 0) + split;
-    bytes = bytes > need ? bytes : need;
-  }
-  return bytes;
+  return std::max(workspace_need(batch, m, n, k, true, k, k), workspace_need(batch, m, n, k, false, k, n));
+}
+
+extern "C" int64_t sph_gemm_workspace_bytes_ex(int trans_a, int trans_b, int64_t batch, int64_t m,
+                                               int64_t n, int64_t k, int64_t lda, int64_t ldb) {
+  if (batch <= 0 || m <= 0 || n <= 0 || k <= 0 || trans_a) return 0;
+  return workspace_need(batch, m, n, k, trans_b != 0, lda, ldb);
 }
 
 extern "C" int sph_gemm_ex(sph_dtype dtype, int trans_a, int trans_b, int64_t batch, int64_t m,

@@ -25,6 +25,16 @@
 namespace sph {
 namespace {
 
+template <typename T>
+__device__ inline u32x2 pack4(f32x4 v) {
+  u32x2 w;
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    w[e] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e]))) |
+           (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e + 1]))) << 16);
+  return w;
+}
+
 // Four output columns of one row: epilogue (unless done: SwiGLU) and store.
 template <typename T, bool PLAIN>
 __device__ inline void store4(const GemmArgs& p, T* D, f32x4 v, int64_t bz, int row, int col) {
@@ -35,13 +45,8 @@ __device__ inline void store4(const GemmArgs& p, T* D, f32x4 v, int64_t bz, int 
   }
   T* dp = D + row * p.ldd + col;
   if (col + 4 <= p.n) {
-    u32x2 w;
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-      w[e] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e]))) |
-             (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, Num<T>::from_f(v[2 * e + 1]))) << 16);
     typedef u32x2 u32x2_any __attribute__((aligned(2)));
-    *reinterpret_cast<u32x2_any*>(dp) = w;
+    *reinterpret_cast<u32x2_any*>(dp) = pack4<T>(v);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -268,25 +273,54 @@ __global__ void __launch_bounds__(NW_ * 64) gemm_ring_kernel(const GemmArgs p) {
     }
     return;
   }
+  // Each wave stages 16 rows of its tile in LDS (its own part of the ring:
+  // every DMA has landed, the barrier ends the other waves' reads) and stores
+  // them 16 bytes a lane, whole tile rows at a time: 8-byte stores of the
+  // accumulators as they lie write 32-byte pieces (8 x 3108 x 777 x 128: 49.4
+  // us, 37.6 through LDS).
   T* D = static_cast<T*>(p.d) + bz * p.stride_d;
-  constexpr int TO = SWIGLU ? TN / 2 : TN;
+  constexpr int TO = SWIGLU ? TN / 2 : TN, WO = TO * 16;  // output columns of the wave
+  constexpr int CPO = WO / 8, RPI = 64 / CPO;             // 16-byte chunks per row, rows per store
+  constexpr int SP = WO + 8;                               // slab pitch (elements)
+  static_assert(C::NW * 16 * SP * 2 <= ST * C::STAGE, "slabs fit the ring");
+  __syncthreads();
+  T* slab = reinterpret_cast<T*>(lds) + wave * (16 * SP);
+  const int colw = n0 + wn * WO;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int row = row0 + 16 * i;
 #pragma unroll
     for (int j = 0; j < TO; ++j) {
-      const int col = n0 + wn * (C::WTN / (SWIGLU ? 2 : 1)) + 16 * j + 4 * g4;
-      if (row < m && col < n) {
-        f32x4 v;
-        if constexpr (SWIGLU) {
+      const int col = colw + 16 * j + 4 * g4;
+      f32x4 v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = silu(acc[i][2 * j][e]) * acc[i][2 * j + 1][e];
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (SWIGLU)
+          v[e] = silu(acc[i][2 * j][e]) * acc[i][2 * j + 1][e];
+        else
+          v[e] = row < m && col + e < n ? epilogue_one<T>(p, acc[i][j][e], bz, row, col + e) : 0.f;
+      }
+      *reinterpret_cast<u32x2*>(slab + m16 * SP + 16 * j + 4 * g4) = pack4<T>(v);
+    }
+    wait_lgkmcnt0();
+#pragma unroll
+    for (int r = 0; r < 16; r += RPI) {
+      const int rr = r + lane / CPO, cc = (lane % CPO) * 8;
+      const int orow = m0 + wm * C::WTM + 16 * i + rr, ocol = colw + cc;
+      if (rr < 16 && orow < m && ocol < n) {
+        const u32x4 w = *reinterpret_cast<const u32x4*>(slab + rr * SP + cc);
+        T* dp = D + orow * p.ldd + ocol;
+        if (ocol + 8 <= n) {
+          *reinterpret_cast<u32x4_any*>(dp) = w;
         } else {
-          v = acc[i][j];
+          const T* e = reinterpret_cast<const T*>(&w);
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            if (ocol + q < n) dp[q] = e[q];
         }
-        store4<T, SWIGLU>(p, D, v, bz, row, col);
       }
     }
+    wait_lgkmcnt0();
   }
 }
 
@@ -350,8 +384,8 @@ constexpr int64_t kCUs = 256;
 
 }  // namespace
 
-// Time of a plan: ~6 us of launch, first bytes and tail, plus the K columns
-// of the fullest CU, but no less than the operands' time from HBM (~5.2
+// Time of a plan: ~2 us of launch and, per round of workgroups, ~4 us of first
+// bytes and output plus the K columns of the fullest CU, but no less than the operands' time from HBM (~5.2
 // TB/s); a K split adds the reduce launch (~2 us) and its partial sums'
 // write and read (~6 TB/s, mostly from the caches).  At least 256 K columns
 // a slice and at most 8 slices: past that the partial sums cost more than
@@ -375,7 +409,8 @@ RingPlan ring_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool b_kcont,
       const int64_t wgs = tiles * s, slots = kCUs * f.per_cu, rest = wgs % slots;
       double ns = static_cast<double>(wgs / slots) * f.ns[f.per_cu - 1];
       if (rest > 0) ns += f.ns[(rest - 1) / kCUs];
-      double us = 6.0 + static_cast<double>(slice * f.bk) * ns * 1e-3;
+      double us = 2.0 + 4.0 * static_cast<double>(ceil_div(wgs, slots)) +
+                  static_cast<double>(slice * f.bk) * ns * 1e-3;
       us = us > mem_us ? us : mem_us;
       if (s > 1) us += 2.0 + 2.0 * static_cast<double>(bytes) / 6e6;
       if (best.cfg < 0 || us < best.us) {
