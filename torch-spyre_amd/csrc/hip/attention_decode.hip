@@ -19,7 +19,7 @@
 //     workspace and a combine kernel merges the splits per row; without a
 //     workspace one workgroup per batch entry walks every chunk and writes O.
 // Rows whose keys are all masked yield NaN, as softmax over all -inf does.
-#include "sph_common.h"
+#include "gemm_common.h"
 
 #include <type_traits>
 
@@ -397,8 +397,7 @@ extern "C" int sph_attention_decode(sph_dtype dtype, int64_t batch, int64_t mq, 
 // one 64-key chunk (grid = chunks of max_len x units; P is only known on
 // the device, so chunks past P do nothing but report), stages the chunk's
 // K and V in LDS while the queries are rotated, computes the G x 64 scores
-// (one key per lane, one query head per wave, v_dot2_f32_f16 on the
-// rounded query), their softmax state (max, sum) and the unnormalised
+// (MFMA on the rounded query), their softmax state (max, sum) and the unnormalised
 // G x 128 output, and writes that partial to the workspace (a chunk past P
 // writes a neutral one); a second kernel merges each unit's partials and
 // writes O.  Measured alternatives (c5: 4 x 8 KV heads, 1152 slots,
@@ -442,7 +441,7 @@ struct StepArgs {
   int64_t k_sb, k_sh, k_ss;
   void* vc;
   int64_t v_sb, v_sh, v_ks, v_ds;
-  int v_al;  // dim-major V rows 16-byte aligned (else read element by element)
+  int wait_pos;  // read the position before the chunk (grids past one residency)
   int64_t max_len;
   int n_heads, n_kv, g, nchunks;
   float scale_log2;
@@ -477,31 +476,33 @@ __device__ inline float dot8(u32x4 a, u32x4 b, float acc) {
   return acc;
 }
 
-// One workgroup of NT threads: one unit (blockIdx.y) and one chunk of SKC
-// keys (blockIdx.x).  The chunk's K and V (SKC * 16 / NT 16-byte loads of
-// each per thread, all in flight at once) are loaded before P is known.
-// Scores: work item (query head i, 64-key block kb) on a wave, one key per
-// lane; each block keeps its own max and sum, so no barrier joins the
-// blocks before P V.  P V: item (query head i, key split r) on a slot of
-// 128 threads, one head-dim column per thread; the R splits of a head meet
-// in LDS, each block's sum scaled by 2^(m_block - m_chunk).
-template <typename T, bool VT, int SKC, int NT>
-__global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) {
-  constexpr int NB = SKC / SKB;       // score blocks per chunk
-  constexpr int NW = NT / 64;         // waves
-  constexpr int SLOTS = NT / DD;      // P V thread slots
+// One workgroup of 4 waves: one unit (blockIdx.y) and one chunk of 64 keys
+// (blockIdx.x), K and V staged in LDS (4 16-byte loads of each per thread, all
+// in flight at once).  While the grid fits the chip the chunk is loaded before
+// P is known; larger grids (batches from ~8 up) read P first, other
+// workgroups covering that wait, and skip the chunks past it.
+// Scores on the matrix cores (the queries and keys are 16-bit, the sums
+// fp32): wave w takes keys 16 w .. + 15 against the G query heads as the 16
+// columns of four 16x16x32 MFMAs, 16 LDS reads a chunk instead of 32 per head.
+// P V in fp32 FMAs (the probabilities stay fp32): thread (half, d) sums head
+// dim d over half the chunk's keys for every head, so V is read and widened
+// once, not once per head; the halves meet in LDS.
+// 24 sequences at position 700 of 1000 slots (192 units, bf16): @AB@.
+constexpr int SKC = 64, SNT = 256;
+constexpr int64_t kSpeculateWGs = 3 * 256;  // one residency: three workgroups per CU
+template <typename T, bool VT>
+__global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p) {
+  constexpr int NT = SNT;
   constexpr int LOADS = SKC * DD / 8 / NT;  // 16-byte K (and V) loads per thread
   constexpr int SVPITCH = SKC + 8;    // dim-major V rows in LDS
   constexpr int VCH = SKC / 8;        // 16-byte chunks per dim-major V row
-  static_assert(LOADS * NT * 8 == SKC * DD && NB * SKB == SKC && SLOTS >= 1, "launch shape");
-  // ps holds the probabilities, then (after the P V sums) the split sums
-  constexpr int PS = SKC > DD ? SG * SKC : SG * DD;
-  constexpr int MAXW = (SG + SLOTS - 1) / SLOTS;  // P V items per slot, at most
+  static_assert(LOADS * NT * 8 == SKC * DD && NT == 2 * DD && SKC == SKB, "launch shape");
   __shared__ __attribute__((aligned(16))) T ks[SKC][KPITCH];
   __shared__ __attribute__((aligned(16))) T vs[VT ? DD : SKC][VT ? SVPITCH : KPITCH];
-  __shared__ __attribute__((aligned(16))) T qs[SG][DD];
-  __shared__ __attribute__((aligned(16))) float ps[PS];
-  __shared__ float mblk[SG][NB], lblk[SG][NB];
+  __shared__ __attribute__((aligned(16))) T qs[SG][KPITCH];
+  // ps holds the scores, then the probabilities, then the second half's sums
+  __shared__ __attribute__((aligned(16))) float ps[SG * DD];
+  __shared__ float mblk[SG], lblk[SG];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int unit = blockIdx.y, chunk = blockIdx.x;
   const int b = unit / p.n_kv, h = unit % p.n_kv, G = p.g;
@@ -513,6 +514,14 @@ __global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) 
   // every address is inside the cache) and P itself are loaded together.
   const int64_t P = *p.pos;
   const int kmax = static_cast<int>(min<int64_t>(SKC, p.max_len - kbase));
+  float* part = p.part + (static_cast<int64_t>(unit) * p.nchunks + chunk) * G * kStepPart;
+  auto neutral = [&] {  // a chunk past P: m = -inf, the merge skips it
+    if (t < G) {
+      part[t * kStepPart] = -INFINITY;
+      part[t * kStepPart + 1] = 0.f;
+    }
+  };
+  if (p.wait_pos && P >= 0 && P < p.max_len && kbase > P) return neutral();
   u32x4 kr[LOADS], vr[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
@@ -522,11 +531,10 @@ __global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) 
     if constexpr (VT) {
       const int dm = x / VCH, kc = (x % VCH) * 8;
       const T* src = Vc + dm * p.v_ds + kbase + kc;
-      if (p.v_al && kc + 8 <= kmax) {
-        vr[i] = *reinterpret_cast<const u32x4*>(src);
+      if (kc + 8 <= kmax) {
+        vr[i] = *reinterpret_cast<const u32x4_any*>(src);  // (rows at any alignment)
       } else {
-        // the cache's last, partial chunk, or rows that are not 16-byte
-        // aligned: element loads, zeros past the cache
+        // the cache's last, partial chunk: element loads, zeros past the cache
         const uint16_t* s16 = reinterpret_cast<const uint16_t*>(src);
         uint32_t e[8];
 #pragma unroll
@@ -562,16 +570,7 @@ __global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) 
     if (t == 0 && chunk == 0 && unit == 0 && p.err != nullptr) *p.err = kStepBadPos;
     return;
   }
-  const bool active = kbase <= P;
-  float* part = p.part + (static_cast<int64_t>(unit) * p.nchunks + chunk) * G * kStepPart;
-  if (!active) {
-    // a chunk past P: a neutral partial (m = -inf; the merge skips it)
-    if (t < G) {
-      part[t * kStepPart] = -INFINITY;
-      part[t * kStepPart + 1] = 0.f;
-    }
-    return;
-  }
+  if (kbase > P) return neutral();
   const int nkeys = static_cast<int>(min<int64_t>(SKC, P + 1 - kbase));
   const T* cs = static_cast<const T*>(p.cos) + P * p.ld_rope;
   const T* sn = static_cast<const T*>(p.sin) + P * p.ld_rope;
@@ -621,17 +620,30 @@ __global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) 
     else Vc[P * p.v_ks + t] = vr_;
   }
   __syncthreads();
-  // scores: item (head i, block kb), key kb * 64 + lane; each block's
-  // probabilities relative to its own max (a block with no visible key has
-  // max -inf and contributes nothing)
-  for (int it = wave; it < G * NB; it += NW) {
-    const int i = it / NB, kb = it % NB, key = kb * SKB + lane;
-    float s = 0.f;
+  // scores: MFMA rows are the wave's 16 keys, columns the query heads (those
+  // past G repeat other rows of qs and are dropped)
+  {
+    const int m16 = lane & 15, g4 = lane >> 4;
+    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int cc = 0; cc < DD; cc += 8)
-      s = dot8<T>(*reinterpret_cast<const u32x4*>(&qs[i][cc]),
-                  *reinterpret_cast<const u32x4*>(&ks[key][cc]), s);
-    s = key < nkeys ? s * p.scale_log2 : -INFINITY;
+    for (int kk = 0; kk < DD / 32; ++kk) {
+      const u32x4 kf = *reinterpret_cast<const u32x4*>(&ks[16 * wave + m16][32 * kk + 8 * g4]);
+      const u32x4 qf = *reinterpret_cast<const u32x4*>(&qs[m16 % SG][32 * kk + 8 * g4]);
+      sc = mfma16<T>(kf, qf, sc);
+    }
+    if (m16 < G) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = 16 * wave + 4 * g4 + r;
+        ps[m16 * SKC + key] = key < nkeys ? sc[r] * p.scale_log2 : -INFINITY;
+      }
+    }
+  }
+  __syncthreads();
+  // each head's softmax state over the chunk, one key per lane (key kbase <= P
+  // is visible, so the max is finite unless a score is not)
+  for (int i = wave; i < G; i += NT / 64) {
+    const float s = ps[i * SKC + lane];
     float mx = s;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
@@ -639,80 +651,56 @@ __global__ void __launch_bounds__(NT) attn_decode_step_kernel(const StepArgs p) 
     float sum = pj;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    ps[i * SKC + key] = pj;
+    ps[i * SKC + lane] = pj;
     if (lane == 0) {
-      mblk[i][kb] = mx;
-      lblk[i][kb] = sum;
+      mblk[i] = mx;
+      lblk[i] = sum;
     }
   }
   __syncthreads();
-  // unnormalised P V: R key splits per head, the largest power of two
-  // dividing NB with G * R <= SLOTS (at least 1: a slot then takes several
-  // heads)
-  int R = 1;
-  while (2 * R <= NB && G * 2 * R <= SLOTS) R *= 2;
-  const int slot = t >> 7, d = t & (DD - 1);
-  const int bps = NB / R;  // blocks per split
-  float acc_w[MAXW];
+  // unnormalised P V of this thread's half of the keys and column
+  const int half = t >> 7, d = t & (DD - 1);
+  float acc[SG];
 #pragma unroll
-  for (int n = 0; n < MAXW; ++n) {
-    const int w = slot + n * SLOTS;
-    acc_w[n] = 0.f;
-    if (w >= G * R) continue;
-    const int i = w / R, split = w % R;
-    float mi = -INFINITY;
+  for (int i = 0; i < SG; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int kb = 0; kb < NB; ++kb) mi = fmaxf(mi, mblk[i][kb]);
-    float acc = 0.f;
-    for (int kb = split * bps; kb < (split + 1) * bps; ++kb) {
-      const float m = mblk[i][kb];
-      if (m == -INFINITY) continue;
-      float a = 0.f;
+  for (int j = 0; j < SKC / 2; j += 8) {
+    const int key = half * (SKC / 2) + j;
+    float vf[8];
+    if constexpr (VT) {
+      const u32x4 vw = *reinterpret_cast<const u32x4*>(&vs[d][key]);
+      const T* ve = reinterpret_cast<const T*>(&vw);
 #pragma unroll
-      for (int j = kb * SKB; j < (kb + 1) * SKB; j += 8) {
-        float vf[8];
-        if constexpr (VT) {
-          const u32x4 vw = *reinterpret_cast<const u32x4*>(&vs[d][j]);
-          const T* ve = reinterpret_cast<const T*>(&vw);
+      for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(ve[e]);
+    } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(ve[e]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(vs[j + e][d]);
-        }
-        const float4 p0 = *reinterpret_cast<const float4*>(&ps[i * SKC + j]);
-        const float4 p1 = *reinterpret_cast<const float4*>(&ps[i * SKC + j + 4]);
-        const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) a = fmaf(pv[e], vf[e], a);
-      }
-      acc = fmaf(a, __builtin_amdgcn_exp2f(m - mi), acc);
+      for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(vs[key + e][d]);
     }
-    acc_w[n] = acc;
-  }
-  __syncthreads();  // every P V read of ps is done: it now takes the split sums
 #pragma unroll
-  for (int n = 0; n < MAXW; ++n) {
-    const int w = slot + n * SLOTS;
-    if (w < G * R) ps[w * DD + d] = acc_w[n];
+    for (int i = 0; i < SG; ++i) {
+      if (i >= G) break;
+      const f32x4 p0 = *reinterpret_cast<const f32x4*>(&ps[i * SKC + key]);
+      const f32x4 p1 = *reinterpret_cast<const f32x4*>(&ps[i * SKC + key + 4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i] = fmaf(p0[e], vf[e], acc[i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i] = fmaf(p1[e], vf[e + 4], acc[i]);
+    }
+  }
+  __syncthreads();  // every read of the probabilities is done
+  if (half == 1) {
+#pragma unroll
+    for (int i = 0; i < SG; ++i)
+      if (i < G) ps[i * DD + d] = acc[i];
   }
   __syncthreads();
-  for (int i = slot; i < G; i += SLOTS) {
-    float acc = 0.f;
-    for (int r = 0; r < R; ++r) acc += ps[(i * R + r) * DD + d];
-    part[i * kStepPart + 2 + d] = acc;
-    if (d == 0) {
-      float mi = -INFINITY;
+  if (half == 0) {
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb) mi = fmaxf(mi, mblk[i][kb]);
-      float l = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < NB; ++kb) {
-        const float m = mblk[i][kb];
-        l += m == -INFINITY ? 0.f : lblk[i][kb] * __builtin_amdgcn_exp2f(m - mi);
-      }
-      part[i * kStepPart] = mi;
-      part[i * kStepPart + 1] = l;
+    for (int i = 0; i < SG; ++i)
+      if (i < G) part[i * kStepPart + 2 + d] = acc[i] + ps[i * DD + d];
+    if (t < G) {
+      part[t * kStepPart] = mblk[t];
+      part[t * kStepPart + 1] = lblk[t];
     }
   }
 }
@@ -840,7 +828,6 @@ extern "C" int sph_decode_attention_step(
   p.v_sh = v_stride_h;
   p.v_ks = v_key_stride;
   p.v_ds = v_dim_stride;
-  p.v_al = v_al ? 1 : 0;
   p.max_len = max_len;
   p.n_heads = static_cast<int>(n_heads);
   p.n_kv = static_cast<int>(n_kv_heads);
@@ -852,8 +839,8 @@ extern "C" int sph_decode_attention_step(
   // 10.1 / 8.6 / 11.3 / 9.5 us for 128 x 256 / 128 x 512 / 256 x 512 /
   // 256 x 1024 (larger chunks leave fewer workgroups per CU to overlap one's
   // loads with another's arithmetic).
-  constexpr int kChunk = 64, kThreads = 256;
-  p.nchunks = static_cast<int>((max_len + kChunk - 1) / kChunk);
+  p.nchunks = static_cast<int>((max_len + SKC - 1) / SKC);
+  p.wait_pos = p.nchunks * batch * n_kv_heads > kSpeculateWGs;
   p.scale_log2 = scale * kLog2eD;
   p.out = out;
   p.ld_out = ld_out;
@@ -864,7 +851,7 @@ extern "C" int sph_decode_attention_step(
   auto go = [&](auto tag, auto vt_tag) {
     using T = decltype(tag);
     constexpr bool VT = decltype(vt_tag)::value;
-    attn_decode_step_kernel<T, VT, kChunk, kThreads><<<grid, kThreads, 0, st>>>(p);
+    attn_decode_step_kernel<T, VT><<<grid, SNT, 0, st>>>(p);
     attn_decode_step_merge<T><<<mgrid, kMergeThreads, 0, st>>>(p);
   };
   if (dtype == SPH_F16) {
