@@ -476,36 +476,50 @@ __device__ inline float dot8(u32x4 a, u32x4 b, float acc) {
   return acc;
 }
 
-// One workgroup of 4 waves: one unit (blockIdx.y) and one chunk of 64 keys
-// (blockIdx.x), K and V staged in LDS (4 16-byte loads of each per thread, all
-// in flight at once).  While the grid fits the chip the chunk is loaded before
-// P is known; larger grids (batches from ~8 up) read P first, other
-// workgroups covering that wait, and skip the chunks past it.
+// One workgroup of 4 waves: one unit and one chunk of 64 keys.  While the grid
+// fits the chip the chunk is loaded before P is known; larger grids (batches
+// from ~8 up) read P first, other workgroups covering that wait, and skip the
+// chunks past it.  The chunks of a unit run on one XCD: with a dim-major V
+// whose rows are off 128 bytes, neighbouring chunks share V's cache lines.
 // Scores on the matrix cores (the queries and keys are 16-bit, the sums
 // fp32): wave w takes keys 16 w .. + 15 against the G query heads as the 16
-// columns of four 16x16x32 MFMAs, 16 LDS reads a chunk instead of 32 per head.
-// P V in fp32 FMAs (the probabilities stay fp32): thread (half, d) sums head
-// dim d over half the chunk's keys for every head, so V is read and widened
-// once, not once per head; the halves meet in LDS.
-// 24 sequences at position 700 of 1000 slots (192 units, bf16): @AB@.
+// columns of four 16x16x32 MFMAs, the key fragments loaded straight from the
+// cache (a lane's 16 bytes of one key row).  P V in fp32 FMAs (the
+// probabilities stay fp32) from the registers that V was loaded into: a
+// thread holds 8 keys of 4 head dims (dim-major V), sums them for every head
+// and 8 neighbouring lanes meet by DPP; only a key-major V is staged in LDS.
+// Without K and V in LDS five workgroups share a CU instead of three, which is
+// what hides the chain of loads, scores and softmax.
+// 24 sequences at position 700 of 1000 slots (192 units, bf16): 37.1 us with
+// dot products over staged chunks, 32.7 with MFMA scores over staged chunks,
+// 23.5 like this.
+template <int CTRL>
+__device__ inline float dpp_step(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
 constexpr int SKC = 64, SNT = 256;
-constexpr int64_t kSpeculateWGs = 3 * 256;  // one residency: three workgroups per CU
+constexpr int64_t kSpeculateWGs = 3 * 256;  // about half of what the chip holds at once
 template <typename T, bool VT>
 __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p) {
   constexpr int NT = SNT;
   constexpr int LOADS = SKC * DD / 8 / NT;  // 16-byte K (and V) loads per thread
-  constexpr int SVPITCH = SKC + 8;    // dim-major V rows in LDS
   constexpr int VCH = SKC / 8;        // 16-byte chunks per dim-major V row
   static_assert(LOADS * NT * 8 == SKC * DD && NT == 2 * DD && SKC == SKB, "launch shape");
-  __shared__ __attribute__((aligned(16))) T ks[SKC][KPITCH];
-  __shared__ __attribute__((aligned(16))) T vs[VT ? DD : SKC][VT ? SVPITCH : KPITCH];
+  __shared__ __attribute__((aligned(16))) T vs[VT ? 1 : SKC][KPITCH];
   __shared__ __attribute__((aligned(16))) T qs[SG][KPITCH];
-  // ps holds the scores, then the probabilities, then the second half's sums
+  __shared__ __attribute__((aligned(16))) T kn[DD];  // the new key, rotated
+  // ps holds the scores, then the probabilities, then (key-major V) the second half's sums
   __shared__ __attribute__((aligned(16))) float ps[SG * DD];
   __shared__ float mblk[SG], lblk[SG];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int unit = blockIdx.y, chunk = blockIdx.x;
+  int id = blockIdx.x;  // dispatch is round-robin over 8 XCDs: contiguous runs to each
+  {
+    const int total = gridDim.x, q = total >> 3, r = total & 7, x = id & 7;
+    id = x * q + min(x, r) + (id >> 3);
+  }
+  const int unit = id / p.nchunks, chunk = id % p.nchunks;
   const int b = unit / p.n_kv, h = unit % p.n_kv, G = p.g;
+  const int m16 = lane & 15, g4 = lane >> 4;
   const int64_t kbase = static_cast<int64_t>(chunk) * SKC;
   T* Kc = static_cast<T*>(p.kc) + b * p.k_sb + h * p.k_sh;
   T* Vc = static_cast<T*>(p.vc) + b * p.v_sb + h * p.v_sh;
@@ -525,9 +539,11 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
   u32x4 kr[LOADS], vr[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
+    // K fragment i: key row 16 wave + lane % 16, dims 32 i + 8 (lane / 16) ..
+    const int krow = 16 * wave + m16;
+    kr[i] = krow < kmax ? *reinterpret_cast<const u32x4*>(Kc + (kbase + krow) * p.k_ss + 32 * i + 8 * g4)
+                        : zero_chunk();
     const int x = t + NT * i, key = x >> 4, cc = (x & 15) * 8;
-    kr[i] = key < kmax ? *reinterpret_cast<const u32x4*>(Kc + (kbase + key) * p.k_ss + cc)
-                       : zero_chunk();
     if constexpr (VT) {
       const int dm = x / VCH, kc = (x % VCH) * 8;
       const T* src = Vc + dm * p.v_ds + kbase + kc;
@@ -590,9 +606,8 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     const int x = t + NT * i, key = x >> 4, cc = (x & 15) * 8;
-    *reinterpret_cast<u32x4*>(&ks[key][cc]) = kr[i];
     if constexpr (VT) {
-      const int dm = x / VCH, kc = (x % VCH) * 8;
+      const int kc = (x % VCH) * 8;
       u32x4 w = vr[i];
       if (kc + 8 > nkeys) {
 #pragma unroll
@@ -602,32 +617,46 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
           w[q] &= keep;
         }
       }
-      *reinterpret_cast<u32x4*>(&vs[dm][kc]) = w;
+      vr[i] = w;
     } else {
       *reinterpret_cast<u32x4*>(&vs[key][cc]) = key < nkeys ? vr[i] : zero_chunk();
     }
   }
   const int own = static_cast<int>(P - kbase);  // the new key's slot, if here
-  __syncthreads();  // chunk staged: the new key / value replace slot `own`
-  if (own < SKC && t < DD) {
+  const bool here = own < SKC;  // the new key and value replace slot `own`
+  if (here && t < DD) {
     const T kr_ = Num<T>::from_f(ka * cd + sgn * kb_ * sd);
-    const T vr_ = vv;
-    ks[own][t] = kr_;
-    if constexpr (VT) vs[t][own] = vr_;
-    else vs[own][t] = vr_;
+    kn[t] = kr_;
     Kc[P * p.k_ss + t] = kr_;
-    if constexpr (VT) Vc[t * p.v_ds + P] = vr_;
-    else Vc[P * p.v_ks + t] = vr_;
+    if constexpr (VT) Vc[t * p.v_ds + P] = vv;
+    else Vc[P * p.v_ks + t] = vv;
+  }
+  if constexpr (VT) {
+    if (here && (t % VCH) == own / 8) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const uint32_t nv = __builtin_bit_cast(uint16_t, vnew[(t + NT * i) / VCH]);
+        const int q = own % 8;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (q == 2 * e) vr[i][e] = (vr[i][e] & 0xffff0000u) | nv;
+          if (q == 2 * e + 1) vr[i][e] = (vr[i][e] & 0xffffu) | (nv << 16);
+        }
+      }
+    }
   }
   __syncthreads();
+  if constexpr (!VT) {
+    if (here && t < DD) vs[own][t] = vv;  // (read after the barriers below)
+  }
   // scores: MFMA rows are the wave's 16 keys, columns the query heads (those
   // past G repeat other rows of qs and are dropped)
   {
-    const int m16 = lane & 15, g4 = lane >> 4;
+    const bool mine = here && own == 16 * wave + m16;
     f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kk = 0; kk < DD / 32; ++kk) {
-      const u32x4 kf = *reinterpret_cast<const u32x4*>(&ks[16 * wave + m16][32 * kk + 8 * g4]);
+    for (int kk = 0; kk < LOADS; ++kk) {
+      const u32x4 kf = mine ? *reinterpret_cast<const u32x4*>(&kn[32 * kk + 8 * g4]) : kr[kk];
       const u32x4 qf = *reinterpret_cast<const u32x4*>(&qs[m16 % SG][32 * kk + 8 * g4]);
       sc = mfma16<T>(kf, qf, sc);
     }
@@ -658,7 +687,42 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
     }
   }
   __syncthreads();
-  // unnormalised P V of this thread's half of the keys and column
+  if (t < G) {
+    part[t * kStepPart] = mblk[t];
+    part[t * kStepPart + 1] = lblk[t];
+  }
+  if constexpr (VT) {
+    // unnormalised P V of this thread's 8 keys for its dims (t + 256 i) / 8;
+    // lane i of each 8 writes head i
+    const int kc = (t % VCH) * 8;
+    float vf[LOADS][8];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const T* ve = reinterpret_cast<const T*>(&vr[i]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vf[i][e] = Num<T>::to_f(ve[e]);
+    }
+#pragma unroll
+    for (int hd = 0; hd < SG; ++hd) {
+      if (hd >= G) break;
+      const f32x4 p0 = *reinterpret_cast<const f32x4*>(&ps[hd * SKC + kc]);
+      const f32x4 p1 = *reinterpret_cast<const f32x4*>(&ps[hd * SKC + kc + 4]);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        float a = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a = fmaf(p0[e], vf[i][e], a);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a = fmaf(p1[e], vf[i][e + 4], a);
+        a += dpp_step<0xB1>(a);   // lanes 1 apart,
+        a += dpp_step<0x4E>(a);   // 2 apart,
+        a += dpp_step<0x141>(a);  // and the mirrored half row: all 8
+        if ((t % VCH) == hd) part[hd * kStepPart + 2 + (t + NT * i) / VCH] = a;
+      }
+    }
+    return;
+  }
+  // key-major V: this thread's half of the keys and column
   const int half = t >> 7, d = t & (DD - 1);
   float acc[SG];
 #pragma unroll
@@ -667,15 +731,8 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
   for (int j = 0; j < SKC / 2; j += 8) {
     const int key = half * (SKC / 2) + j;
     float vf[8];
-    if constexpr (VT) {
-      const u32x4 vw = *reinterpret_cast<const u32x4*>(&vs[d][key]);
-      const T* ve = reinterpret_cast<const T*>(&vw);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(ve[e]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(vs[key + e][d]);
-    }
+    for (int e = 0; e < 8; ++e) vf[e] = Num<T>::to_f(vs[key + e][d]);
 #pragma unroll
     for (int i = 0; i < SG; ++i) {
       if (i >= G) break;
@@ -698,10 +755,6 @@ __global__ void __launch_bounds__(SNT) attn_decode_step_kernel(const StepArgs p)
 #pragma unroll
     for (int i = 0; i < SG; ++i)
       if (i < G) part[i * kStepPart + 2 + d] = acc[i] + ps[i * DD + d];
-    if (t < G) {
-      part[t * kStepPart] = mblk[t];
-      part[t * kStepPart + 1] = lblk[t];
-    }
   }
 }
 
@@ -846,7 +899,7 @@ extern "C" int sph_decode_attention_step(
   p.ld_out = ld_out;
   p.part = static_cast<float*>(workspace);
   hipStream_t st = as_stream(stream);
-  dim3 grid(static_cast<unsigned>(p.nchunks), static_cast<unsigned>(batch * n_kv_heads));
+  dim3 grid(static_cast<unsigned>(p.nchunks * batch * n_kv_heads));
   const dim3 mgrid(static_cast<unsigned>(batch * n_kv_heads * p.g));
   auto go = [&](auto tag, auto vt_tag) {
     using T = decltype(tag);
