@@ -275,3 +275,27 @@ def test_c3_gelu_chain_bf16_matches_cpu():
         # plus half a bf16 step of each addend
         bound = want.sum(-1).abs() * 2 ** -7 + want.abs().sum(-1) * 2 ** -9 + 1e-2
         assert ((r.cpu().float() - want.sum(-1)).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("cols", [511, 513, 1032, 4095, 5128, 9001])
+def test_row_kernels_of_any_length(cols):
+    # rows off a thread's groups of 8 elements, and off the workgroup's span:
+    # each reduction kind, multi-phase rows and stored intermediates
+    _log(f"compiled row kernels, {cols} columns")
+    R = 37
+    x, r = randn((R, cols), k=0), randn((R, cols), k=1)
+    w, b = randn((cols,), k=2, scale=0.1, mean=1.0), randn((cols,), k=3, scale=0.1)
+    xd, rd, wd, bd = x.to(DEV), r.to(DEV), w.to(DEV), b.to(DEV)
+
+    def ln(a, c, g, e):
+        h = a + c
+        return h, F.layer_norm(h, [cols], g, e, 1e-5)
+
+    h, y = torch.compile(ln, dynamic=False)(xd, rd, wd, bd)
+    hc = x + r
+    assert torch.equal(h.cpu(), hc)
+    assert_close_fp(y, O.layernorm(hc.numpy(), w.numpy(), b.numpy(), 1e-5)[0], what="layer norm")
+    p = torch.compile(lambda a: torch.softmax(a, -1), dynamic=False)(xd)
+    assert_close_fp(p, O.softmax(x.numpy()), what="softmax")
+    m, i = torch.compile(lambda a: (a.amax(-1), a.argmax(-1)), dynamic=False)(xd)
+    assert torch.equal(m.cpu(), x.amax(-1)) and torch.equal(i.cpu(), x.argmax(-1))

@@ -590,26 +590,53 @@ class SpyreKernel(SIMDKernel):
     def _open_rloop(self) -> None:
         if self._rloop_open:
             return
+        self._rinner = IndentedBuffer()
+        self._rloop_open = True
+
+    def _close_rloop(self) -> None:
+        """Writes the open row loop around the collected body.  A thread's
+        groups of VEC elements that lie inside the row run without bounds
+        tests, so that their accesses merge into wide ones; with a row length
+        off VEC the group at the row's end is a copy of the body with a test
+        per element."""
         r, b, v = self._rnumel(), self._block(), self._rvec()
         loops = self._trips()
+        body, inner = self.body, self._rinner
         if loops <= MAX_CACHED_TRIPS:
-            self.body.writeline("#pragma unroll")
-        self.body.writeline(f"for (int64_t r0_cnt = 0; r0_cnt < {loops}LL; ++r0_cnt) {{")
-        self.body.writeline("#pragma unroll")
-        self.body.writeline(f"for (int spy_v = 0; spy_v < {v}; ++spy_v) {{")
-        with self.body.indent():
-            self.body.writeline(
-                f"const int64_t r0_index = (r0_cnt * {b}LL + threadIdx.x) * {v}LL + spy_v;")
-            if loops * b * v != r:
-                self.body.writeline(f"if (r0_index >= {r}LL) break;")
-        self._rloop_open = True
+            body.writeline("#pragma unroll")
+        body.writeline(f"for (int64_t r0_cnt = 0; r0_cnt < {loops}LL; ++r0_cnt) {{")
+        body.writeline(f"const int64_t spy_r = (r0_cnt * {b}LL + threadIdx.x) * {v}LL;")
+
+        def group(guard):
+            body.writeline("#pragma unroll")
+            body.writeline(f"for (int spy_v = 0; spy_v < {v}; ++spy_v) {{")
+            with body.indent():
+                body.writeline("const int64_t r0_index = spy_r + spy_v;")
+                if guard:
+                    body.writeline(f"if (r0_index >= {r}LL) break;")
+                body.splice(inner)
+                body.splice(self.loads)
+                body.splice(self.compute)
+            body.writeline("}")
+
+        if loops * b * v != r and r % v == 0:
+            body.writeline(f"if (spy_r >= {r}LL) break;")
+        if r % v == 0:
+            group(False)
+        else:
+            body.writeline(f"if (spy_r + {v} <= {r}LL) {{")
+            group(False)
+            body.writeline("} else {")
+            group(True)
+            body.writeline("}")
+        body.writeline("}")
+        self._rloop_open = False
 
     def codegen_iteration_ranges_entry(self, entry: IterationRangesEntry) -> None:
         expr = self.kexpr(self.rename_indexing(entry.expr))
         if entry.is_reduction:
             self._open_rloop()
-            with self.body.indent():
-                self.body.writeline(f"const int64_t {entry.name} = {expr};")
+            self._rinner.writeline(f"const int64_t {entry.name} = {expr};")
         else:
             self.indexing_code.writeline(f"const int64_t {entry.name} = {expr};")
             try:
@@ -947,11 +974,7 @@ class SpyreKernel(SIMDKernel):
         if self._pending_accum and not self._rloop_open and self.inside_reduction:
             self._open_rloop()
         if self._rloop_open:
-            with self.body.indent():
-                self.body.splice(self.loads)
-                self.body.splice(self.compute)
-            self.body.writeline("}}")
-            self._rloop_open = False
+            self._close_rloop()
             # values computed inside the loop die with it; reduction results
             # (made after the loop) stay available to later phases
             keep = set()
