@@ -72,3 +72,23 @@ def test_gemm_workspace_bytes(batch, m, n, k, split):
     assert (got > 0) == split, got
     if split:
         assert got % (256 * 256 * 4) == 0 and got <= 256 * 256 * 256 * 4
+
+
+def test_gemm_workspace_bytes_covers_each_layout():
+    # the per-call size never exceeds the size for both layouts of contiguous
+    # operands, is 0 for a transposed A, and stays within the padded copies and
+    # eight slices of partial sums (+ one 256 x 256 tile per CU of a split tail)
+    lib = _capi.lib()
+    for batch in (1, 3):
+        for m in (1, 8, 9, 33, 255, 300, 2100):
+            for n in (64, 65, 504, 4097):
+                for k in (8, 63, 520, 1029, 4096):
+                    both = lib.sph_gemm_workspace_bytes(batch, m, n, k)
+                    one = [lib.sph_gemm_workspace_bytes_ex(0, tb, batch, m, n, k, k, k if tb else n)
+                           for tb in (0, 1)]
+                    assert max(one) == both and min(one) >= 0
+                    assert lib.sph_gemm_workspace_bytes_ex(1, 0, batch, m, n, k, m, n) == 0
+                    pad = 2 * batch * (m + n + 8) * (k + 64) + 512
+                    assert both <= pad + max(8 * m * (n + 3) * 4, 256 * 256 * 256 * 4)
+                    if batch > 1 and n % 8 == 0 and k % 8 == 0:
+                        assert both == 0
