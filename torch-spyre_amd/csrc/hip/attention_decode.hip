@@ -395,10 +395,10 @@ extern "C" int sph_attention_decode(sph_dtype dtype, int64_t batch, int64_t mq, 
 // key-major or dim-major ([.., 128, max_len], key stride 1, the layout the
 // decoders' caches keep).  Each workgroup (256 threads) takes one unit and
 // one 64-key chunk (grid = chunks of max_len x units; P is only known on
-// the device, so chunks past P do nothing but report), stages the chunk's
-// K and V in LDS while the queries are rotated, computes the G x 64 scores
-// (MFMA on the rounded query), their softmax state (max, sum) and the unnormalised
-// G x 128 output, and writes that partial to the workspace (a chunk past P
+// the device, so chunks past P do nothing but report), loads the chunk's K
+// and V into registers (a key-major V into LDS) while the queries are rotated,
+// computes the G x 64 scores (MFMA on the rounded query), their softmax state
+// (max, sum) and the unnormalised G x 128 output, and writes that partial to the workspace (a chunk past P
 // writes a neutral one); a second kernel merges each unit's partials and
 // writes O.  Measured alternatives (c5: 4 x 8 KV heads, 1152 slots,
 // 18.9 MB of K / V): larger chunks on more threads (128 to 256 keys on 256
@@ -453,27 +453,6 @@ struct StepArgs {
 __device__ inline u32x4 zero_chunk() {
   u32x4 z = {0u, 0u, 0u, 0u};
   return z;
-}
-
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-// acc + the dot product of 8 two-byte values a and b (16 bytes each):
-// fp16 as four v_dot2_f32_f16 (exact products, fp32 sums), bf16 widened by
-// shifts into fp32 FMAs.
-template <typename T>
-__device__ inline float dot8(u32x4 a, u32x4 b, float acc) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t ai = a[i], bi = b[i];
-    if constexpr (__is_same(T, half_t)) {
-      acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, ai), __builtin_bit_cast(f16x2, bi),
-                                   acc, false);
-    } else {
-      acc = fmaf(__uint_as_float(ai << 16), __uint_as_float(bi << 16), acc);
-      acc = fmaf(__uint_as_float(ai & 0xffff0000u), __uint_as_float(bi & 0xffff0000u), acc);
-    }
-  }
-  return acc;
 }
 
 // One workgroup of 4 waves: one unit and one chunk of 64 keys.  While the grid
@@ -885,13 +864,13 @@ extern "C" int sph_decode_attention_step(
   p.n_heads = static_cast<int>(n_heads);
   p.n_kv = static_cast<int>(n_kv_heads);
   p.g = static_cast<int>(n_heads / n_kv_heads);
-  // Launch shape: 64-key chunks on 256 threads (44 KB of LDS, three
-  // workgroups per CU).  Measured on the c5 decode step (4 x 8 KV heads,
-  // 1152 slots, position 1087): 7.4 us against 8.0 us for 128 keys x 512
-  // threads; before the score dot products became v_dot2, 8.0 us against
-  // 10.1 / 8.6 / 11.3 / 9.5 us for 128 x 256 / 128 x 512 / 256 x 512 /
-  // 256 x 1024 (larger chunks leave fewer workgroups per CU to overlap one's
-  // loads with another's arithmetic).
+  // Launch shape: 64-key chunks on 256 threads.  Chosen when K and V were both
+  // staged in LDS and not swept again since (4 x 8 KV heads, 1152 slots,
+  // position 1087): 7.4 us against 8.0 us for 128 keys x 512 threads, with
+  // dot-product scores; with scalar FMAs 8.0 us against 10.1 / 8.6 / 11.3 /
+  // 9.5 us for 128 x 256 / 128 x 512 / 256 x 512 / 256 x 1024 (larger chunks
+  // left fewer workgroups per CU to overlap one's loads with another's
+  // arithmetic).
   p.nchunks = static_cast<int>((max_len + SKC - 1) / SKC);
   p.wait_pos = p.nchunks * batch * n_kv_heads > kSpeculateWGs;
   p.scale_log2 = scale * kLog2eD;

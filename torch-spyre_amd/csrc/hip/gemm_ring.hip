@@ -368,8 +368,14 @@ void launch(GemmArgs& p, int64_t batch, hipStream_t st) {
 //   128 x 128 on 4 waves   333 x 6144 x 4096 in 3 slices 36.6, 333 x 4096 x 12800 in 5 59.5
 //   192 x 128  2331 x 4096 x 4096 102.6, 333 x 2*12800 x 4096 (SwiGLU) 111.7
 // (the kernels these products ran on before: 24 rows 60-140 us, 333 x 6144 x
-// 4096 64 us).  Not kept: 3- to 6-stage rings of 32-deep K tiles (5-15 %
-// slower at 128 x 128), 256-row tiles, 128 x 256 tiles, 96-row tiles.
+// 4096 64 us).  Not kept, from the same sweep of 16 products (us
+// beside the best tile above): 128 x 128 with 3 to 5 stages of 32-deep K tiles
+// (41.7 beside 36.6 at 333 x 6144 x 4096, 170.4 beside 144.9 at 2331 x 6144 x
+// 4096; within 4 % at 128 x 6144); 128 x 256 tiles (107.8 beside 102.6 at
+// 2331 x 4096 x 4096, nowhere the fastest); 96-row tiles (nowhere among the
+// first seven).  256-row tiles were 2-3 % faster on two (142.3 beside 144.9 at
+// 2331 x 6144, which gemm.hip's 256-row tiles take, and 28.7 beside 29.6 at
+// 200 x 6144) and slower on the others: not worth an instance.
 struct RingCfg {
   int bm, bn, bk, per_cu;
   double ns[3];
