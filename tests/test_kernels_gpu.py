@@ -683,6 +683,9 @@ def test_gemm_swiglu(m, n, k, pad, dtype):
     (1, 200, 4100, 4096, 1, 8, 0, torch.float16),    # N % 128 != 0 through the reduce
     (1, 193, 512, 96, 1, 0, 0, torch.bfloat16),      # 32-deep K tiles
     (3, 300, 136, 776, 0, 0, 0, torch.float16),      # batched, ragged M, N and K
+    (32, 300, 392, 384, 0, 0, 0, torch.float16),     # batched short K, uneven round: last K register-staged
+    (32, 300, 392, 392, 0, 0, 0, torch.bfloat16),    # the same past it, on the ring kernel
+    (8, 512, 1280, 64, 0, 8, 3, torch.float16),      # whole 256-row tiles of such a round
     (1, 2100, 4104, 576, 1, 0, 3, torch.float16),    # ragged rows and columns of 256-row tiles
     (1, 2100, 4104, 576, 0, 8, 0, torch.bfloat16),   # the same, row-major B
     (1, 1100, 3000, 4096, 1, 0, 2, torch.float16)])  # ragged, K-split tail of 256-row tiles

@@ -1174,6 +1174,19 @@ inline void launch_pack(const GemmArgs& p, const GemmArgs& q, int64_t batch, boo
   gemm_pack_kernel<<<grid, 256, 0, st>>>(oa, ob);
 }
 
+// Row-major B, short K and a ring plan of 128 x 128 tiles that gives a part of
+// the CUs a second workgroup: the plan costs ~10 us + 20 ns per K column there
+// (the time model has 6 + 16.5), the register-staged kernel's 128 x 128 tiles 8
+// + 26, so they lead up to K ~ 400 (32 x 300 x 400 fp16, register-staged beside
+// ring: K 256 14.7 / 15.6 us, 320 16.5 / 17.1, 384 18.2 / 18.5, 512 21.3 /
+// 20.8; 10 x 1571 x 328 x 128 11.2 / 13.1).  Not where that kernel would take
+// 256 x 256 tiles.
+constexpr int64_t kStagedShortK = 384;
+inline bool staged_leads(const GemmArgs& p, int64_t batch, bool b_kcont, const GemmRoute& r) {
+  return r.ring && r.rp.uneven && !b_kcont && p.k <= kStagedShortK &&
+         ceil_div(p.m, 256) * ceil_div(p.n, 256) * batch < kNumCUs;
+}
+
 // Small row counts on the streaming kernels, short K on theirs, then the
 // direct-load and ring kernels; what neither takes (A transposed, K or rows
 // off 16-byte chunks) on the register-staged kernel: 256x256 tiles when they
@@ -1181,7 +1194,7 @@ inline void launch_pack(const GemmArgs& p, const GemmArgs& q, int64_t batch, boo
 // CUs), else 64x64 for small problems.
 template <typename T>
 int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont,
-                  hipStream_t st) {
+                  hipStream_t st, bool packed = false) {
   if (stream_fits(p, batch, a_kcont, b_kcont))
     return launch_stream(__is_same(T, bf16_t), p, false, false, st);
   if (p.m <= kSmallRows && a_kcont && b_kcont && p.vec_a && p.vec_b && p.k > 0 && p.k % 8 == 0 &&
@@ -1219,9 +1232,13 @@ int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont,
   if (pp.use) {
     GemmArgs q = packed_args(p, batch, b_kcont, pp);
     launch_pack(p, q, batch, b_kcont, pp, st);
-    return gemm_dispatch<T>(q, batch, true, b_kcont, st);  // (aligned: packs nothing)
+    return gemm_dispatch<T>(q, batch, true, b_kcont, st, true);  // (aligned: packs nothing)
   }
-  const GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
+  GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
+  if (!packed && staged_leads(p, batch, b_kcont, r)) {
+    r.ring = false;
+    if (p.m % dl::BM != 0 || p.n % 128 != 0) r.dc.kind = 0;  // whole tiles stay direct-load
+  }
   if (r.ring) return launch_ring(__is_same(T, bf16_t), p, batch, b_kcont, false, r.rp, st);
   switch (r.dc.kind) {
     case 256: return launch_dl<T, 256>(p, batch, b_kcont, st, &r.dc.split);

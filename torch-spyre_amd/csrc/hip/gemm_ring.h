@@ -11,6 +11,7 @@ struct RingPlan {
   int kslice = 0;      // K tiles per slice
   int64_t bytes = 0;   // workspace of the partial sums (0: one slice)
   double us = 0;       // modelled time
+  bool uneven = false;  // 128 x 128 tiles, unsplit, a second workgroup on part of the CUs
 };
 
 // The fastest plan by the time model whose workspace is at most max_bytes.

@@ -425,6 +425,7 @@ RingPlan ring_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool b_kcont,
         best.kslice = static_cast<int>(slice);
         best.bytes = bytes;
         best.us = us;
+        best.uneven = s == 1 && f.bm == 128 && f.per_cu == 2 && wgs > kCUs && wgs < slots;
       }
     }
   }
