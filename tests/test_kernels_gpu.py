@@ -1068,7 +1068,8 @@ def test_attention_causal_mask_matches_causal_positions():
 @pytest.mark.parametrize("kind,b,mq,sk,causal_q", [
     ("none", 2, 17, 64, 0), ("none", 1, 129, 70, 0), ("positions", 2, 3 * 77, 77, 77),
     ("positions", 1, 255, 255, 255), ("causal", 2, 4 * 77, 80, 77), ("window", 2, 300, 328, 0),
-    ("holes", 3, 200, 320, 0), ("row", 2, 140, 72, 0)])
+    ("holes", 3, 200, 320, 0), ("row", 2, 140, 72, 0),
+    ("lowest", 2, 140, 72, 0), ("lowest", 1, 200, 320, 0)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
     # row counts off the 128-row block: the oracle's rows, the same bits as
@@ -1082,6 +1083,13 @@ def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
     if kind == "row":
         mask = torch.where(torch.arange(sk) < sk - 9, 0.0, float("-inf")).to(dtype).expand(mq, sk)
         md = mask[0].contiguous().to(DEV)
+    elif kind == "lowest":
+        # left padding as finite masks have it: rows with every key at the
+        # type's lowest value (uniform weights), the others with some
+        mask = torch.zeros(mq, sk, dtype=dtype)
+        mask[:, :13] = torch.finfo(dtype).min
+        mask[:37] = torch.finfo(dtype).min
+        md, ldm = mask.to(DEV), sk
     elif kind not in ("none", "positions"):
         mask = _block_mask(kind, b, mq, sk, causal_q).to(dtype)
         md, ldm, sm = mask.to(DEV), sk, mq * sk if mask.dim() == 3 else 0

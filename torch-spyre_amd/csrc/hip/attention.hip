@@ -101,6 +101,7 @@ struct AttnArgs {
   int64_t nkb;          // key blocks (ceil(sk / 64))
   float scale_log2;  // scale * log2(e) (scale > 0)
   float inv_scale;   // 1 / scale: masks join the raw scores as mask / scale
+  float mask_floor;  // lowest finite mask / scale
   void* o;
   int64_t ldo, so;
 };
@@ -157,6 +158,21 @@ __device__ inline void wait_vmcnt() {
 // s_waitcnt immediate for vmcnt(0) alone (gfx9 fields: vmcnt [3:0] and
 // [15:14], expcnt [6:4], lgkmcnt [11:8]; the others at their maximum).
 constexpr int kWaitVmcnt0 = 0x0F70;
+
+// A raw score with its mask value, s + mask / scale.  Masks are often filled with
+// the type's lowest value; in bf16 that overflows to -inf once divided by the
+// scale and turned a row with nothing else into NaN, where softmax over equal
+// values is uniform.  Finite values stop at `floor` instead, a power of two of
+// at most 2^31 in log2 units: ordinary scores vanish beside it, its product with
+// the scale is exact, and the rounding of values above it (2^6) stays inside
+// exp2's range.  -inf and NaN pass, dropped keys stay -inf.
+template <typename T>
+__device__ inline float masked_score(float s, uint16_t bits, float inv_scale, float floor) {
+  const float v = Num<T>::to_f(__builtin_bit_cast(T, bits));
+  const float x = fmaf(v, inv_scale, s);
+  if constexpr (__is_same(T, half_t)) return x;  // (fp16 ends above the floor)
+  return v * inv_scale < floor && v > -INFINITY ? s + floor : x;
+}
 
 // Mask block classes (values of the pre-pass's bytes).
 constexpr uint8_t MB_ZERO = 0, MB_MIXED = 1, MB_NEGINF = 2;
@@ -469,8 +485,7 @@ attn_fwd_kernel(const AttnArgs p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const uint16_t bits = static_cast<uint16_t>(mv[i >> 1] >> (16 * (i & 1)));
-              s[t][4 * rg + i] = fmaf(Num<T>::to_f(__builtin_bit_cast(T, bits)), p.inv_scale,
-                                      s[t][4 * rg + i]);
+              s[t][4 * rg + i] = masked_score<T>(s[t][4 * rg + i], bits, p.inv_scale, p.mask_floor);
             }
           }
       } else {
@@ -481,8 +496,8 @@ attn_fwd_kernel(const AttnArgs p) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               if (k0 + 32 * t + 8 * rg + 4 * h + i < sk32)
-                s[t][4 * rg + i] = fmaf(Num<T>::to_f(reinterpret_cast<const T*>(mp)[32 * t + 8 * rg + i]),
-                                        p.inv_scale, s[t][4 * rg + i]);
+                s[t][4 * rg + i] = masked_score<T>(s[t][4 * rg + i], mp[32 * t + 8 * rg + i],
+                                                p.inv_scale, p.mask_floor);
       }
     }
     float mb = -INFINITY;
@@ -666,6 +681,7 @@ int attention_run(bool any_rows, sph_dtype dtype, int64_t batch, int64_t mq, int
   p.nkb = (sk + AK - 1) / AK;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.inv_scale = 1.0f / scale;
+  p.mask_floor = -exp2f(floorf(31.0f - log2f(p.scale_log2)));
   p.o = o;
   p.ldo = ldo;
   p.so = stride_o;
