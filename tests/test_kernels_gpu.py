@@ -61,6 +61,39 @@ def test_softmax_shapes(rows, cols):
     np.testing.assert_allclose(np32(yd).sum(-1), 1.0, rtol=2e-2)
 
 
+@pytest.mark.parametrize("cols", [100, 512, 4096, 8191, 8193, 20000, 49155, 65537, 131071, 131073])
+@pytest.mark.parametrize("log,causal", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_softmax_finite_extremes(cols, log, causal, dtype):
+    # the type's lowest and largest values are finite: a row of equal values is
+    # uniform whatever they are, a largest value takes the whole weight
+    _log(f"softmax extremes {cols} log={log} causal={causal} {dtype}")
+    lo, hi = torch.finfo(dtype).min, torch.finfo(dtype).max
+    x = randn((7, cols), k=5, scale=3.0).to(dtype)
+    x[0] = lo
+    x[1] = hi
+    x[2, 9] = hi
+    x[3] = lo
+    x[3, 3:11] = hi
+    x[4, : cols // 2] = lo
+    x[5] = lo
+    x[5, 5] = lo / 2
+    x[6] = float("-inf")
+    x[6, 8:30] = lo
+    xd = x.to(DEV)
+    yd = torch.empty_like(xd)
+    _capi.call("sph_softmax_rows", DT[dtype], DT[dtype], _p(xd), cols, _p(yd), cols, 7, cols, 1.0,
+               log + 2 * causal, 7, cols - 20, _stream())
+    _sync()
+    xf = x.double()
+    if causal:
+        c = torch.arange(cols)[None, :] > torch.arange(7)[:, None] + cols - 20
+        xf = xf.masked_fill(c, float("-inf"))
+    want = (torch.log_softmax(xf, -1) if log else torch.softmax(xf, -1)).to(dtype).double()
+    tol = {torch.float16: 2e-3, torch.bfloat16: 1e-2, torch.float32: 1e-4}[dtype]
+    torch.testing.assert_close(yd.cpu().double(), want, rtol=tol, atol=1e-3 if log else 1e-7)
+
+
 @pytest.mark.parametrize("rows,cols", [(3, 8193), (2, 16384), (2, 16391), (2, 32769), (3, 49155),
                                        (2, 65536), (1, 65537), (1, 131071), (1, 131073)])
 @pytest.mark.parametrize("log,causal,scale", [(0, 0, 1.0), (1, 0, 0.5), (0, 1, 1.0), (1, 1, 1.0),

@@ -92,6 +92,17 @@ constexpr float kLn2 = 0.6931471805599453f;
 // ----------------------------------------------------------------------------
 // Softmax
 // ----------------------------------------------------------------------------
+// Units in which the register kernels hold a row: x * scale * kPre, exponents
+// exp2(difference * kExp), logarithms (difference - log2(sum) * kLog) * kOut.
+// fp16 rows are held in log2 units; bf16 and fp32 values past 2.36e38, the
+// types' lowest value among them, would overflow there.
+template <typename TI>
+struct SoftmaxUnit {
+  static constexpr bool kLog2 = __is_same(TI, half_t);
+  static constexpr float kPre = kLog2 ? kLog2e : 1.f, kExp = kLog2 ? 1.f : kLog2e;
+  static constexpr float kLog = kLog2 ? 1.f : kLn2, kOut = kLog2 ? kLn2 : 1.f;
+};
+
 template <typename TI, typename TO, int TPR, int VPT>
 __global__ void __launch_bounds__(block_of<TPR>())
 softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
@@ -115,16 +126,16 @@ softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
       for (int j = 0; j < 8; ++j) v[i][j] = ninf;
   }
   // Row lengths here fit in 32 bits (at most TPR * VPT * 8 columns), so the
-  // causal limit and the column index are 32-bit.  Values are kept in log2
-  // units (x * scale * log2 e): the exponential is then the hardware exp2 of
-  // a difference, whose results below 2^-126 flush to zero, which changes
-  // nothing next to a row sum of at least 1.
+  // causal limit and the column index are 32-bit.  The exponential is the
+  // hardware exp2 of a difference, whose results below 2^-126 flush to zero,
+  // which changes nothing next to a row sum of at least 1.
   int limit = static_cast<int>(cols);
   if ((flags & SPH_SOFTMAX_CAUSAL) && valid) {
     const int64_t lim = (row % qlen) + qoff + 1;
     limit = lim < cols ? static_cast<int>(lim) : limit;
   }
-  const float sl = scale * kLog2e;
+  using U = SoftmaxUnit<TI>;
+  const float sl = scale * U::kPre;
   float m = ninf;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
@@ -143,18 +154,18 @@ softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
   for (int i = 0; i < VPT; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float e = __builtin_amdgcn_exp2f(v[i][j] - m);
+      const float e = __builtin_amdgcn_exp2f((v[i][j] - m) * U::kExp);
       s += e;
       if (!(flags & SPH_SOFTMAX_LOG)) v[i][j] = e;
     }
   s = group_reduce<SumOp, TPR>(s, lds);
   if (!valid) return;
   if (flags & SPH_SOFTMAX_LOG) {
-    const float ls = log2f(s);
+    const float ls = log2f(s) * U::kLog;
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = (v[i][j] - m - ls) * kLn2;
+      for (int j = 0; j < 8; ++j) v[i][j] = (v[i][j] - m - ls) * U::kOut;
   } else {
     const float inv = 1.0f / s;
 #pragma unroll
@@ -165,14 +176,16 @@ softmax_regs(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y,
   store_row<TO, TPR, VPT>(y + row * ldy, cols, t, v);
 }
 
-// (max, sum) state of an online softmax: `s` sums exp2(x - m) over the
-// values seen, m their maximum.  Merging two states rescales both sums to the
+// (max, sum) state of an online softmax: `s` sums e^(x - m) over the
+// values seen, m their maximum (both in U's units).  Merging two states rescales both sums to the
 // larger maximum.  A state that has seen only -inf is (-inf, 0); the base
 // 0 in place of an infinite maximum keeps exp2 away from inf - inf.
+template <typename U>
 __device__ inline void ms_merge(float& m, float& s, float mo, float so) {
   const float mn = fmaxf(m, mo);
   const float base = mn == -INFINITY ? 0.f : mn;
-  s = s * __builtin_amdgcn_exp2f(m - base) + so * __builtin_amdgcn_exp2f(mo - base);
+  s = s * __builtin_amdgcn_exp2f((m - base) * U::kExp) +
+      so * __builtin_amdgcn_exp2f((mo - base) * U::kExp);
   m = mn;
 }
 
@@ -188,13 +201,13 @@ __device__ inline float dpp_f(float v) {
 // of several waves one LDS exchange with a single barrier.  `lds_m` and
 // `lds_s` hold blockDim/64 floats each; every thread of the workgroup must
 // reach the call.
-template <int TPR>
+template <int TPR, typename U>
 __device__ inline void group_ms(float& m, float& s, float* lds_m, float* lds_s) {
   static_assert(TPR % kWave == 0, "row groups of whole waves");
-  ms_merge(m, s, dpp_f<0xB1>(m), dpp_f<0xB1>(s));
-  ms_merge(m, s, dpp_f<0x4E>(m), dpp_f<0x4E>(s));
-  ms_merge(m, s, dpp_f<0x141>(m), dpp_f<0x141>(s));
-  ms_merge(m, s, dpp_f<0x140>(m), dpp_f<0x140>(s));
+  ms_merge<U>(m, s, dpp_f<0xB1>(m), dpp_f<0xB1>(s));
+  ms_merge<U>(m, s, dpp_f<0x4E>(m), dpp_f<0x4E>(s));
+  ms_merge<U>(m, s, dpp_f<0x141>(m), dpp_f<0x141>(s));
+  ms_merge<U>(m, s, dpp_f<0x140>(m), dpp_f<0x140>(s));
   float rm[4], rs[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -204,7 +217,7 @@ __device__ inline void group_ms(float& m, float& s, float* lds_m, float* lds_s) 
   m = rm[0];
   s = rs[0];
 #pragma unroll
-  for (int r = 1; r < 4; ++r) ms_merge(m, s, rm[r], rs[r]);
+  for (int r = 1; r < 4; ++r) ms_merge<U>(m, s, rm[r], rs[r]);
   if constexpr (TPR > kWave) {
     constexpr int NW = TPR / kWave;
     const int wave = threadIdx.x / kWave;
@@ -219,24 +232,24 @@ __device__ inline void group_ms(float& m, float& s, float* lds_m, float* lds_s) 
       // instead of 15 merges in series
       m = lds_m[threadIdx.x & 15];
       s = lds_s[threadIdx.x & 15];
-      ms_merge(m, s, dpp_f<0xB1>(m), dpp_f<0xB1>(s));
-      ms_merge(m, s, dpp_f<0x4E>(m), dpp_f<0x4E>(s));
-      ms_merge(m, s, dpp_f<0x141>(m), dpp_f<0x141>(s));
-      ms_merge(m, s, dpp_f<0x140>(m), dpp_f<0x140>(s));
+      ms_merge<U>(m, s, dpp_f<0xB1>(m), dpp_f<0xB1>(s));
+      ms_merge<U>(m, s, dpp_f<0x4E>(m), dpp_f<0x4E>(s));
+      ms_merge<U>(m, s, dpp_f<0x141>(m), dpp_f<0x141>(s));
+      ms_merge<U>(m, s, dpp_f<0x140>(m), dpp_f<0x140>(s));
     } else {
       m = lds_m[first];
       s = lds_s[first];
 #pragma unroll
-      for (int k = 1; k < NW; ++k) ms_merge(m, s, lds_m[first + k], lds_s[first + k]);
+      for (int k = 1; k < NW; ++k) ms_merge<U>(m, s, lds_m[first + k], lds_s[first + k]);
     }
   }
 }
 
-// Rows of exactly TPR * VPT * 8 columns (c1's [512, 4096] among them): whole chunks without per-chunk bounds tests, the
-// causal mask and log form chosen once per thread rather than tested per
-// element, and one combined (max, sum) reduction per row: each thread sums
-// exp2 of its values against its own maximum, and the states merge in one
-// pass (group_ms).  At this size the kernel is latency-bound: a kernel
+// Rows of exactly TPR * VPT * 8 columns (c1's [512, 4096] among them): whole
+// chunks without per-chunk bounds tests, the causal mask and log form chosen
+// once per thread rather than tested per element, and one combined (max, sum)
+// reduction per row: each thread sums e^x of its values against its own
+// maximum, and the states merge in one pass (group_ms).  At this size the kernel is latency-bound: a kernel
 // launched back to back costs 1.53 us empty and 2.69 us when one thread
 // loads and stores one value, and this one 2.9-3.0 us at [512, 4096] (on
 // 128 threads x 4 chunks per row, two rows per workgroup), against 3.3 us
@@ -256,7 +269,8 @@ softmax_full(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t 
   float v[VPT][8];
 #pragma unroll
   for (int i = 0; i < VPT; ++i) load8u<TI>(x + row * ldx + (i * TPR + t) * 8, v[i]);
-  const float sl = scale * kLog2e;
+  using U = SoftmaxUnit<TI>;
+  const float sl = scale * U::kPre;
   float m = -INFINITY;
   if (flags & SPH_SOFTMAX_CAUSAL) {
     const int64_t lim = (row % qlen) + qoff + 1;
@@ -287,32 +301,32 @@ softmax_full(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t 
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f(v[i][j] - bt);
+      for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f((v[i][j] - bt) * U::kExp);
   } else {
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        v[i][j] = __builtin_amdgcn_exp2f(v[i][j] - bt);
+        v[i][j] = __builtin_amdgcn_exp2f((v[i][j] - bt) * U::kExp);
         s += v[i][j];
       }
   }
-  group_ms<TPR>(m, s, lds_m, lds_s);
+  group_ms<TPR, U>(m, s, lds_m, lds_s);
   if (!valid) return;
   if (lg) {
-    const float ls = m + log2f(s);
+    const float ls = log2f(s) * U::kLog;
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = (v[i][j] - ls) * kLn2;
+      for (int j = 0; j < 8; ++j) v[i][j] = (v[i][j] - m - ls) * U::kOut;
   } else {
-    // e^(x - m) / s = exp2(v - bt) * exp2(bt - m) / s.  A thread whose
+    // e^(x - m) / s = e^(x - bt) * e^(bt - m) / s.  A thread whose
     // values are all masked holds zeros (its factor is 0, never exp2 of a
     // large difference); a row with no finite value is NaN, as softmax over
     // all -inf is.
     const float f = m == -INFINITY   ? NAN
                     : mt == -INFINITY ? 0.f
-                                      : __builtin_amdgcn_exp2f(bt - m) / s;
+                                      : __builtin_amdgcn_exp2f((bt - m) * U::kExp) / s;
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
 #pragma unroll
@@ -328,6 +342,13 @@ softmax_full(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t 
 // as floats, 8 chunks spilled), one combined (max, sum) reduction, the
 // exponentials of the output taken again.  With few rows a CU's own rate sets
 // the time: 64 x 49155 bf16 log-softmax 35 us -> 9.9 us.
+//
+// Exponents are one FMA against the maximum in log2 units, b = m u (u the log2
+// units per unit of x); its rounding is the same for every value of the row.
+// Past |b| = kFarLog2 that rounding outgrows exp2's argument, and b overflows
+// for values past 2.36e38: a row with such a maximum takes the differences to
+// the raw maximum instead (its exponentials cost one operation more).
+constexpr float kFarLog2 = 0x1p24f;
 template <typename TI, typename TO, int VPT>
 __global__ void __launch_bounds__(1024)
 softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_t ldy, int cols,
@@ -373,39 +394,71 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
     const TI* e = reinterpret_cast<const TI*>(&raw[i]);
     return Num<TI>::to_f(e[j]);
   };
+  // Each pass widens the values anew: kept from one pass to the next as floats
+  // they would take twice the registers and spill.
+  auto repack = [&] {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) asm volatile("" : "+v"(raw[i]));
+  };
   float m = -INFINITY;
 #pragma unroll
   for (int i = 0; i < VPT; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) m = fmaxf(m, val(i, j));
-  m *= sl;
-  const float bt = m == -INFINITY ? 0.f : m;
+  repack();
+  // (a thread whose values all lie far below 0 sums to 0 and drops out: state
+  // -inf; far above, the row is one of those)
+  float b = m * sl;
+  const bool near = fabsf(b) <= kFarLog2;
+  const float bt = near ? b : 0.f;
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f(fmaf(val(i, j), sl, -bt));
-  group_ms<1024>(m, s, lds_m, lds_s);
+  repack();
+  if (!near) b = b < 0.f ? -INFINITY : INFINITY;
+  group_ms<1024, SoftmaxUnit<half_t>>(b, s, lds_m, lds_s);  // (log2 units)
   const bool lg = flags & SPH_SOFTMAX_LOG;
-  // (a row with no finite value is NaN in both forms: -inf - -inf)
-  const float off = lg ? m + log2f(s) : m, inv = 1.0f / s;
   TO* yr = y + row * ldy;
+  auto emit = [&](auto f) {
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    const int c0 = (i * 1024 + threadIdx.x) * 8;
-    if (c0 >= cols) continue;
-    float v[8];
-    if (lg) {
+    for (int i = 0; i < VPT; ++i) {
+      const int c0 = (i * 1024 + threadIdx.x) * 8;
+      if (c0 >= cols) continue;
+      float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = fmaf(val(i, j), sl, -off) * kLn2;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_exp2f(fmaf(val(i, j), sl, -off)) * inv;
+      for (int j = 0; j < 8; ++j) v[j] = f(val(i, j));
+      if (c0 + 8 <= cols)
+        store8u<TO>(yr + c0, v);
+      else
+        store8_partial<TO>(yr + c0, cols - c0, v);
     }
-    if (c0 + 8 <= cols)
-      store8u<TO>(yr + c0, v);
-    else
-      store8_partial<TO>(yr + c0, cols - c0, v);
+  };
+  if (!(fabsf(b) <= kFarLog2)) {  // (the same in every thread)
+    __syncthreads();              // group_ms has read its states
+    m = group_reduce<MaxOp, 1024>(m, lds_m);
+    s = 0.f;  // (a row of -inf alone is NaN: -inf - -inf)
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += __builtin_amdgcn_exp2f((val(i, j) - m) * sl);
+    repack();
+    s = group_reduce<SumOp, 1024>(s, lds_m);
+    const float ls = log2f(s) * kLn2, inv = 1.0f / s;
+    emit([&](float a) {
+      return lg ? fmaf(a - m, scale, -ls) : __builtin_amdgcn_exp2f((a - m) * sl) * inv;
+    });
+    return;
+  }
+  if (lg) {
+    // the maximum itself is the 16-bit value next to b / u; s is relative to b
+    m = Num<TI>::to_f(Num<TI>::from_f(b / sl));
+    const float ls = (log2f(s) - fmaf(m, sl, -b)) * kLn2;
+    emit([&](float a) { return fmaf(a - m, scale, -ls); });
+  } else {
+    const float inv = 1.0f / s;
+    emit([&](float a) { return __builtin_amdgcn_exp2f(fmaf(a, sl, -b)) * inv; });
   }
 }
 
