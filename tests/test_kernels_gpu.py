@@ -94,6 +94,32 @@ def test_softmax_finite_extremes(cols, log, causal, dtype):
     torch.testing.assert_close(yd.cpu().double(), want, rtol=tol, atol=1e-3 if log else 1e-7)
 
 
+@pytest.mark.parametrize("cols", [100, 4096, 8193, 16384, 40001, 70000, 131073])
+@pytest.mark.parametrize("scale", [-1.5, 0.0])
+@pytest.mark.parametrize("log,causal", [(0, 1), (1, 0)])
+def test_softmax_scales_not_positive(cols, scale, log, causal):
+    # a negative scale puts the weight on the smallest values, a scale of 0
+    # makes the row uniform over its visible columns
+    _log(f"softmax {cols} scale={scale} log={log} causal={causal}")
+    for dtype in (torch.float16, torch.bfloat16):
+        x = randn((4, cols), k=6, scale=3.0, dtype=dtype)
+        if not scale:
+            x[1, 7] = float("inf")  # inf * 0: the row is NaN
+        xd = x.to(DEV)
+        yd = torch.empty_like(xd)
+        _capi.call("sph_softmax_rows", DT[dtype], DT[dtype], _p(xd), cols, _p(yd), cols, 4, cols,
+                   scale, log + 2 * causal, 4, cols - 30, _stream())
+        _sync()
+        xf = x.double() * scale
+        if causal:
+            c = torch.arange(cols)[None, :] > torch.arange(4)[:, None] + cols - 30
+            xf = xf.masked_fill(c, float("-inf"))
+        want = torch.log_softmax(xf, -1) if log else torch.softmax(xf, -1)
+        tol = 2e-3 if dtype == torch.float16 else 1e-2
+        torch.testing.assert_close(yd.cpu().double(), want, rtol=tol, atol=1e-3 if log else 1e-7,
+                                   equal_nan=True)
+
+
 @pytest.mark.parametrize("rows,cols", [(3, 8193), (2, 16384), (2, 16391), (2, 32769), (3, 49155),
                                        (2, 65536), (1, 65537), (1, 131071), (1, 131073)])
 @pytest.mark.parametrize("log,causal,scale", [(0, 0, 1.0), (1, 0, 0.5), (0, 1, 1.0), (1, 1, 1.0),

@@ -364,7 +364,7 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
   }
   // columns past the limit become -inf in the registers, so the passes below
   // test nothing (a CU's vector ALUs are as busy as its memory path here)
-  constexpr uint32_t kNegInf = __is_same(TI, bf16_t) ? 0xff80u : 0xfc00u;
+  constexpr uint32_t kInf = __is_same(TI, bf16_t) ? 0x7f80u : 0x7c00u, kNegInf = kInf | 0x8000u;
   u32x4 raw[VPT];
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
@@ -379,6 +379,33 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
         raw[i][j] = lo | (hi << 16);
       }
   }
+  // Each pass widens the values anew: kept from one pass to the next as floats
+  // they would take twice the registers and spill.
+  auto repack = [&] {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) asm volatile("" : "+v"(raw[i]));
+  };
+  // A negative scale: negated values under its magnitude; 0 (or NaN): every
+  // finite value 0 (NaN), the others NaN.  The columns past the row stay -inf.
+  float as = scale;
+  if (!(scale > 0.f)) {
+    as = scale < 0.f ? -scale : 1.f;
+    auto half = [&](uint32_t h) -> uint32_t {
+      if (scale < 0.f) return h ^ 0x8000u;
+      return scale == 0.f && (h & kInf) != kInf ? 0u : 0x7fffu;
+    };
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int n = cols - (i * 1024 + static_cast<int>(threadIdx.x)) * 8;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t w = raw[i][j];
+        raw[i][j] = (2 * j < n ? half(w & 0xffffu) : kNegInf) |
+                    ((2 * j + 1 < n ? half(w >> 16) : kNegInf) << 16);
+      }
+      asm volatile("" : "+v"(raw[i]));
+    }
+  }
   if (limit < cols) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
@@ -389,16 +416,10 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
         if (c + 1 >= limit) raw[i][j] = (raw[i][j] & 0xffffu) | (kNegInf << 16);
       }
   }
-  const float sl = scale * kLog2e;  // log2 units; scale > 0
+  const float sl = as * kLog2e;  // log2 units per unit of x
   auto val = [&](int i, int j) {
     const TI* e = reinterpret_cast<const TI*>(&raw[i]);
     return Num<TI>::to_f(e[j]);
-  };
-  // Each pass widens the values anew: kept from one pass to the next as floats
-  // they would take twice the registers and spill.
-  auto repack = [&] {
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) asm volatile("" : "+v"(raw[i]));
   };
   float m = -INFINITY;
 #pragma unroll
@@ -447,7 +468,7 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
     s = group_reduce<SumOp, 1024>(s, lds_m);
     const float ls = log2f(s) * kLn2, inv = 1.0f / s;
     emit([&](float a) {
-      return lg ? fmaf(a - m, scale, -ls) : __builtin_amdgcn_exp2f((a - m) * sl) * inv;
+      return lg ? fmaf(a - m, as, -ls) : __builtin_amdgcn_exp2f((a - m) * sl) * inv;
     });
     return;
   }
@@ -455,7 +476,7 @@ softmax_packed(const TI* __restrict__ x, int64_t ldx, TO* __restrict__ y, int64_
     // the maximum itself is the 16-bit value next to b / u; s is relative to b
     m = Num<TI>::to_f(Num<TI>::from_f(b / sl));
     const float ls = (log2f(s) - fmaf(m, sl, -b)) * kLn2;
-    emit([&](float a) { return fmaf(a - m, scale, -ls); });
+    emit([&](float a) { return fmaf(a - m, as, -ls); });
   } else {
     const float inv = 1.0f / s;
     emit([&](float a) { return __builtin_amdgcn_exp2f(fmaf(a, sl, -b)) * inv; });
@@ -809,7 +830,7 @@ int softmax_impl(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
     return check_launch("sph_softmax_rows");
   }
   if constexpr (sizeof(TI) == 2) {
-    if (cols > 8192 && cols <= 131072 && scale > 0.f) {
+    if (cols > 8192 && cols <= 131072) {
       const unsigned g = static_cast<unsigned>(rows);
       const int n = static_cast<int>(cols);
       if (cols <= 16384)
@@ -843,7 +864,7 @@ int softmax_impl(const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows,
     SPH_SOFTMAX_CASE(2)
     SPH_SOFTMAX_CASE(3)
     default:
-      if constexpr (sizeof(TI) == 4) {  // (16-bit rows: softmax_packed; looped for scale <= 0)
+      if constexpr (sizeof(TI) == 4) {  // (16-bit rows: softmax_packed)
         switch (cfg) {
           SPH_SOFTMAX_CASE(4)
           SPH_SOFTMAX_CASE(5)
