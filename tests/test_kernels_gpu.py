@@ -1177,6 +1177,47 @@ def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
     assert rc == 1002
 
 
+@pytest.mark.parametrize("kind", ["levels", "lowest", "largest"])
+@pytest.mark.parametrize("b,mq,sk", [(2, 17, 72), (2, 140, 328), (1, 256, 256)])
+@pytest.mark.parametrize("scale", [1 / math.sqrt(128), 2.0])  # 2.0: the lowest overflows in log2 units only
+def test_attention_finite_mask_values(kind, b, mq, sk, scale):
+    # bf16 masks of finite values: each keeps its rank (padding at the type's
+    # lowest value below a causal fill of -1e9; the largest value above all),
+    # and rows with nothing else than the lowest are uniform whatever the
+    # scores are
+    _log(f"attention finite mask {kind} b={b} mq={mq} sk={sk} scale={scale}")
+    dtype = torch.bfloat16
+    f = torch.finfo(dtype)
+    wide = 4.0 if kind == "lowest" else 1.0  # raw scores to ~700
+    q = randn((b, mq, 128), k=71, scale=wide, dtype=dtype)
+    k = randn((b, sk, 128), k=72, scale=wide, dtype=dtype)
+    v = randn((b, sk, 128), k=73, dtype=dtype)
+    mask = torch.zeros(b, mq, sk)
+    if kind == "levels":
+        mask[:, :, 30:] = -1e9          # later keys
+        mask[:, :, :30] = f.min         # padding: rows with no visible key
+        mask[:, 1::2, 5:9] = 0.0        # every other row sees some
+    elif kind == "lowest":
+        mask[:, :, :13] = f.min
+        mask[:, ::3] = f.min
+    else:
+        mask[:, ::2, 11:17] = f.max
+        mask[:, :, 40:] = f.min
+    mask = mask.to(dtype)
+    want = O.attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), scale,
+                       mask=mask.float().numpy())
+    qd, kd, vd, md = q.to(DEV), k.to(DEV), v.to(DEV), mask.to(DEV)
+    nws = _capi.lib().sph_attention_workspace_bytes(b, mq, sk, mq * sk)
+    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
+    for w_n in (0, nws):
+        o = torch.full((b, mq, 128), 7.0, dtype=dtype, device=DEV)
+        _capi.call("sph_attention_fwd_rows", DT[dtype], b, mq, sk, 128, _p(qd), 128, mq * 128,
+                   _p(kd), 128, sk * 128, _p(vd), 128, sk * 128, _p(md), sk, mq * sk, 0, 0, scale,
+                   _p(o), 128, mq * 128, _p(ws) if w_n else None, w_n, _stream())
+        _sync()
+        assert_close_fp(o, want, out_dtype=dtype, what="finite masks", rtol=2e-2, atol=2e-2)
+
+
 def test_attention_fused_c4_shape():
     # the c4 layer's attention: 8 KV heads, 4 query heads stacked per KV
     # head (mq = 4 * 2048), causal over 2048 keys; one batch element

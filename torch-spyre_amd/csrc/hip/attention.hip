@@ -56,6 +56,7 @@
 //     length thus keeps its scores on chip: 3 x 777 tokens (24 x 3108 rows x
 //     777 keys, causal mask, bf16) 57 us + 9 us of pre-pass, against 860 us
 //     for the two products, the masking and the softmax it replaces there.
+#include <cstring>
 #include <mutex>
 
 #include "sph_common.h"
@@ -67,6 +68,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 #define SPH_LDS __attribute__((address_space(3)))
@@ -101,7 +103,10 @@ struct AttnArgs {
   int64_t nkb;          // key blocks (ceil(sk / 64))
   float scale_log2;  // scale * log2(e) (scale > 0)
   float inv_scale;   // 1 / scale: masks join the raw scores as mask / scale
-  float mask_floor;  // lowest finite mask / scale
+  float far_raw;     // 2^24 log2 units in raw scores: past it, differences first
+  // bf16 mask magnitudes (bits) from huge_lo on, huge_n of them below infinity,
+  // may overflow in mask / scale
+  uint32_t huge_lo, huge_n;
   void* o;
   int64_t ldo, so;
 };
@@ -159,19 +164,10 @@ __device__ inline void wait_vmcnt() {
 // [15:14], expcnt [6:4], lgkmcnt [11:8]; the others at their maximum).
 constexpr int kWaitVmcnt0 = 0x0F70;
 
-// A raw score with its mask value, s + mask / scale.  Masks are often filled with
-// the type's lowest value; in bf16 that overflows to -inf once divided by the
-// scale and turned a row with nothing else into NaN, where softmax over equal
-// values is uniform.  Finite values stop at `floor` instead, a power of two of
-// at most 2^31 in log2 units: ordinary scores vanish beside it, its product with
-// the scale is exact, and the rounding of values above it (2^6) stays inside
-// exp2's range.  -inf and NaN pass, dropped keys stay -inf.
-template <typename T>
-__device__ inline float masked_score(float s, uint16_t bits, float inv_scale, float floor) {
-  const float v = Num<T>::to_f(__builtin_bit_cast(T, bits));
-  const float x = fmaf(v, inv_scale, s);
-  if constexpr (__is_same(T, half_t)) return x;  // (fp16 ends above the floor)
-  return v * inv_scale < floor && v > -INFINITY ? s + floor : x;
+// a * b, never contracted into an FMA with what uses it.
+__device__ inline float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
 }
 
 // Mask block classes (values of the pre-pass's bytes).
@@ -408,8 +404,12 @@ attn_fwd_kernel(const AttnArgs p) {
   // Online softmax state per row, in log2 units: O and l are relative to
   // 2^m_ref; m_ref follows the running max lazily (moved only when a row's
   // max passes it by more than 8, so exp2 arguments stay <= 8 and most
-  // blocks skip the rescale of O).
-  float m_ref = -INFINITY, l_run = 0.f;
+  // blocks skip the rescale of O).  With a mask the reference is also kept as a
+  // raw score: a row that has only seen huge finite masks takes differences to
+  // it, since the products with the scale would round by more than exp2's range
+  // or overflow.
+  float m_ref = -INFINITY, r_ref = -INFINITY, l_run = 0.f;
+  auto is_far = [&](float raw) { return fabsf(raw) > p.far_raw; };  // (infinite ones too)
   const uint16_t* Mrow =
       MASK ? static_cast<const uint16_t*>(p.mask) + b * p.smb + qrow * p.ldm : nullptr;
 
@@ -474,18 +474,28 @@ attn_fwd_kernel(const AttnArgs p) {
     }
     // Mixed mask blocks: add mask / scale.  Lane's keys for (t, rg):
     // k0 + 32 t + 8 rg + 4 h .. + 3, one 8-byte load each.
+    constexpr bool HUGE_MASK = MASK && !__is_same(T, half_t);  // (fp16 ends at 65504)
+    u16x2 near2 = {0xffffu, 0xffffu};  // least magnitude - huge_lo, modulo 2^16
     if (MASK && cls == MB_MIXED) {
       const uint16_t* mp = Mrow + k0 + 4 * h;
+      const u16x2 lo2 = {static_cast<uint16_t>(p.huge_lo), static_cast<uint16_t>(p.huge_lo)};
       if (k0 + AK <= p.sk) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg) {
             const u32x2 mv = *reinterpret_cast<const u32x2*>(mp + 32 * t + 8 * rg);
+            if constexpr (HUGE_MASK) {
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                near2 = __builtin_elementwise_min(
+                    near2, __builtin_bit_cast(u16x2, mv[i] & 0x7fff7fffu) - lo2);
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const uint16_t bits = static_cast<uint16_t>(mv[i >> 1] >> (16 * (i & 1)));
-              s[t][4 * rg + i] = masked_score<T>(s[t][4 * rg + i], bits, p.inv_scale, p.mask_floor);
+              s[t][4 * rg + i] = fmaf(Num<T>::to_f(__builtin_bit_cast(T, bits)), p.inv_scale,
+                                      s[t][4 * rg + i]);
             }
           }
       } else {
@@ -495,31 +505,81 @@ attn_fwd_kernel(const AttnArgs p) {
           for (int rg = 0; rg < 4; ++rg)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              if (k0 + 32 * t + 8 * rg + 4 * h + i < sk32)
-                s[t][4 * rg + i] = masked_score<T>(s[t][4 * rg + i], mp[32 * t + 8 * rg + i],
-                                                p.inv_scale, p.mask_floor);
+              if (k0 + 32 * t + 8 * rg + 4 * h + i < sk32) {
+                const uint16_t bits = mp[32 * t + 8 * rg + i];
+                if constexpr (HUGE_MASK)
+                  near2[0] = min(near2[0], static_cast<uint16_t>((bits & 0x7fffu) - p.huge_lo));
+                s[t][4 * rg + i] = fmaf(Num<T>::to_f(__builtin_bit_cast(T, bits)), p.inv_scale,
+                                        s[t][4 * rg + i]);
+              }
       }
     }
-    float mb = -INFINITY;
+    float mb;
+    auto block_max = [&] {
+      mb = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[t][r]);
-    mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+        for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[t][r]);
+      mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+    };
+    block_max();
+    // Finite bf16 masks whose quotient overflows (the type's lowest value, with
+    // which masks are often filled) became infinite.  Where that matters, in a
+    // row with no visible key yet or with a positive one, they become fp32's
+    // lowest (largest) value, beside which every score vanishes: rows with
+    // nothing else get uniform weights, as softmax over equal values does, and
+    // smaller masks (a causal fill of -1e9) keep their rank above.  (Clamped per
+    // element instead, blocks full of mask values took 6 % longer.)
+    if constexpr (HUGE_MASK) {
+      const bool huge = min(near2[0], near2[1]) < p.huge_n;
+      const bool redo = mb == INFINITY || (mb == -INFINITY && !(r_ref >= -p.far_raw));
+      if (__ballot(huge) != 0 && __ballot(redo) != 0) {
+        const T* mp = reinterpret_cast<const T*>(Mrow) + k0 + 4 * h;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int kx = 32 * t + 8 * (r >> 2) + (r & 3), key = k0 + 4 * h + kx;
+            bool keep = key < sk32;
+            if constexpr (CAUSAL) keep = keep && key <= qpos;
+            if (!keep || fabsf(s[t][r]) != INFINITY) continue;
+            const float v = Num<T>::to_f(mp[kx]);
+            if (fabsf(v) < INFINITY && fabsf(v * p.inv_scale) == INFINITY)
+              s[t][r] = copysignf(3.402823466e38f, v);
+          }
+        block_max();
+      }
+    }
     const float c = p.scale_log2;
     const float mbc = mb * c;  // block max, log2 units (-inf: nothing visible)
-    const bool grow = mbc > m_ref + 8.f;
+    bool grow = mbc > m_ref + 8.f;
+    const bool far_step = MASK && (is_far(mb) || is_far(r_ref));
+    const float step = (r_ref - mb) * c;
+    if (far_step) grow = step < -8.f;
     if (__ballot(grow) != 0) {  // wave-uniform: some row moves its reference
       const float m_new = grow ? mbc : m_ref;
-      const float alpha = grow ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;
+      const float alpha = grow ? __builtin_amdgcn_exp2f(far_step ? step : m_ref - m_new) : 1.f;
       l_run *= alpha;
 #pragma unroll
       for (int dt = 0; dt < AD / 32; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
       m_ref = m_new;
+      if (MASK && grow) r_ref = mb;
     }
-    const float neg = m_ref == -INFINITY ? 0.f : -m_ref;
+    float neg = m_ref == -INFINITY ? 0.f : -m_ref;
+    if constexpr (MASK) {
+      const bool far = is_far(r_ref) && r_ref > -INFINITY;
+      if (__ballot(far) != 0) {
+        const float sub = far ? r_ref : 0.f;
+        neg = far ? 0.f : neg;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[t][r] -= sub;
+      }
+    }
     float lb = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -562,7 +622,7 @@ attn_fwd_kernel(const AttnArgs p) {
   // through LDS (all DMA has landed: the loop ends with a wait + barrier).
   float* mg = reinterpret_cast<float*>(lds) + wq * (66 * 64) + lane;
   if (grp == 1) {
-    mg[0] = m_ref;
+    mg[0] = MASK ? r_ref : m_ref;
     mg[64] = l_run;
 #pragma unroll
     for (int dt = 0; dt < AD / 32; ++dt)
@@ -572,10 +632,19 @@ attn_fwd_kernel(const AttnArgs p) {
   __syncthreads();
   if (grp == 1) return;
   {
-    const float m1 = mg[0], l1 = mg[64];
-    const float m = fmaxf(m_ref, m1);
-    const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m);
-    const float a1 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
+    const float l1 = mg[64];
+    float m0 = m_ref, m1 = mg[0];
+    if constexpr (MASK) {
+      const float r1 = m1, r = fmaxf(r_ref, r1);
+      m1 = rounded_product(r1, p.scale_log2);  // (group 1's m_ref)
+      if (is_far(r_ref) || is_far(r1)) {  // relative to the larger one
+        m0 = (r_ref - r) * p.scale_log2;
+        m1 = (r1 - r) * p.scale_log2;
+      }
+    }
+    const float m = fmaxf(m0, m1);
+    const float a0 = m0 > -INFINITY ? __builtin_amdgcn_exp2f(m0 - m) : 0.f;
+    const float a1 = m1 > -INFINITY ? __builtin_amdgcn_exp2f(m1 - m) : 0.f;
     l_run = l_run * a0 + l1 * a1;
 #pragma unroll
     for (int dt = 0; dt < AD / 32; ++dt)
@@ -681,7 +750,13 @@ int attention_run(bool any_rows, sph_dtype dtype, int64_t batch, int64_t mq, int
   p.nkb = (sk + AK - 1) / AK;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.inv_scale = 1.0f / scale;
-  p.mask_floor = -exp2f(floorf(31.0f - log2f(p.scale_log2)));
+  p.far_raw = 0x1p24f / p.scale_log2;
+  // (bits of FLT_MAX * scale, rounded towards zero)
+  const float huge = 3.402823466e38f * (scale < 1.f ? scale : 1.f);
+  uint32_t hb;
+  std::memcpy(&hb, &huge, 4);
+  p.huge_lo = scale < 1.f ? hb >> 16 : 0x7f80u;
+  p.huge_n = 0x7f80u - p.huge_lo;
   p.o = o;
   p.ldo = ldo;
   p.so = stride_o;
