@@ -1178,13 +1178,13 @@ def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
 
 
 @pytest.mark.parametrize("kind", ["levels", "lowest", "largest"])
-@pytest.mark.parametrize("b,mq,sk", [(2, 17, 72), (2, 140, 328), (1, 256, 256)])
+@pytest.mark.parametrize("b,mq,sk", [(3, 1, 72), (2, 16, 320), (2, 17, 72), (2, 140, 328), (1, 256, 256)])
 @pytest.mark.parametrize("scale", [1 / math.sqrt(128), 2.0])  # 2.0: the lowest overflows in log2 units only
 def test_attention_finite_mask_values(kind, b, mq, sk, scale):
     # bf16 masks of finite values: each keeps its rank (padding at the type's
     # lowest value below a causal fill of -1e9; the largest value above all),
     # and rows with nothing else than the lowest are uniform whatever the
-    # scores are
+    # scores are (up to 16 rows run the decode kernel)
     _log(f"attention finite mask {kind} b={b} mq={mq} sk={sk} scale={scale}")
     dtype = torch.bfloat16
     f = torch.finfo(dtype)

@@ -44,7 +44,10 @@ struct DecArgs {
   int64_t ldm, smb;
   int64_t causal_q, causal_off;
   int mq, sk, nchunks, cps, nsplit;
-  float scale_log2;
+  // Scores are q * q_scale . k (+ mask) and exponents exp2(difference * unit):
+  // in log2 units, or with a mask in natural units, where a finite mask at
+  // bf16's lowest value (-3.39e38) stays finite.
+  float q_scale, unit;
   void* o;
   int64_t ldo, so;
   float* part;  // [batch][nsplit][mq][2 + 128] fp32, or null
@@ -69,13 +72,13 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(const DecArgs p) {
   const T* V = static_cast<const T*>(p.v) + b * p.svb;
   const T* M = p.mask ? static_cast<const T*>(p.mask) + b * p.smb : nullptr;
 
-  // Q rows, pre-multiplied by scale * log2(e)
+  // Q rows, pre-multiplied by the scale
   for (int x = t; x < mq * (DD / 8); x += 256) {
     const int i = x / (DD / 8), c = (x % (DD / 8)) * 8;
     float f[8];
     load8<T>(Q + i * p.ldq + c, f);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) qs[i][c + e] = f[e] * p.scale_log2;
+    for (int e = 0; e < 8; ++e) qs[i][c + e] = f[e] * p.q_scale;
   }
   // per-row softmax state, replicated across the lanes of the row's wave
   float m_run[4], l_run[4];
@@ -156,7 +159,7 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(const DecArgs p) {
       if (i >= mq) continue;  // uniform per wave
       float x = s[r];
       bool vis = lane < kn;
-      if (vis && M) x = fmaf(Num<T>::to_f(M[i * p.ldm + key]), kLog2eD, x);
+      if (vis && M) x += Num<T>::to_f(M[i * p.ldm + key]);
       if (p.causal_q > 0) vis = vis && key <= (i % p.causal_q) + p.causal_off;
       x = vis ? x : -INFINITY;
       float mx = x;
@@ -164,8 +167,8 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(const DecArgs p) {
       for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
       const float m_new = fmaxf(m_run[r], mx);
       // a row with nothing visible so far keeps a zero state (no -inf - -inf)
-      const float a = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run[r] - m_new);
-      const float pj = m_new == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x - m_new);
+      const float a = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run[r] - m_new) * p.unit);
+      const float pj = m_new == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((x - m_new) * p.unit);
       float sum = pj;
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
@@ -239,7 +242,7 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(const DecArgs p) {
 }
 
 // Merges the splits of batch entry blockIdx.y, row blockIdx.x: O = sum_s
-// 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s with M the largest m_s.  One
+// 2^((m_s - M) unit) o_s / sum_s 2^((m_s - M) unit) l_s with M the largest m_s.  One
 // thread per head-dim column; every split's values are loaded before use
 // (at most kMaxSplit splits).
 constexpr int kMaxSplit = 32;
@@ -263,7 +266,7 @@ __global__ void __launch_bounds__(DD) attn_decode_combine(const DecArgs p) {
   float lsum = 0.f, acc = 0.f;
 #pragma unroll
   for (int s = 0; s < kMaxSplit; ++s) {
-    const float w = (mx == -INFINITY || m[s] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[s] - mx);
+    const float w = (mx == -INFINITY || m[s] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m[s] - mx) * p.unit);
     lsum = fmaf(l[s], w, lsum);
     acc = fmaf(o[s], w, acc);
   }
@@ -352,7 +355,8 @@ extern "C" int sph_attention_decode(sph_dtype dtype, int64_t batch, int64_t mq, 
   p.causal_off = causal_off;
   p.mq = static_cast<int>(mq);
   p.sk = static_cast<int>(sk);
-  p.scale_log2 = scale * kLog2eD;
+  p.q_scale = mask != nullptr ? scale : scale * kLog2eD;
+  p.unit = mask != nullptr ? kLog2eD : 1.f;
   p.o = o;
   p.ldo = ldo;
   p.so = stride_o;
