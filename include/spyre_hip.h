@@ -261,6 +261,25 @@ int64_t sph_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k)
 int64_t sph_gemm_workspace_bytes_ex(int trans_a, int trans_b, int64_t batch, int64_t m, int64_t n,
                                     int64_t k, int64_t lda, int64_t ldb);
 
+/* What a product of these sizes runs on, without launching it (host only):
+ * plan[0] the kernel, [1] and [2] its tile (direct-load and ring kernels, else
+ * 0), [3] the K slices of its tiles, [4] which operands are copied into padded
+ * rows first (1: A, 2: B).  Operands and D with 16-byte aligned bases, batches
+ * and D without gaps; plain: alpha 1, no C, no activation; swiglu: the product
+ * of sph_gemm_swiglu_any. */
+typedef enum sph_gemm_kernel {
+  SPH_GEMM_STREAM = 1,       /* weight stream, batch 1, up to 8 rows */
+  SPH_GEMM_SKINNY = 2,       /* few rows, any batch */
+  SPH_GEMM_SHORT_K = 3,      /* K of 64 or 128, whole 128 x 128 tiles */
+  SPH_GEMM_SHORT_K_RING = 4, /* the same, persistent */
+  SPH_GEMM_DIRECT = 5,       /* direct global -> LDS loads, 256-row tiles */
+  SPH_GEMM_RING = 6,         /* ring of LDS stages, small and ragged rows */
+  SPH_GEMM_STAGED = 7        /* register-staged, any layout and alignment */
+} sph_gemm_kernel;
+int sph_gemm_plan(int trans_a, int trans_b, int64_t batch, int64_t m, int64_t n, int64_t k,
+                  int64_t lda, int64_t ldb, int plain, int swiglu, int64_t workspace_bytes,
+                  int32_t* plan);
+
 /* fp16 shorthands: contiguous row-major, no transpose, no C. */
 int sph_gemm_f16(int64_t m, int64_t n, int64_t k, const void* a,
                  const void* b, void* d, sph_stream_t stream);

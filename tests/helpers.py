@@ -8,6 +8,7 @@ torch.Generator().manual_seed(0xAFFE + k), then cast.
 
 from __future__ import annotations
 
+import ctypes
 import json
 import os
 
@@ -49,3 +50,27 @@ def assert_close_fp(actual: torch.Tensor, expected_f32: np.ndarray, out_dtype=to
     act = actual.detach().to("cpu")
     torch.testing.assert_close(act.float(), exp.float(), rtol=rtol, atol=atol, equal_nan=True,
                                msg=lambda m: f"{what}: {m}")
+
+
+GEMM_KERNELS = {1: "stream", 2: "skinny", 3: "short-K", 4: "short-K ring", 5: "direct", 6: "ring",
+                7: "staged"}
+
+
+def gemm_plan(batch, m, n, k, tb, workspace=None, lda=None, ldb=None, plain=False, swiglu=False,
+              trans_a=False):
+    """(kernel, (tile rows, tile columns), K slices, padded operands) that the
+    library runs a product on (host only).  workspace None: the size that the
+    library names for the call."""
+    from torch_spyre import _capi
+
+    lib = _capi.lib()
+    lda = lda or (m if trans_a else k)
+    ldb = ldb or (k if tb else n)
+    if workspace is None:
+        workspace = (lib.sph_gemm_swiglu_workspace_bytes(m, n, k) if swiglu else
+                     lib.sph_gemm_workspace_bytes_ex(int(trans_a), int(tb), batch, m, n, k, lda, ldb))
+    out = (ctypes.c_int32 * 5)()
+    rc = lib.sph_gemm_plan(int(trans_a), int(tb), batch, m, n, k, lda, ldb, int(plain), int(swiglu),
+                           workspace, ctypes.addressof(out))
+    assert rc == 0, lib.sph_last_error()
+    return GEMM_KERNELS[out[0]], (out[1], out[2]), out[3], {0: "", 1: "A", 2: "B", 3: "AB"}[out[4]]

@@ -10,6 +10,8 @@ from torch_spyre import _capi
 
 from oracle import layout as L
 
+from helpers import gemm_plan
+
 
 def test_library_exports_every_declared_function():
     lib = _capi.lib()
@@ -92,3 +94,20 @@ def test_gemm_workspace_bytes_covers_each_layout():
                     assert both <= pad + max(8 * m * (n + 3) * 4, 256 * 256 * 256 * 4)
                     if batch > 1 and n % 8 == 0 and k % 8 == 0:
                         assert both == 0
+
+
+@pytest.mark.parametrize("batch,m,n,k,tb,want", [
+    # short K on the register-staged kernel where the ring kernel's epilogue or
+    # its 192 x 128 tiles cost more than its loads save
+    (10, 250, 1024, 32, 1, "staged"), (24, 552, 512, 128, 1, "staged"),
+    (4, 1608, 608, 224, 1, "staged"), (1, 2184, 5424, 32, 1, "staged"),
+    (16, 110, 744, 64, 1, "staged"), (10, 1571, 328, 128, 0, "staged"),
+    (16, 1152, 528, 64, 0, "staged"),
+    # the ring kernel elsewhere: one round of tiles, longer K, a transposing B
+    (4, 256, 2115, 384, 1, "ring"), (8, 1280, 146, 640, 1, "ring"),
+    (24, 128, 5671, 448, 1, "ring"), (64, 128, 4864, 96, 1, "ring"),
+    (8, 401, 463, 320, 0, "ring"), (1, 333, 6144, 4096, 1, "ring"), (10, 1571, 328, 2048, 0, "ring"),
+    # whole 256-row tiles of such a product stay on the direct-load kernel
+    (8, 512, 1280, 64, 0, "direct")])
+def test_gemm_plan_short_k(batch, m, n, k, tb, want):
+    assert gemm_plan(batch, m, n, k, tb)[0] == want

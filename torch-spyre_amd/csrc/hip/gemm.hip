@@ -3,7 +3,7 @@
 // of whole and ragged 256-row tiles (v_mfma_f32_16x16x32), the short-K kernels
 // (v_mfma_f32_32x32x16) and the C entry points.  gemm_ring.hip holds the
 // kernel of small and ragged row counts, gemm_small.hip the streaming kernels
-// of up to 16 rows, gemm_staged.hip the register-staged kernel that takes
+// of few rows, gemm_staged.hip the register-staged kernel that takes
 // every layout and alignment.
 #include <algorithm>
 #include <type_traits>
@@ -1174,38 +1174,97 @@ inline void launch_pack(const GemmArgs& p, const GemmArgs& q, int64_t batch, boo
   gemm_pack_kernel<<<grid, 256, 0, st>>>(oa, ob);
 }
 
-// Row-major B, short K and a ring plan of 128 x 128 tiles that gives a part of
-// the CUs a second workgroup: the plan costs ~10 us + 20 ns per K column there
-// (the time model has 6 + 16.5), the register-staged kernel's 128 x 128 tiles 8
-// + 26, so they lead up to K ~ 400 (32 x 300 x 400 fp16, register-staged beside
-// ring: K 256 14.7 / 15.6 us, 320 16.5 / 17.1, 384 18.2 / 18.5, 512 21.3 /
-// 20.8; 10 x 1571 x 328 x 128 11.2 / 13.1).  Not where that kernel would take
-// 256 x 256 tiles.
-constexpr int64_t kStagedShortK = 384;
-inline bool staged_leads(const GemmArgs& p, int64_t batch, bool b_kcont, const GemmRoute& r) {
-  return r.ring && r.rp.uneven && !b_kcont && p.k <= kStagedShortK &&
-         ceil_div(p.m, 256) * ceil_div(p.n, 256) * batch < kNumCUs;
+// Time of the register-staged kernel on aligned operands in the caches, K up to
+// ~1500 (us; fitted with the ring kernel's hot_us): per round of 512 tiles of 128
+// x 128, or of 256 x 256 tiles where those give every CU one, or one round of
+// 64 x 64 tiles.
+inline double staged_us(const GemmArgs& p, int64_t batch, bool b_kcont) {
+  const double k = static_cast<double>(p.k) * 1e-3;
+  const int64_t t256 = ceil_div(p.m, 256) * ceil_div(p.n, 256) * batch;
+  const int64_t t128 = ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
+  if (t256 >= kNumCUs) return static_cast<double>(ceil_div(t256, kNumCUs)) * (11.5 + 36.0 * k);
+  if (t128 >= 128) {
+    const double one = b_kcont ? 6.3 + 14.6 * k : 6.7 + 19.7 * k, two = b_kcont ? 7.3 + 19.0 * k : 7.4 + 25.6 * k;
+    const int64_t rest = t128 % (2 * kNumCUs);
+    return static_cast<double>(t128 / (2 * kNumCUs)) * two + (rest > kNumCUs ? two : rest > 0 ? one : 0.0);
+  }
+  if (ceil_div(p.m, 64) * ceil_div(p.n, 64) * batch <= kNumCUs) return b_kcont ? 3.6 + 7.2 * k : 4.2 + 14.4 * k;
+  return b_kcont ? 4.2 + 9.6 * k : 5.2 + 16.0 * k;
 }
 
-// Small row counts on the streaming kernels, short K on theirs, then the
-// direct-load and ring kernels; what neither takes (A transposed, K or rows
-// off 16-byte chunks) on the register-staged kernel: 256x256 tiles when they
-// give at least one tile per CU, else 128x128 (more workgroups for the 256
-// CUs), else 64x64 for small problems.
-template <typename T>
-int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont,
-                  hipStream_t st, bool packed = false) {
-  if (stream_fits(p, batch, a_kcont, b_kcont))
-    return launch_stream(__is_same(T, bf16_t), p, false, false, st);
+// Short K where the ring kernel's epilogue or tiles cost more than its loads
+// save (fp16, K-contiguous B, ring beside register-staged: 10 x 250 x 1024 x 32
+// 12.3 / 7.0 us, 24 x 552 x 512 x 128 13.3 / 11.3, 4 x 1608 x 608 x 224 16.5 /
+// 13.1; row-major 10 x 1571 x 328 x 128 13.1 / 11.2).  Past the K of both fits the
+// ring kernel is ahead (bmm of 250 to 500 tiles: K 1024 even, 2048 5 % ahead).
+constexpr int64_t kStagedMaxK = 1536;
+inline bool staged_leads(const GemmArgs& p, int64_t batch, bool b_kcont, const GemmRoute& r) {
+  return r.ring && r.rp.splits == 1 && p.k <= kStagedMaxK && staged_us(p, batch, b_kcont) < r.rp.hot_us;
+}
+
+// The kernel of a call: small row counts on the streaming kernels, short K on
+// theirs, then the direct-load and ring kernels; what neither takes (A
+// transposed, K or rows off 16-byte chunks) on the register-staged kernel:
+// 256x256 tiles when they give at least one tile per CU, else 128x128 (more
+// workgroups for the 256 CUs), else 64x64 for small problems.  With padded
+// copies, the kernel is that of the product on them.
+struct GemmChoice {
+  sph_gemm_kernel kernel = SPH_GEMM_STAGED;
+  PackPlan pack;
+  RingPlan ring;
+  DlChoice dl;
+};
+GemmChoice gemm_choice(const GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont, bool packed = false) {
+  GemmChoice c;
+  if (stream_fits(p, batch, a_kcont, b_kcont)) {
+    c.kernel = SPH_GEMM_STREAM;
+    return c;
+  }
   if (p.m <= kSmallRows && a_kcont && b_kcont && p.vec_a && p.vec_b && p.k > 0 && p.k % 8 == 0 &&
-      ceil_div(p.n, 2) < (1LL << 40))
-    return launch_skinny(__is_same(T, bf16_t), p, batch, false, st);
+      ceil_div(p.n, 2) < (1LL << 40)) {
+    c.kernel = SPH_GEMM_SKINNY;
+    return c;
+  }
   if (shortk_fits(p, a_kcont, b_kcont)) {
-    p.tiles_m = static_cast<int>(p.m / sk::BM);
-    p.tiles_n = static_cast<int>(p.n / sk::BN);
-    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n * batch;
-    if (tiles >= kShortkRingTiles && p.tiles_n >= 2) {
-      // persistent: one workgroup per CU over runs of at least two tiles
+    // persistent from two tiles per workgroup on: one workgroup per CU
+    const int64_t tiles = p.m / sk::BM * (p.n / sk::BN) * batch;
+    c.kernel = tiles >= kShortkRingTiles && p.n / sk::BN >= 2 ? SPH_GEMM_SHORT_K_RING : SPH_GEMM_SHORT_K;
+    return c;
+  }
+  const PackPlan pp = packed ? PackPlan{} : pack_plan(p, batch, a_kcont, b_kcont);
+  if (pp.use) {  // (aligned: packs nothing more)
+    c = gemm_choice(packed_args(p, batch, b_kcont, pp), batch, true, b_kcont, true);
+    c.pack = pp;
+    return c;
+  }
+  const GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
+  c.ring = r.rp;
+  c.dl = r.dc;
+  bool ring = r.ring;
+  if (!packed && staged_leads(p, batch, b_kcont, r)) {
+    ring = false;
+    if (p.m % dl::BM != 0 || p.n % 128 != 0) c.dl.kind = 0;  // whole tiles stay direct-load
+  }
+  c.kernel = ring ? SPH_GEMM_RING : c.dl.kind != 0 ? SPH_GEMM_DIRECT : SPH_GEMM_STAGED;
+  return c;
+}
+
+template <typename T>
+int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont, hipStream_t st) {
+  const GemmChoice c = gemm_choice(p, batch, a_kcont, b_kcont);
+  if (c.pack.use) {
+    GemmArgs q = packed_args(p, batch, b_kcont, c.pack);
+    launch_pack(p, q, batch, b_kcont, c.pack, st);
+    p = q;
+    a_kcont = true;
+  }
+  constexpr bool bf16 = __is_same(T, bf16_t);
+  switch (c.kernel) {
+    case SPH_GEMM_STREAM: return launch_stream(bf16, p, false, false, st);
+    case SPH_GEMM_SKINNY: return launch_skinny(bf16, p, batch, false, st);
+    case SPH_GEMM_SHORT_K_RING: {
+      p.tiles_m = static_cast<int>(p.m / sk::BM);
+      p.tiles_n = static_cast<int>(p.n / sk::BN);
       p.batches = batch;
       const dim3 grid(static_cast<unsigned>(kNumCUs));
       constexpr int RWM = 2, RWN = 2, RNT = skr::L<RWM, RWN>::NT;
@@ -1218,34 +1277,26 @@ int gemm_dispatch(GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont,
       }
       return check_launch("sph_gemm (short K)");
     }
-    dim3 grid(static_cast<unsigned>(p.tiles_m) * p.tiles_n, static_cast<unsigned>(batch));
-    if (p.k == 64) {
-      if (b_kcont) gemm_shortk_kernel<T, true, 1><<<grid, dim3(sk::NT), 0, st>>>(p);
-      else gemm_shortk_kernel<T, false, 1><<<grid, dim3(sk::NT), 0, st>>>(p);
-    } else {
-      if (b_kcont) gemm_shortk_kernel<T, true, 2><<<grid, dim3(sk::NT), 0, st>>>(p);
-      else gemm_shortk_kernel<T, false, 2><<<grid, dim3(sk::NT), 0, st>>>(p);
+    case SPH_GEMM_SHORT_K: {
+      p.tiles_m = static_cast<int>(p.m / sk::BM);
+      p.tiles_n = static_cast<int>(p.n / sk::BN);
+      dim3 grid(static_cast<unsigned>(p.tiles_m) * p.tiles_n, static_cast<unsigned>(batch));
+      if (p.k == 64) {
+        if (b_kcont) gemm_shortk_kernel<T, true, 1><<<grid, dim3(sk::NT), 0, st>>>(p);
+        else gemm_shortk_kernel<T, false, 1><<<grid, dim3(sk::NT), 0, st>>>(p);
+      } else {
+        if (b_kcont) gemm_shortk_kernel<T, true, 2><<<grid, dim3(sk::NT), 0, st>>>(p);
+        else gemm_shortk_kernel<T, false, 2><<<grid, dim3(sk::NT), 0, st>>>(p);
+      }
+      return check_launch("sph_gemm (short K)");
     }
-    return check_launch("sph_gemm (short K)");
+    case SPH_GEMM_RING: return launch_ring(bf16, p, batch, b_kcont, false, c.ring, st);
+    case SPH_GEMM_DIRECT:
+      if (c.dl.kind == 256) return launch_dl<T, 256>(p, batch, b_kcont, st, &c.dl.split);
+      if (c.dl.kind == 192) return launch_dl<T, 192, false, 48>(p, batch, b_kcont, st);
+      return launch_dl<T, 128, false, 32>(p, batch, b_kcont, st);
+    default: return launch_staged(bf16, p, batch, a_kcont, b_kcont, st);
   }
-  const PackPlan pp = pack_plan(p, batch, a_kcont, b_kcont);
-  if (pp.use) {
-    GemmArgs q = packed_args(p, batch, b_kcont, pp);
-    launch_pack(p, q, batch, b_kcont, pp, st);
-    return gemm_dispatch<T>(q, batch, true, b_kcont, st, true);  // (aligned: packs nothing)
-  }
-  GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
-  if (!packed && staged_leads(p, batch, b_kcont, r)) {
-    r.ring = false;
-    if (p.m % dl::BM != 0 || p.n % 128 != 0) r.dc.kind = 0;  // whole tiles stay direct-load
-  }
-  if (r.ring) return launch_ring(__is_same(T, bf16_t), p, batch, b_kcont, false, r.rp, st);
-  switch (r.dc.kind) {
-    case 256: return launch_dl<T, 256>(p, batch, b_kcont, st, &r.dc.split);
-    case 192: return launch_dl<T, 192, false, 48>(p, batch, b_kcont, st);
-    case 128: return launch_dl<T, 128, false, 32>(p, batch, b_kcont, st);
-  }
-  return launch_staged(__is_same(T, bf16_t), p, batch, a_kcont, b_kcont, st);
 }
 
 }  // namespace
@@ -1509,6 +1560,52 @@ extern "C" int sph_gemm_swiglu_any(sph_dtype dtype, int64_t m, int64_t n, int64_
     return swiglu_stream(dtype, m, n, k, a, lda, w, ldw, d, ldd, st);
   SPH_REQUIRE(k > 0 && k % 8 == 0, SPH_ERR_UNSUPPORTED, "gemm_swiglu: k must be a multiple of 8");
   return swiglu_run(dtype, m, n, k, a, lda, w, ldw, d, ldd, workspace, workspace_bytes, st);
+}
+
+extern "C" int sph_gemm_plan(int trans_a, int trans_b, int64_t batch, int64_t m, int64_t n,
+                             int64_t k, int64_t lda, int64_t ldb, int plain, int swiglu,
+                             int64_t workspace_bytes, int32_t* plan) {
+  SPH_REQUIRE(plan != nullptr && batch > 0 && m > 0 && n > 0 && k > 0 && workspace_bytes >= 0,
+              SPH_ERR_INVALID_ARG, "gemm_plan: sizes must be positive");
+  GemmArgs p{};
+  p.m = m;
+  p.n = p.nb = n;
+  p.k = k;
+  p.lda = lda;
+  p.ldb = ldb;
+  p.ldd = n;
+  p.stride_a = trans_a ? k * lda : m * lda;
+  p.stride_b = trans_b ? n * ldb : k * ldb;
+  p.vec_a = lda % 8 == 0 && (batch == 1 || p.stride_a % 8 == 0);
+  p.vec_b = ldb % 8 == 0 && (batch == 1 || p.stride_b % 8 == 0);
+  p.vec_d = n % 8 == 0;
+  p.alpha = plain ? 1.f : 0.5f;
+  p.part = workspace_bytes > 0 ? reinterpret_cast<float*>(uintptr_t{256}) : nullptr;  // (not read)
+  p.part_bytes = workspace_bytes;
+  GemmChoice c;
+  if (swiglu) {
+    SPH_REQUIRE(!trans_a && trans_b && batch == 1 && k % 8 == 0 && p.vec_a && p.vec_b,
+                SPH_ERR_UNSUPPORTED, "gemm_plan: not a SwiGLU product");
+    if (m <= 8 && k >= 64 && k <= 8192) {
+      c.kernel = SPH_GEMM_STREAM;
+    } else {
+      const SwigluRoute r = swiglu_route(p, workspace_bytes);
+      SPH_REQUIRE(r.ring || r.dl, SPH_ERR_TOO_LARGE, "gemm_plan: operands too large");
+      c.kernel = r.ring ? SPH_GEMM_RING : SPH_GEMM_DIRECT;
+      c.ring = r.rp;
+      c.dl.kind = 256;
+      c.dl.split = r.split;
+    }
+  } else {
+    c = gemm_choice(p, batch, !trans_a, trans_b != 0);
+  }
+  const bool ring = c.kernel == SPH_GEMM_RING, dl_ = c.kernel == SPH_GEMM_DIRECT;
+  plan[0] = c.kernel;
+  plan[1] = ring ? c.ring.bm : dl_ ? static_cast<int>(dl::BM) : 0;
+  plan[2] = ring ? c.ring.bn : dl_ ? c.dl.kind : 0;
+  plan[3] = ring ? c.ring.splits : dl_ ? c.dl.split.splits : 1;
+  plan[4] = (c.pack.a ? 1 : 0) + (c.pack.b ? 2 : 0);
+  return SPH_OK;
 }
 
 extern "C" int sph_gemm_rmsnorm(sph_dtype dtype, int64_t m, int64_t n, int64_t k, const void* a,

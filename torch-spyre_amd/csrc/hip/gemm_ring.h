@@ -7,11 +7,12 @@ namespace sph {
 
 struct RingPlan {
   int cfg = -1;        // tile configuration; -1: none fits
+  int bm = 0, bn = 0;  // its tile
   int splits = 1;      // K slices
   int kslice = 0;      // K tiles per slice
   int64_t bytes = 0;   // workspace of the partial sums (0: one slice)
   double us = 0;       // modelled time
-  bool uneven = false;  // 128 x 128 tiles, unsplit, a second workgroup on part of the CUs
+  double hot_us = 0;   // unsplit: time with operands in the caches (K up to ~1500)
 };
 
 // The fastest plan by the time model whose workspace is at most max_bytes.
