@@ -111,3 +111,15 @@ def test_gemm_workspace_bytes_covers_each_layout():
     (8, 512, 1280, 64, 0, "direct")])
 def test_gemm_plan_short_k(batch, m, n, k, tb, want):
     assert gemm_plan(batch, m, n, k, tb)[0] == want
+
+
+@pytest.mark.parametrize("batch,m,n,k,ws,want", [
+    # 9 to 16 rows, few columns, long K: the small-row kernel where the ring
+    # kernel has no K slices
+    (8, 15, 128, 4096, None, "skinny"), (2, 9, 256, 1024, None, "skinny"),
+    (16, 16, 128, 8192, None, "skinny"), (1, 12, 1024, 2048, 0, "skinny"),
+    (1, 12, 1024, 2048, None, "ring"), (16, 16, 128, 1024, None, "ring"),
+    (8, 17, 128, 4096, None, "ring"), (2, 16, 512, 512, None, "ring"),
+    (32, 12, 128, 4096, None, "ring"), (32, 12, 128, 8192, None, "skinny")])
+def test_gemm_plan_16_rows(batch, m, n, k, ws, want):
+    assert gemm_plan(batch, m, n, k, 1, workspace=ws)[0] == want

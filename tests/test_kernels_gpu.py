@@ -18,7 +18,7 @@ from torch_spyre import _capi
 from oracle import layout as L
 from oracle import ops as O
 
-from helpers import assert_close_fp, np32, randn, uniform
+from helpers import assert_close_fp, gemm_plan, np32, randn, uniform
 
 pytestmark = pytest.mark.gpu
 
@@ -658,6 +658,34 @@ def test_gemm_small_m_weight_layout(m, n, k, dtype):
     tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
     assert_close_fp(d, O.gemm(X.float().numpy(), W.float().numpy().T), out_dtype=dtype,
                     what=f"small-M {dtype}", **tol)
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(3, 9, 33, 1024), (2, 16, 129, 2056), (4, 13, 64, 4096),
+                                         (1, 16, 1001, 1544), (3, 11, 1027, 8200)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gemm_16_rows_long_k(batch, m, n, k, dtype):
+    # the small-row kernel at 9 to 16 rows: batches, odd columns, K tails, bias
+    # and activation
+    assert gemm_plan(batch, m, n, k, 1, workspace=0, lda=k + 8, ldb=k + 16)[0] == "skinny"
+    _log(f"gemm 16 rows {batch}x{m}x{n}x{k} {dtype}")
+    X = uniform((batch, m, k), k=13, dtype=dtype)
+    W = (uniform((batch, n, k), k=14) * 0.05).to(dtype)
+    bias = uniform((n,), k=15, dtype=dtype)
+    xd = torch.full((batch, m, k + 8), float("nan"), dtype=dtype, device=DEV)
+    xd[..., :k] = X.to(DEV)
+    wd = torch.full((batch, n, k + 16), float("nan"), dtype=dtype, device=DEV)
+    wd[..., :k] = W.to(DEV)
+    bd = bias.to(DEV)
+    d = torch.full((batch, m + 1, n), 7.0, dtype=dtype, device=DEV)
+    _capi.call("sph_gemm_ex", DT[dtype], 0, 1, batch, m, n, k, 0.75, _p(xd), k + 8, m * (k + 8),
+               _p(wd), k + 16, n * (k + 16), 0.5, _p(bd), 0, 1, 0, _p(d), n, (m + 1) * n, 3, None, 0,
+               _stream())
+    _sync()
+    want = O.gemm(X.float().numpy(), np.swapaxes(W.float().numpy(), 1, 2), alpha=0.75, beta=0.5,
+                  c=bias.float().numpy()[None, None, :], epilogue="silu")
+    tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    assert_close_fp(d[:, :m], want, out_dtype=dtype, what=f"16 rows {dtype}", **tol)
+    assert bool((d[:, m] == 7.0).all()), "rows past M written"
 
 
 @pytest.mark.parametrize("m,n,k", [(4, 25600, 4096), (4, 49155, 4096), (5, 16400, 2056),

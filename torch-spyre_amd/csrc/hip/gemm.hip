@@ -1202,6 +1202,18 @@ inline bool staged_leads(const GemmArgs& p, int64_t batch, bool b_kcont, const G
   return r.ring && r.rp.splits == 1 && p.k <= kStagedMaxK && staged_us(p, batch, b_kcont) < r.rp.hot_us;
 }
 
+// 9 to 16 rows times few columns with a long K that the ring kernel does not
+// split (a batch, or no workspace): its tiles leave most CUs idle and each walks
+// all of K, which the small-row kernel spreads over a workgroup per two columns.
+// Ring beside small-row kernel, us: columns (of the whole batch) 512 x K 1024 7.3
+// / 6.6, 2048 x 1024 7.4 / 9.0; 1024 x 2048 11.6 / 8.5, 2048 x 2048 11.7 / 13.7;
+// 2048 x 4096 20.7 / 17, 4096 x 4096 20.8 / 24.5; 512 x 8192 38 / 10.2, 2048 x
+// 8192 38 / 28, 4096 x 8192 38 / 31.
+inline bool skinny16_leads(const GemmArgs& p, int64_t batch, bool a_kcont, bool b_kcont, const GemmRoute& r) {
+  return p.m <= 16 && a_kcont && b_kcont && r.ring && r.rp.splits == 1 && p.k >= 1024 &&
+         p.n * batch <= std::clamp<int64_t>(p.k / 2, 1024, 4096);
+}
+
 // The kernel of a call: small row counts on the streaming kernels, short K on
 // theirs, then the direct-load and ring kernels; what neither takes (A
 // transposed, K or rows off 16-byte chunks) on the register-staged kernel:
@@ -1238,6 +1250,10 @@ GemmChoice gemm_choice(const GemmArgs& p, int64_t batch, bool a_kcont, bool b_kc
     return c;
   }
   const GemmRoute r = gemm_route(p, batch, a_kcont, b_kcont);
+  if (skinny16_leads(p, batch, a_kcont, b_kcont, r)) {
+    c.kernel = SPH_GEMM_SKINNY;
+    return c;
+  }
   c.ring = r.rp;
   c.dl = r.dc;
   bool ring = r.ring;

@@ -3,7 +3,8 @@
 // are HBM-bound on reading W once and run as streams of packed dot products,
 // which keep every CU on its own rows of W, with an RMSNorm prologue and a
 // SwiGLU epilogue.  (From 9 rows on the MFMA ring kernel is ahead: 16 x 6144 x
-// 4096 32.9 us here, 16.8 there; 8 x 6144 x 4096 17.2 here.)
+// 4096 32.9 us here, 16.8 there; 8 x 6144 x 4096 17.2 here.  Up to 16 rows run
+// here where that kernel cannot split a long K over the CUs and has few tiles.)
 #include <algorithm>
 
 #include "gemm_route.h"
@@ -252,8 +253,16 @@ void skinny_t(const GemmArgs& p, int64_t batch, hipStream_t st) {
     launch_skinny_m<T, 1, NORM>(p, batch, st);
   else if (p.m <= 4)
     launch_skinny_m<T, 4, NORM>(p, batch, st);
-  else
+  else if (NORM || p.m <= 8)
     launch_skinny_m<T, 8, NORM>(p, batch, st);
+  else if constexpr (!NORM) {  // (skinny16_leads: few columns, long rows)
+    if (p.n * batch > 2048)  // (K >= 4096: 8 x 10 x 512 x 8192 31 us, 42 in two columns)
+      launch_skinny_cfg<T, 16, 4, 128>(p, batch, st);
+    else if (p.k >= 2048)
+      launch_skinny_cfg<T, 16, 2, 256>(p, batch, st);
+    else
+      launch_skinny_cfg<T, 16, 2, 128>(p, batch, st);
+  }
 }
 
 // ---------------------------------------------------------------------------
