@@ -189,6 +189,28 @@ def test_nonpositive_or_infinite_scales_stay_unfused(form):
     torch.testing.assert_close(out, ref, rtol=1e-2, atol=1e-2, equal_nan=True)
 
 
+@pytest.mark.parametrize("b,mq,sk,masked,fused", [
+    (24, 3108, 777, True, True), (8, 4 * 100, 100, True, True), (8, 17, 512, False, True),
+    (16, 300, 2048, False, True), (64, 700, 4096, True, True), (8, 3001, 3001, True, True),
+    # few rows against many keys: the chain's products fill the chip
+    (1, 17, 4096, False, False), (8, 68, 4096, True, False), (1, 1000, 4096, False, False),
+    (8, 300, 8192, True, False), (4, 200, 4096, False, False),
+    (2, 17, 64, False, False)])  # too small to matter
+def test_ragged_rows_rule(b, mq, sk, masked, fused):
+    import importlib
+
+    # (the package exports the pass function under the module's name)
+    mod = importlib.import_module("torch_spyre._inductor.passes.fuse_attention")
+    assert mod._ragged_leads(b, mq, sk, masked) == fused
+
+
+def test_few_ragged_rows_with_many_keys_stay_the_chain():
+    q, k, v = _qkv(2, 20, 2048, seed=7)
+    out, n = _run(lambda q, k, v: _chain(q, k, v), q, k, v)
+    assert n == 0
+    torch.testing.assert_close(out, _chain(q, k, v), rtol=2e-3, atol=2e-3)
+
+
 @pytest.mark.parametrize("mq,sk", [(300, 130), (4 * 77, 77)])
 def test_ragged_rows_fuse(mq, sk):
     # row counts off the 128-row block, from 2^16 scores on

@@ -6,8 +6,8 @@ separate ops (spyre__bmm_default, codegen/inputs/spyre_torch_ops.cpp:297-377;
 add and _softmax, codegen/inputs/Metadata.yaml:275-277) and forbids fusion
 in its scheduler (torch_spyre/_inductor/choices.py:58-83).  Here the chain
 is replaced, on spyre graphs only, when the fused kernel takes its shapes:
-fp16 / bf16, head dim 128, query rows a multiple of 128 (or, from 2^16
-scores on, any number above 16: `torch.ops.spyre.attention_rows`), and a
+fp16 / bf16, head dim 128, query rows a multiple of 128 (or any number above
+16 where the fused kernel is ahead: `torch.ops.spyre.attention_rows`), and a
 mask (if any) of the same dtype shaped [mq, sk] or [B or 1, mq, sk], or one mask row
 [sk] / [1, sk] broadcast over the rows (expanded to [mq, sk] as a view).  The fused op
 computes the same function (fp32 scores and softmax, probabilities rounded
@@ -42,6 +42,22 @@ ROW_BLOCK = 128
 # Ragged row counts: below this many scores the chain's products and softmax
 # are one small launch each, which a last, mostly empty row block does not beat.
 RAGGED_SCORES = 1 << 16
+CUS = 256
+
+
+def _ragged_leads(B: int, mq: int, sk: int, masked: bool) -> bool:
+    """Whether the fused kernel is ahead of the chain at a row count off the
+    block.  A workgroup of 128 rows walks every key block (1.2 us for 64 keys
+    while workgroups do not share a CU), so few rows against many keys leave
+    most of the chip idle, where the chain's products spread over it: 1 x 1000
+    rows x 4096 keys 79 us fused, 31 as the chain (two products, softmax); 8 x 68
+    x 4096 78 / 42; 8 x 700 x 4096 80 / 82; 16 x 300 x 2048 43 / 48; 8 x 2500 x
+    625 21 / 71.  The chain: launches, 8 bytes of HBM traffic per score, and the
+    second product's walk over the keys, split over CUs for a single batch
+    entry only."""
+    fused = (9 if masked else 3) + 1.17 * (-(-sk // 64)) * max(1.0, B * -(-mq // ROW_BLOCK) / CUS)
+    chain = 14 + 2.1e-6 * B * mq * sk + sk * (4.4e-3 if B > 1 else 1.5e-3)
+    return B * mq * sk >= RAGGED_SCORES and fused < chain
 
 
 def _val(n):
@@ -184,7 +200,7 @@ def _finish(bmm2, bmm1, chain, v, mask, scale) -> Optional[tuple]:
     # the c5 decode step (4.77 against 4.65 ms per step).
     if d != HEAD_DIM or tuple(kv.shape) != (B, sk, d) or tuple(vv.shape) != (B, sk, d):
         return None
-    if mq % ROW_BLOCK and (mq <= 16 or B * mq * sk < RAGGED_SCORES):
+    if mq % ROW_BLOCK and (mq <= 16 or not _ragged_leads(B, mq, sk, mask is not None)):
         return None
     expand = None
     if mask is not None:
