@@ -375,7 +375,7 @@ int64_t sph_attention_decode_workspace_bytes(int64_t batch, int64_t mq, int64_t 
  * 1, 16-byte aligned rows); V cache key-major (v_dim_stride 1, 16-byte
  * aligned rows) or dim-major (v_key_stride 1, rows of any length).
  * dtype F16 / BF16; fp32 scores and sums; n_heads / n_kv_heads <= 8;
- * batch * n_kv_heads <= 4096.  workspace: at least
+ * batch * n_kv_heads <= 4096, and times ceil(max_len / 64) below 2^24.  workspace: at least
  * sph_decode_attention_step_workspace_bytes(...) bytes for the per-chunk
  * partials.  A P outside [0, max_len) writes nothing and sets *error_word
  * (device-visible int32, may be NULL) to 2.  Two launches on `stream`:

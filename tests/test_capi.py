@@ -123,3 +123,17 @@ def test_gemm_plan_short_k(batch, m, n, k, tb, want):
     (32, 12, 128, 4096, None, "ring"), (32, 12, 128, 8192, None, "skinny")])
 def test_gemm_plan_16_rows(batch, m, n, k, ws, want):
     assert gemm_plan(batch, m, n, k, 1, workspace=ws)[0] == want
+
+
+@pytest.mark.parametrize("batch,max_len,rc", [
+    (512, (1 << 30) - 1, 1003),   # 2^24 chunks of 64 positions x 4096 units: past the grid
+    (512, 64 * 4096, 1003),       # exactly 2^24 workgroups
+    (512, 64 * 4096 - 64, 1001)])  # the largest grid: refused for its workspace only
+def test_decode_step_grid_limit(batch, max_len, rc):
+    # refused before any launch (the pointers below are never read)
+    a = 4096
+    got = _capi.lib().sph_decode_attention_step(
+        _capi.F16, batch, 8, 8, 128, a, 24 * 128, a, a, 128, a, None, a, 8 * max_len * 128,
+        max_len * 128, 128, a, 8 * max_len * 128, max_len * 128, 128, 1, max_len,
+        ctypes.c_float(0.1), a, 8 * 128, a, 1 << 62 if rc != 1001 else 16, None)
+    assert got == rc

@@ -445,7 +445,7 @@ struct StepArgs {
   int64_t k_sb, k_sh, k_ss;
   void* vc;
   int64_t v_sb, v_sh, v_ks, v_ds;
-  int wait_pos;  // read the position before the chunk (grids past one residency)
+  int wait_pos;  // read the position before the chunk (more than kSpeculateWGs)
   int64_t max_len;
   int n_heads, n_kv, g, nchunks;
   float scale_log2;
@@ -459,9 +459,9 @@ __device__ inline u32x4 zero_chunk() {
   return z;
 }
 
-// One workgroup of 4 waves: one unit and one chunk of 64 keys.  While the grid
-// fits the chip the chunk is loaded before P is known; larger grids (batches
-// from ~8 up) read P first, other workgroups covering that wait, and skip the
+// One workgroup of 4 waves: one unit and one chunk of 64 keys.  Up to
+// kSpeculateWGs workgroups the chunk is loaded before P is known; larger grids
+// (batches from ~8 up) read P first, other workgroups covering that wait, and skip the
 // chunks past it.  The chunks of a unit run on one XCD: with a dim-major V
 // whose rows are off 128 bytes, neighbouring chunks share V's cache lines.
 // Scores on the matrix cores (the queries and keys are 16-bit, the sums
@@ -819,6 +819,10 @@ extern "C" int sph_decode_attention_step(
               "decode attention step: query heads per KV head must divide and be <= 8");
   SPH_REQUIRE(batch * n_kv_heads <= kMaxUnits && max_len < (1LL << 30), SPH_ERR_TOO_LARGE,
               "decode attention step: at most 4096 (batch x KV heads) and 2^30 positions");
+  // one workgroup of 256 threads per unit and chunk in one grid dimension, which
+  // holds 2^32 threads
+  SPH_REQUIRE((max_len + SKC - 1) / SKC * batch * n_kv_heads < (1LL << 24), SPH_ERR_TOO_LARGE,
+              "decode attention step: at most 2^24 chunks of 64 positions over the batch's KV heads");
   SPH_REQUIRE(scale > 0.f && scale < INFINITY, SPH_ERR_INVALID_ARG,
               "decode attention step: scale must be positive and finite");
   SPH_REQUIRE(pos != nullptr && qkv != nullptr && k_cache != nullptr && v_cache != nullptr &&
