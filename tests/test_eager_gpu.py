@@ -556,3 +556,37 @@ def test_single_row_projections_take_any_row_stride(swiglu):
         wide = torch.ops.spyre.swiglu_mm(x.expand(20, K), w).cpu()
         torch.testing.assert_close(wide.float(), a.cpu().expand(20, n).float(), rtol=1e-2,
                                    atol=1e-2)
+
+
+def test_products_run_without_room_for_their_workspace():
+    """Padded copies and K slices are optional: with the device full, products
+    run without them."""
+    from torch_spyre import _C
+
+    a, b = (uniform(s, k=i).to(DEV) for i, s in enumerate(((1501, 2003), (2003, 999))))
+    x, w = (uniform(s, k=i).to(DEV) for i, s in enumerate(((24, 4096), (4096, 4096)), 2))
+    p, q = (uniform(s, k=i).to(DEV) for i, s in enumerate(((3, 130, 1201), (3, 1201, 777)), 4))
+    u, g = (uniform(s, k=i).to(DEV) for i, s in enumerate(((24, 4096), (2048, 4096)), 6))
+    outs = [torch.empty(s, dtype=torch.float16).to(DEV)
+            for s in ((1501, 999), (24, 4096), (3, 130, 777))]
+    run = lambda: (torch.mm(a, b, out=outs[0]), torch.mm(x, w.t(), out=outs[1]),  # noqa: E731
+                   torch.bmm(p, q, out=outs[2]))
+    want = [t.cpu().float() for t in run()]
+    swi = torch.ops.spyre.swiglu_mm(u, g)  # (its output's block stays in the cache)
+    want_swi = swi.cpu().float()
+    del swi
+    torch.spyre.synchronize()
+    torch.spyre.empty_cache()
+    room = torch.empty(24, 1024, dtype=torch.float16).to(DEV)  # a block for swiglu's output
+    _C._set_memory_limit(0)
+    try:
+        with pytest.raises(RuntimeError, match="out of device memory"):
+            torch.empty(1 << 20, dtype=torch.float16, device=DEV)
+        got = [t.cpu().float() for t in run()]
+        del room
+        got_swi = torch.ops.spyre.swiglu_mm(u, g).cpu().float()
+    finally:
+        _C._set_memory_limit(-1)
+    for g_, w_ in zip(got + [got_swi], want + [want_swi]):
+        # the same sums in another order: a rounding step of the result
+        torch.testing.assert_close(g_, w_, rtol=2e-3, atol=2e-3 * w_.abs().max().item())

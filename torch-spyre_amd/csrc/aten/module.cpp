@@ -120,6 +120,7 @@ PYBIND11_MODULE(_C, m) {
     return r;
   }, py::arg("device") = -1);
   m.def("empty_cache", &spyre::empty_cache);
+  m.def("_set_memory_limit", &spyre::set_memory_limit);
   m.def("stick_alloc_nbytes", [](std::vector<int64_t> sizes, int64_t elem_bytes) {
     return spyre::stick_alloc_nbytes(sizes, elem_bytes);
   });

@@ -93,7 +93,7 @@ void gemm2d(const at::Tensor& a, const at::Tensor& b, const at::Tensor& d, float
   // workspace for K slices' partial sums, or for padded copies of operands
   // off 16-byte chunks, when the shape has either
   const int64_t nws = sph_gemm_workspace_bytes_ex(va.trans, vb.trans, 1, m, n, k, va.ld, vb.ld);
-  at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
+  const at::Tensor ws = optional_workspace(nws, d.device());
   SPYRE_SPH_CHECK(sph_gemm_ex(to_sph(d.scalar_type()), va.trans, vb.trans, 1, m, n, k, alpha,
                               va.ptr, va.ld, 0, vb.ptr, vb.ld, 0, cp ? beta : 0.f, cp, ldc_r,
                               ldc_c, 0, dd.data_ptr(), m == 1 ? n : dd.stride(0), 0,
@@ -145,7 +145,7 @@ void gemm3d(const at::Tensor& a_in, const at::Tensor& b_in, const at::Tensor& d,
   c10::DeviceGuard guard(d.device());
   // workspace for padded copies of operands off 16-byte chunks
   const int64_t nws = sph_gemm_workspace_bytes_ex(va.trans, vb.trans, bs, m, n, k, va.ld, vb.ld);
-  at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, d.device()) : at::Tensor();
+  const at::Tensor ws = optional_workspace(nws, d.device());
   SPYRE_SPH_CHECK(sph_gemm_ex(
       to_sph(d.scalar_type()), va.trans, vb.trans, bs, m, n, k, alpha, va.ptr, va.ld, sa, vb.ptr,
       vb.ld, sb, cp ? beta : 0.f, cp, ldc_r, ldc_c, sc, dd.data_ptr(), n, m * n, SPH_EPI_NONE,
@@ -224,7 +224,7 @@ at::Tensor gemm_swiglu(const at::Tensor& x_in, const at::Tensor& w_in) {
     check_matrix_extent(x, x.data_ptr(), m, k, ldx, 0, 1, 0, "swiglu_mm x");
     check_matrix_extent(w, w.data_ptr(), 2 * n, k, ldw, 0, 1, 0, "swiglu_mm w");
     const int64_t nws = sph_gemm_swiglu_workspace_bytes(m, n, k);
-    at::Tensor ws = nws > 0 ? empty_spyre({nws}, at::kByte, out.device()) : at::Tensor();
+    const at::Tensor ws = optional_workspace(nws, out.device());
     const int rc = sph_gemm_swiglu_any(to_sph(out.scalar_type()), m, n, k, x.data_ptr(), ldx,
                                    w.data_ptr(), ldw, out.data_ptr(), n,
                                    ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? nws : 0,

@@ -67,6 +67,15 @@ at::Tensor empty_spyre(at::IntArrayRef sizes, at::ScalarType dtype, c10::Device 
   return make_tensor(sizes, c10::contiguous_strides(sizes), dtype, device);
 }
 
+at::Tensor optional_workspace(int64_t nbytes, c10::Device device) {
+  if (nbytes <= 0) return at::Tensor();
+  try {
+    return empty_spyre({nbytes}, at::kByte, device);
+  } catch (const c10::OutOfMemoryError&) {
+    return at::Tensor();
+  }
+}
+
 at::Tensor spyre_empty_strided(c10::IntArrayRef size, c10::IntArrayRef stride,
                                std::optional<c10::ScalarType> dtype_opt,
                                std::optional<c10::Layout> layout_opt,

@@ -45,4 +45,8 @@ void check_matrix_extent(const at::Tensor& t, const void* ptr, int64_t rows, int
 // Allocates an uninitialised spyre tensor (contiguous).
 at::Tensor empty_spyre(at::IntArrayRef sizes, at::ScalarType dtype, c10::Device device);
 
+// `nbytes` of workspace for a kernel that also runs without one: undefined for
+// 0 bytes and when the device has no room for them.
+at::Tensor optional_workspace(int64_t nbytes, c10::Device device);
+
 }  // namespace spyre

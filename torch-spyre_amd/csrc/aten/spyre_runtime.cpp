@@ -308,6 +308,11 @@ class CachingAllocator final : public c10::Allocator {
     return stats_[dev];
   }
 
+  void set_limit(int64_t bytes) {
+    std::lock_guard<std::mutex> lk(mu_);
+    limit_ = bytes;
+  }
+
   void empty_cache() {
     synchronize(-1);
     std::lock_guard<std::mutex> lk(mu_);
@@ -363,18 +368,27 @@ class CachingAllocator final : public c10::Allocator {
     return (n + kLarge - 1) / kLarge * kLarge;
   }
 
+  hipError_t device_malloc(void** p, size_t size, int dev) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (limit_ >= 0 && stats_[dev].reserved + static_cast<int64_t>(size) > limit_)
+        return hipErrorOutOfMemory;
+    }
+    return hipMalloc(p, size);
+  }
+
   Block* fresh_block(int dev, size_t size, int64_t pool_id) {
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, size);
+    hipError_t e = device_malloc(&p, size, dev);
     if (e == hipErrorOutOfMemory) {
       (void)hipGetLastError();
       empty_cache();
-      e = hipMalloc(&p, size);
+      e = device_malloc(&p, size, dev);
     }
     if (e != hipSuccess) {
       (void)hipGetLastError();
       MemoryStats st = stats(dev);
-      TORCH_CHECK(false, "spyre: out of device memory allocating ", size, " bytes on spyre:",
+      TORCH_CHECK_WITH(OutOfMemoryError, false, "spyre: out of device memory allocating ", size, " bytes on spyre:",
                   dev, " (allocated ", st.allocated, ", reserved ", st.reserved, "): ",
                   hipGetErrorString(e));
     }
@@ -406,6 +420,7 @@ class CachingAllocator final : public c10::Allocator {
   std::unordered_map<int64_t, std::multimap<size_t, Block*>> private_free_;
   std::unordered_set<int64_t> live_pools_;
   int64_t next_pool_ = 0;
+  int64_t limit_ = -1;  // reserved bytes per device past which allocations fail; -1: none
 };
 
 // Pinned host memory for copy staging (hipHostMalloc, never hipHostRegister).
@@ -466,6 +481,7 @@ MemoryStats memory_stats(int device) {
 }
 
 void empty_cache() { CachingAllocator::instance().empty_cache(); }
+void set_memory_limit(int64_t bytes) { CachingAllocator::instance().set_limit(bytes); }
 
 // ---------------------------------------------------------------------------
 // HIP graphs of the spyre stream

@@ -98,6 +98,9 @@ struct MemoryStats {
 };
 MemoryStats memory_stats(int device);
 void empty_cache();
+// Device memory (bytes per device, -1: none) past which allocations fail as
+// they do when the device is full.
+void set_memory_limit(int64_t bytes);
 
 // A HIP graph captured from the spyre stream of the current device.
 // Allocations made during the capture come from a private pool that stays
