@@ -264,7 +264,7 @@ int64_t sph_gemm_workspace_bytes_ex(int trans_a, int trans_b, int64_t batch, int
 /* What a product of these sizes runs on, without launching it (host only):
  * plan[0] the kernel, [1] and [2] its tile (direct-load and ring kernels, else
  * 0), [3] the K slices of its tiles, [4] which operands are copied into padded
- * rows first (1: A, 2: B).  Operands and D with 16-byte aligned bases, batches
+ * rows first (1: A, 2: B), [5] the ring kernel's configuration (else -1).  Operands and D with 16-byte aligned bases, batches
  * and D without gaps; plain: alpha 1, no C, no activation; swiglu: the product
  * of sph_gemm_swiglu_any. */
 typedef enum sph_gemm_kernel {

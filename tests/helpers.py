@@ -58,8 +58,8 @@ GEMM_KERNELS = {1: "stream", 2: "skinny", 3: "short-K", 4: "short-K ring", 5: "d
 
 def gemm_plan(batch, m, n, k, tb, workspace=None, lda=None, ldb=None, plain=False, swiglu=False,
               trans_a=False):
-    """(kernel, (tile rows, tile columns), K slices, padded operands) that the
-    library runs a product on (host only).  workspace None: the size that the
+    """(kernel, (tile rows, tile columns), K slices, padded operands, ring
+    configuration) that the library runs a product on (host only).  workspace None: the size that the
     library names for the call."""
     from torch_spyre import _capi
 
@@ -69,8 +69,9 @@ def gemm_plan(batch, m, n, k, tb, workspace=None, lda=None, ldb=None, plain=Fals
     if workspace is None:
         workspace = (lib.sph_gemm_swiglu_workspace_bytes(m, n, k) if swiglu else
                      lib.sph_gemm_workspace_bytes_ex(int(trans_a), int(tb), batch, m, n, k, lda, ldb))
-    out = (ctypes.c_int32 * 5)()
+    out = (ctypes.c_int32 * 6)()
     rc = lib.sph_gemm_plan(int(trans_a), int(tb), batch, m, n, k, lda, ldb, int(plain), int(swiglu),
                            workspace, ctypes.addressof(out))
     assert rc == 0, lib.sph_last_error()
-    return GEMM_KERNELS[out[0]], (out[1], out[2]), out[3], {0: "", 1: "A", 2: "B", 3: "AB"}[out[4]]
+    return (GEMM_KERNELS[out[0]], (out[1], out[2]), out[3], {0: "", 1: "A", 2: "B", 3: "AB"}[out[4]],
+            out[5])

@@ -77,21 +77,33 @@ def test_gemm_workspace_bytes(batch, m, n, k, split):
 
 
 def test_gemm_workspace_bytes_covers_each_layout():
-    # the per-call size never exceeds the size for both layouts of contiguous
-    # operands, is 0 for a transposed A, and stays within the padded copies and
-    # eight slices of partial sums (+ one 256 x 256 tile per CU of a split tail)
+    # the size without a layout covers the calls of either, leading dimensions of
+    # whole 16-byte chunks need no copies, a transposed A takes neither copies
+    # nor slices, and the size is what the plan of the call uses: the padded
+    # copies and at most eight slices of partial sums (or one 256 x 256 tile per
+    # CU of a split tail)
     lib = _capi.lib()
     for batch in (1, 3):
         for m in (1, 8, 9, 33, 255, 300, 2100):
             for n in (64, 65, 504, 4097):
                 for k in (8, 63, 520, 1029, 4096):
                     both = lib.sph_gemm_workspace_bytes(batch, m, n, k)
-                    one = [lib.sph_gemm_workspace_bytes_ex(0, tb, batch, m, n, k, k, k if tb else n)
-                           for tb in (0, 1)]
-                    assert max(one) == both and min(one) >= 0
+                    for tb in (0, 1):
+                        ldb = k if tb else n
+                        one = lib.sph_gemm_workspace_bytes_ex(0, tb, batch, m, n, k, k, ldb)
+                        _, tile, slices, packed, _ = gemm_plan(batch, m, n, k, tb)
+                        assert 0 <= one <= both
+                        assert (one > 0) == (slices > 1 or packed != "")
+                        pads = 2 * (k + 64) * ((m if "A" in packed else 0) + (n + 8 if "B" in packed else 0))
+                        # (few padded rows: sized for slices, run on a small-row kernel)
+                        parts = (max(8 * m * (n + 3) * 4, 256 ** 3 * 4) if slices > 1 else
+                                 8 * m * (n + 3) * 4 if m <= 16 else 0)
+                        assert one <= batch * pads + 512 + parts
+                        # less than that: the call runs without slices or copies
+                        if one > 0:
+                            _, _, fewer, unpacked, _ = gemm_plan(batch, m, n, k, tb, workspace=0)
+                            assert fewer == 1 and unpacked == ""
                     assert lib.sph_gemm_workspace_bytes_ex(1, 0, batch, m, n, k, m, n) == 0
-                    pad = 2 * batch * (m + n + 8) * (k + 64) + 512
-                    assert both <= pad + max(8 * m * (n + 3) * 4, 256 * 256 * 256 * 4)
                     if batch > 1 and n % 8 == 0 and k % 8 == 0:
                         assert both == 0
 

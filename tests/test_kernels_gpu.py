@@ -429,11 +429,12 @@ def test_gemm_bias_alpha_beta_epilogue(epi, name):
                                           (4096, 4096, 4096, False, 0)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_gemm_whole_tile_direct_load(m, n, k, tb, pad, dtype):
-    # whole 256-row tiles with K-contiguous A run the direct-to-LDS kernel,
-    # 256 or 128 columns wide (n = 384, 128, 640 only fit 128; 2048 x 4096
-    # picks 128 for a full round of tiles): odd and even K-tile counts (k/64 =
-    # 1, 2, 3, 5, 8, 19, 64, 200), row-major and K-contiguous B, leading
-    # dimensions wider than the matrix (pad); c2's 4096^3 through the C-ABI
+    # whole 256-row tiles with K-contiguous A, the direct-to-LDS kernel's
+    # shapes: the large ones run it, the small ones the ring kernel, which the
+    # time model puts ahead there (the same products through it in
+    # test_gemm_ragged_rows and test_gemm_128_wide_tiles).  Odd and even K-tile counts (k/64 = 1, 2, 3, 5, 8, 19, 64, 200),
+    # row-major and K-contiguous B, leading dimensions wider than the matrix
+    # (pad); c2's 4096^3 through the C-ABI
     _log(f"gemm direct-load {m}x{n}x{k} tb={tb} pad={pad} {dtype}")
     A = uniform((m, k), k=21, dtype=dtype)
     B = uniform((k, n), k=22, dtype=dtype)
@@ -515,7 +516,7 @@ def test_gemm_whole_tile_epilogue_and_batch(tb):
 
 @pytest.mark.parametrize("batch,m,n,k,pad,epi,dtype", [
     (1, 2048, 6144, 4096, 0, 0, torch.float16),     # c4 QKV: 256 tiles of 256 x 192
-    (1, 4096, 6144, 512, 8, 2, torch.float16),      # 512 tiles, padded rows, GELU
+    (1, 4096, 6144, 320, 8, 2, torch.float16),      # 512 tiles, padded rows, GELU
     (1, 2048, 6144, 1216, 0, 3, torch.bfloat16),    # bf16, SiLU, 19 K tiles
     (2, 1024, 6144, 256, 0, 0, torch.float16)])     # batched: 2 x 128 tiles
 def test_gemm_192_wide_tiles(batch, m, n, k, pad, epi, dtype):
@@ -524,6 +525,7 @@ def test_gemm_192_wide_tiles(batch, m, n, k, pad, epi, dtype):
     # 48): alpha, beta * C (a bias row), activation; with and without a
     # workspace (the 192-wide tiles take precedence over a split-K tail)
     _log(f"gemm 192-wide {batch}x{m}x{n}x{k} pad={pad} epi={epi} {dtype}")
+    assert gemm_plan(batch, m, n, k, 1, lda=k + pad, ldb=k + pad)[:2] == ("direct", (256, 192))
     A = uniform((batch, m, k), k=31, dtype=dtype)
     W = (uniform((batch, n, k), k=32, dtype=dtype).float() * 0.05).to(dtype)
     bias = uniform((n,), k=33, dtype=dtype)
@@ -554,14 +556,16 @@ def test_gemm_192_wide_tiles(batch, m, n, k, pad, epi, dtype):
 @pytest.mark.parametrize("batch,m,n,k,tb,pad,epi,dtype", [
     (1, 2048, 4096, 4096, 1, 0, 0, torch.float16),   # c4 O (no workspace): 256 tiles of 256 x 128
     (1, 2048, 4096, 4096, 0, 0, 3, torch.bfloat16),  # row-major B, bf16, SiLU
-    (2, 1024, 2048, 1024, 1, 8, 2, torch.float16),   # batched, padded rows, GELU
-    (3, 512, 1024, 512, 0, 8, 3, torch.bfloat16),    # batched row-major B, bf16
-    (1, 512, 384, 192, 0, 0, 0, torch.float16)])     # N % 256 != 0: 6 tiles, 3 K tiles
+    (4, 1024, 2048, 1024, 1, 8, 2, torch.float16),   # batched, padded rows, GELU
+    (3, 768, 1152, 64, 1, 8, 3, torch.bfloat16),     # batched, one K tile, bf16
+    (1, 768, 1408, 64, 0, 8, 0, torch.float16)])     # N % 256 != 0, row-major B, one K tile
 def test_gemm_128_wide_tiles(batch, m, n, k, tb, pad, epi, dtype):
     # shapes whose 256-wide tiles leave most CUs idle and that have no
     # split-K workspace run 256 x 128 tiles (8 waves of 128 x 32): alpha,
     # beta * C (a bias row), activation
     _log(f"gemm 128-wide {batch}x{m}x{n}x{k} tb={tb} pad={pad} epi={epi} {dtype}")
+    assert gemm_plan(batch, m, n, k, tb, workspace=0, lda=k + pad,
+                     ldb=(k if tb else n) + pad)[:2] == ("direct", (256, 128))
     A = uniform((batch, m, k), k=34, dtype=dtype)
     ld_b = (k if tb else n) + pad
     W = (uniform((batch, n, k) if tb else (batch, k, n), k=35, dtype=dtype).float() * 0.05).to(dtype)
@@ -584,20 +588,28 @@ def test_gemm_128_wide_tiles(batch, m, n, k, tb, pad, epi, dtype):
     assert_close_fp(d, want, out_dtype=dtype, what="128-wide gemm", **tol)
 
 
-@pytest.mark.parametrize("m,n,k,c_lay,epi,dtype,split", [
-    (4096, 4096, 1024, "row", 0, torch.float16, False),      # 256-wide tiles: 16-byte C reads
-    (1024, 2048, 1024, "row", 3, torch.bfloat16, False),     # 128-wide tiles, bf16
-    (2048, 6144, 512, "row", 2, torch.float16, False),       # 192-wide tiles
-    (4096, 4096, 1024, "row_off", 0, torch.float16, False),  # C rows not 16-byte aligned
-    (512, 2048, 1024, "col", 3, torch.float16, False),       # column-major C: per element
-    (200, 328, 96, "row", 2, torch.bfloat16, False),         # register-staged kernel, ragged
-    (768, 512, 2048, "row", 3, torch.float16, True),         # split-K tail: C in the reduce
-    (768, 512, 2048, "col", 2, torch.bfloat16, True)])
-def test_gemm_full_c_epilogue(m, n, k, c_lay, epi, dtype, split):
+@pytest.mark.parametrize("m,n,k,c_lay,epi,dtype,split,route", [
+    (4096, 4096, 1024, "row", 0, torch.float16, False, ("direct", (256, 256))),  # 16-byte C reads
+    (2048, 4096, 4096, "row", 3, torch.bfloat16, False, ("direct", (256, 128))),
+    (1024, 2048, 1024, "row", 3, torch.bfloat16, False, ("ring", (64, 128))),
+    (2048, 6144, 512, "row", 2, torch.float16, False, ("direct", (256, 192))),
+    (4096, 4096, 1024, "row_off", 0, torch.float16, False, ("direct", (256, 256))),  # C rows off 16 bytes
+    (512, 2048, 1024, "col", 3, torch.float16, False, ("ring", (32, 128))),  # column-major C: per element
+    (200, 328, 96, "row", 2, torch.bfloat16, False, ("ring", (32, 64))),
+    (363, 777, 8, "col", 2, torch.float16, False, ("staged", (0, 0))),
+    # K slices: C in the direct-load kernel's reduce, whole and ragged tiles
+    (1280, 1792, 4608, "row", 3, torch.float16, True, ("direct", (256, 256))),
+    (1220, 3235, 3584, "col", 2, torch.bfloat16, True, ("direct", (256, 256))),
+    (1220, 3235, 3584, "row", 0, torch.float16, True, ("direct", (256, 256))),
+    # and in the ring kernel's, N % 4 != 0 too
+    (256, 256, 2048, "row", 2, torch.bfloat16, True, ("ring", (32, 64))),
+    (81, 2746, 2752, "col", 3, torch.float16, True, ("ring", (128, 128))),
+    (10, 46, 912, "row", 0, torch.bfloat16, True, ("ring", (32, 64)))])
+def test_gemm_full_c_epilogue(m, n, k, c_lay, epi, dtype, split, route):
     # D = epi(alpha A B^T + beta C) with a whole matrix C (a residual): the
     # epilogue reads row-major, 16-byte aligned C rows 16 bytes a lane ahead
-    # of the stores, other layouts element by element; with a workspace the
-    # split-K reduce applies the same epilogue
+    # of the stores, other layouts element by element; with K slices the reduce
+    # applies the same epilogue
     _log(f"gemm full C {m}x{n}x{k} {c_lay} epi={epi} {dtype} split={split}")
     A = uniform((m, k), k=37, dtype=dtype)
     W = (uniform((n, k), k=38, dtype=dtype).float() * 0.05).to(dtype)
@@ -614,8 +626,9 @@ def test_gemm_full_c_epilogue(m, n, k, c_lay, epi, dtype, split):
         c_ptr, ldc_r, ldc_c = _p(cbuf) + off * cbuf.element_size(), n, 1
     want = O.gemm(A.float().numpy(), W.float().numpy().T, alpha=0.75, beta=0.5,
                   c=Cm.float().numpy(), epilogue={0: "none", 2: "gelu", 3: "silu"}[epi])
-    nws = _capi.lib().sph_gemm_workspace_bytes(1, m, n, k) if split else 0
-    assert (nws > 0) == split
+    nws = _capi.lib().sph_gemm_workspace_bytes_ex(0, 1, 1, m, n, k, k, k) if split else 0
+    plan = gemm_plan(1, m, n, k, 1, workspace=nws)
+    assert plan[:2] == route and (plan[2] > 1) == split == (nws > 0)
     ws = torch.empty(max(nws, 1), dtype=torch.uint8, device=DEV)
     d = torch.empty(m, n, dtype=dtype, device=DEV)
     _capi.call("sph_gemm_ex", DT[dtype], 0, 1, 1, m, n, k, 0.75, _p(ad), k, 0, _p(wd), k, 0,
@@ -730,15 +743,19 @@ def test_gemm_stream_epilogue(n, k):
                     what="stream residual epilogue")
 
 
-@pytest.mark.parametrize("m,n,k,pad", [(256, 128, 64, 0), (512, 384, 256, 8), (1024, 1280, 4096, 0),
-                                       (768, 256, 1024, 16), (256, 1280, 2048, 8),
-                                       (4, 12800, 4096, 0), (1, 300, 64, 8),
-                                       (8, 1000, 2056, 0), (5, 4100, 8192, 16)])
+@pytest.mark.parametrize("m,n,k,pad,route", [
+    (256, 128, 64, 0, ("ring", 1)), (512, 384, 256, 8, ("ring", 1)), (1024, 1280, 4096, 0, ("ring", 3)),
+    (768, 256, 1024, 16, ("ring", 1)), (256, 1280, 2048, 8, ("ring", 3)),
+    # whole 256-row tiles of the direct-load kernel, without and with K slices
+    (2560, 2688, 64, 8, ("direct", 1)), (1024, 896, 7232, 0, ("direct", 8)),
+    (512, 2560, 4800, 8, ("direct", 6)),
+    (4, 12800, 4096, 0, ("stream", 1)), (1, 300, 64, 8, ("stream", 1)),
+    (8, 1000, 2056, 0, ("stream", 1)), (5, 4100, 8192, 16, ("stream", 1))])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_gemm_swiglu(m, n, k, pad, dtype):
+def test_gemm_swiglu(m, n, k, pad, route, dtype):
     # silu(x Wg^T) * (x Wu^T) from one [2n, k] weight (gate rows first),
-    # padded leading dims on every operand; whole 256-row tiles (direct-load
-    # GEMM) and decode rows (m <= 8, weight-stream kernel)
+    # padded leading dims on every operand; whole 256-row tiles (ring or
+    # direct-load GEMM) and decode rows (m <= 8, weight-stream kernel)
     _log(f"gemm swiglu {m}x{n}x{k} pad={pad} {dtype}")
     X = uniform((m, k), k=31, dtype=dtype)
     W = (uniform((2 * n, k), k=32) * 0.05).to(dtype)
@@ -747,6 +764,8 @@ def test_gemm_swiglu(m, n, k, pad, dtype):
     wd = torch.zeros(2 * n, k + pad, dtype=dtype, device=DEV)
     wd[:, :k] = W.to(DEV)
     d = torch.full((m, n + pad), 7.0, dtype=dtype, device=DEV)
+    plan = gemm_plan(1, m, n, k, 1, lda=k + pad, ldb=k + pad, swiglu=True)
+    assert (plan[0], plan[2]) == route
     nws = _capi.lib().sph_gemm_swiglu_workspace_bytes(m, n, k)
     ws = torch.empty(max(nws, 1), dtype=torch.uint8, device=DEV)
     _capi.call("sph_gemm_swiglu", DT[dtype], m, n, k, _p(xd), k + pad, _p(wd), k + pad, _p(d),
@@ -760,28 +779,56 @@ def test_gemm_swiglu(m, n, k, pad, dtype):
         assert bool((d[:, n:] == 7.0).all()), "padding columns written"
 
 
-@pytest.mark.parametrize("batch,m,n,k,tb,pad,epi,dtype", [
-    (1, 9, 1024, 4096, 1, 0, 0, torch.float16),      # smallest ring rows, K split
-    (1, 33, 4096, 1032, 1, 8, 3, torch.bfloat16),    # last K tile one chunk deep, split
-    (1, 31, 65, 8, 1, 0, 2, torch.float16),          # one chunk of K, odd N
-    (1, 64, 300, 520, 0, 8, 0, torch.bfloat16),      # row-major B, partial K tile (padded rows)
-    (1, 65, 264, 1544, 0, 0, 3, torch.float16),      # row-major B, split, N % 128 != 0
-    (1, 129, 1001, 2048, 1, 0, 2, torch.bfloat16),   # odd N: element stores, no split
-    (1, 200, 4100, 4096, 1, 8, 0, torch.float16),    # N % 128 != 0 through the reduce
-    (1, 193, 512, 96, 1, 0, 0, torch.bfloat16),      # 32-deep K tiles
-    (3, 300, 136, 776, 0, 0, 0, torch.float16),      # batched, ragged M, N and K
-    (32, 300, 392, 384, 0, 0, 0, torch.float16),     # batched short K, uneven round: last K register-staged
-    (32, 300, 392, 392, 0, 0, 0, torch.bfloat16),    # the same past it, on the ring kernel
-    (8, 512, 1280, 64, 0, 8, 3, torch.float16),      # whole 256-row tiles of such a round
-    (1, 2100, 4104, 576, 1, 0, 3, torch.float16),    # ragged rows and columns of 256-row tiles
-    (1, 2100, 4104, 576, 0, 8, 0, torch.bfloat16),   # the same, row-major B
-    (1, 1100, 3000, 4096, 1, 0, 2, torch.float16)])  # ragged, K-split tail of 256-row tiles
-def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype):
+@pytest.mark.parametrize("batch,m,n,k,tb,pad,epi,dtype,route", [
+    (1, 9, 1024, 4096, 1, 0, 0, torch.float16, ("ring", 8)),     # smallest ring rows, K split
+    (1, 33, 4096, 1032, 1, 8, 3, torch.bfloat16, ("ring", 1)),   # last K tile one chunk deep
+    (1, 37, 2141, 2192, 1, 8, 3, torch.float16, ("ring", 7)),    # K slices, a partial last K tile
+    (1, 31, 65, 8, 1, 0, 2, torch.float16, ("staged", 1)),       # one chunk of K, odd N
+    (1, 64, 300, 520, 0, 8, 0, torch.bfloat16, ("ring", 1)),     # row-major B, partial K tile (padded rows)
+    (1, 65, 264, 1544, 0, 0, 3, torch.float16, ("ring", 5)),     # row-major B, split, N % 128 != 0
+    (1, 129, 1001, 2048, 1, 0, 2, torch.bfloat16, ("ring", 3)),  # odd N: element stores
+    (1, 200, 4100, 4096, 1, 8, 0, torch.float16, ("ring", 3)),   # N % 128 != 0 through the reduce
+    (1, 193, 512, 96, 1, 0, 0, torch.bfloat16, ("ring", 1)),
+    (3, 300, 136, 776, 0, 0, 0, torch.float16, ("ring", 1)),     # batched, ragged M, N and K
+    (32, 300, 392, 384, 0, 0, 0, torch.float16, ("staged", 1)),  # batched short K, uneven round
+    (32, 300, 392, 712, 0, 0, 0, torch.bfloat16, ("ring", 1)),   # the same past it
+    (8, 512, 1280, 64, 0, 8, 3, torch.float16, ("direct", 1)),   # whole 256-row tiles of such a round
+    (1, 2100, 4104, 576, 1, 0, 3, torch.float16, ("staged", 1)),
+    (1, 2100, 4104, 576, 0, 8, 0, torch.bfloat16, ("ring", 1)),
+    (1, 1100, 3000, 4096, 1, 0, 2, torch.float16, ("ring", 1)),
+    # ragged rows and columns of the direct-load kernel's tiles, 256 and 128 wide
+    (1, 2616, 4841, 64, 1, 0, 0, torch.bfloat16, ("direct", 1)),
+    (1, 2191, 5840, 64, 0, 8, 3, torch.float16, ("direct", 1)),
+    (1, 1993, 5056, 192, 0, 0, 2, torch.bfloat16, ("direct", 1)),
+    (1, 2236, 2994, 3136, 1, 8, 0, torch.float16, ("direct", 1)),
+    (1, 1311, 3864, 3520, 0, 0, 3, torch.bfloat16, ("direct", 1)),
+    (1, 2000, 6144, 320, 1, 0, 2, torch.float16, ("direct", 1)),   # 192 wide
+    # K slices of such tiles
+    (1, 1220, 3235, 3584, 1, 0, 3, torch.bfloat16, ("direct", 3)),
+    (1, 2835, 1528, 3072, 0, 8, 0, torch.float16, ("direct", 3)),
+    (1, 453, 4352, 4672, 1, 8, 2, torch.float16, ("direct", 7)),
+    # every tile of the ring kernel that the cases above leave out, with and
+    # without K slices
+    (1, 41, 2693, 1472, 1, 0, 0, torch.bfloat16, ("ring", 5)),
+    (1, 311, 5589, 16, 1, 0, 3, torch.float16, ("ring", 1)),
+    (1, 2102, 48, 1024, 0, 0, 0, torch.bfloat16, ("ring", 4)),
+    (1, 1205, 1968, 8, 0, 0, 2, torch.float16, ("ring", 1)),
+    (1, 2488, 48, 2432, 0, 8, 0, torch.bfloat16, ("ring", 8)),
+    (1, 81, 2746, 2752, 1, 0, 0, torch.float16, ("ring", 8)),
+    (1, 987, 5465, 1736, 1, 0, 2, torch.bfloat16, ("ring", 1)),
+    (1, 1855, 1080, 2672, 0, 0, 0, torch.float16, ("ring", 3)),
+    (1, 1280, 1609, 2880, 1, 8, 3, torch.bfloat16, ("ring", 3)),
+    (1, 980, 4488, 1704, 1, 0, 0, torch.float16, ("ring", 1)),
+    (1, 549, 3280, 4440, 1, 8, 0, torch.bfloat16, ("ring", 3))])
+def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype, route):
     # rows that do not fill 256-row tiles, K down to one 16-byte chunk: every
-    # element against the oracle, with and without the K-split workspace, and
-    # nothing written outside D
+    # element against the oracle, with the K-split workspace of the size that
+    # the library names and without it, and nothing written outside D or past
+    # the workspace.  route: kernel and K slices with the workspace.
     if tb == 0 and (n + pad) % 8:
         n += 8 - (n + pad) % 8
+    plan = gemm_plan(batch, m, n, k, tb, lda=k + pad, ldb=(k if tb else n) + pad)
+    assert (plan[0], plan[2]) == route
     _log(f"gemm ragged {batch}x{m}x{n}x{k} tb={tb} pad={pad} epi={epi} {dtype}")
     A = uniform((batch, m, k), k=51, dtype=dtype)
     W = (uniform((batch, n, k) if tb else (batch, k, n), k=52, dtype=dtype).float() * 0.05).to(dtype)
@@ -797,9 +844,12 @@ def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype):
                   c=bias.float().numpy()[None, None, :],
                   epilogue={0: "none", 2: "gelu", 3: "silu"}[epi])
     tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
-    nws = _capi.lib().sph_gemm_workspace_bytes(batch, m, n, k)
-    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
+    nws = _capi.lib().sph_gemm_workspace_bytes_ex(0, tb, batch, m, n, k, k + pad,
+                                                  (k if tb else n) + pad)
+    ws = torch.full((nws + 4096,), 255, dtype=torch.uint8, device=DEV)
     for w_ptr, w_n in ((None, 0), (_p(ws), nws)):
+        if w_ptr and not w_n:
+            continue
         d = torch.full((batch, m + 1, n), 7.0, dtype=dtype, device=DEV)
         _capi.call("sph_gemm_ex", DT[dtype], 0, tb, batch, m, n, k, 0.75, _p(ad), k + pad,
                    a_buf[0].numel(), _p(wd), w_buf.shape[2], w_buf[0].numel(), 0.5, _p(bd), 0, 1,
@@ -807,54 +857,84 @@ def test_gemm_ragged_rows(batch, m, n, k, tb, pad, epi, dtype):
         _sync()
         assert_close_fp(d[:, :m], want, out_dtype=dtype, what="ragged gemm", **tol)
         assert bool((d[:, m] == 7.0).all()), "rows past M written"
+        assert bool((ws[nws:] == 255).all()), "bytes past the workspace written"
 
 
-@pytest.mark.parametrize("batch,m,n,k,tb,share,epi,dtype", [
-    (1, 300, 500, 700, 0, 0, 0, torch.float16),       # N and K off 8: both operands padded
-    (1, 301, 505, 704, 0, 0, 3, torch.bfloat16),      # K whole: only B's rows padded
-    (1, 1001, 777, 1029, 1, 0, 2, torch.float16),     # K-contiguous B, odd K
-    (1, 5, 2001, 1001, 0, 0, 0, torch.float16),       # few rows
-    (1, 1300, 1283, 515, 0, 0, 0, torch.bfloat16),    # 256-row tiles on padded operands
-    (3, 130, 777, 200, 0, 0, 0, torch.float16),       # batched, odd N
-    (3, 257, 129, 301, 0, 1, 2, torch.bfloat16)])     # one B for the batch
-def test_gemm_operands_off_16_bytes(batch, m, n, k, tb, share, epi, dtype):
-    # contiguous operands whose rows are off 16-byte chunks, with the
-    # workspace (padded copies where the model takes them) and without it
-    _log(f"gemm off 16 bytes {batch}x{m}x{n}x{k} tb={tb} share={share} epi={epi} {dtype}")
-    A = uniform((batch, m, k), k=61, dtype=dtype)
-    nb = 1 if share else batch
+@pytest.mark.parametrize("batch,m,n,k,tb,share,epi,dtype,layout", [
+    (1, 300, 500, 700, 0, 0, 0, torch.float16, ""),       # N and K off 8: both operands padded
+    (1, 301, 505, 704, 0, 0, 3, torch.bfloat16, ""),      # K whole: only B's rows padded
+    (1, 1001, 777, 1029, 1, 0, 2, torch.float16, ""),     # K-contiguous B, odd K
+    (1, 5, 2001, 1001, 0, 0, 0, torch.float16, ""),       # few rows
+    (1, 1300, 1283, 515, 0, 0, 0, torch.bfloat16, ""),
+    (1, 2300, 5001, 1501, 0, 0, 0, torch.bfloat16, ""),   # 256-row tiles on padded operands
+    (3, 130, 777, 200, 0, 0, 0, torch.float16, ""),       # batched, odd N
+    (3, 257, 129, 301, 0, 1, 2, torch.bfloat16, ""),  # one B for the batch
+    (3, 257, 129, 301, 0, 2, 0, torch.float16, ""),   # one A for the batch
+    (1, 300, 505, 700, 0, 0, 0, torch.bfloat16, "wide"),   # rows longer than the matrix
+    (1, 1001, 777, 1029, 1, 0, 2, torch.float16, "wide"),
+    (3, 130, 777, 203, 0, 0, 3, torch.float16, "wide"),
+    (1, 300, 505, 701, 0, 0, 0, torch.float16, "base"),    # operands 2 bytes off 16
+    (1, 512, 768, 1024, 0, 0, 0, torch.bfloat16, "base"),  # whole rows, but not their first
+    (2, 300, 512, 704, 1, 0, 0, torch.float16, "base")])
+def test_gemm_operands_off_16_bytes(batch, m, n, k, tb, share, epi, dtype, layout):
+    # operands whose rows are off 16-byte chunks (contiguous; in rows 3 longer
+    # than the matrix; one element past a 16-byte boundary), with the workspace
+    # (padded copies where the model takes them), without it and with less
+    _log(f"gemm off 16 bytes {batch}x{m}x{n}x{k} tb={tb} share={share} {layout} epi={epi} {dtype}")
+    extra, off = 3 if layout == "wide" else 0, 1 if layout == "base" else 0
+    na, nb = 1 if share == 2 else batch, 1 if share == 1 else batch
+    A = uniform((na, m, k), k=61, dtype=dtype)
+    lda, ldb = k + extra, (k if tb else n) + extra
     W = (uniform((nb, n, k) if tb else (nb, k, n), k=62, dtype=dtype).float() * 0.05).to(dtype)
     bias = uniform((n,), k=63, dtype=dtype)
     # the elements next to the operands must not enter the product
-    ad = torch.full((A.numel() + 16,), float("nan"), dtype=dtype, device=DEV)
-    ad[:A.numel()] = A.flatten().to(DEV)
-    wd = torch.full((W.numel() + 16,), float("nan"), dtype=dtype, device=DEV)
-    wd[:W.numel()] = W.flatten().to(DEV)
+    def place(t, ld):
+        buf = torch.full((t.shape[0] * t.shape[1] * ld + 16,), float("nan"), dtype=dtype)
+        buf[off:off + t.shape[0] * t.shape[1] * ld].view(t.shape[0], t.shape[1], ld)[..., :t.shape[2]] = t
+        return buf.to(DEV)
+
+    ad, wd = place(A, lda), place(W, ldb)
+    eb = 2 * off
     bd = bias.to(DEV)
     wf = W.float().numpy()
     want = O.gemm(A.float().numpy(), np.swapaxes(wf, 1, 2) if tb else wf, alpha=0.75, beta=0.5,
                   c=bias.float().numpy()[None, None, :],
                   epilogue={0: "none", 2: "gelu", 3: "silu"}[epi])
     tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
-    nws = _capi.lib().sph_gemm_workspace_bytes(batch, m, n, k)
-    assert nws > 0
-    ws = torch.full((nws,), 255, dtype=torch.uint8, device=DEV)
+    nws = _capi.lib().sph_gemm_workspace_bytes_ex(0, tb, batch, m, n, k, lda, ldb)
+    if layout != "base":  # (the sizing knows leading dimensions, not addresses)
+        assert nws > 0 and gemm_plan(batch, m, n, k, tb, lda=lda, ldb=ldb)[3]
+    nws = max(nws, 8 << 20)
+    ws = torch.full((nws + 4096,), 255, dtype=torch.uint8, device=DEV)
     for w_n in (0, nws, nws - 256):
         d = torch.full((batch, m + 1, n), 7.0, dtype=dtype, device=DEV)
-        _capi.call("sph_gemm_ex", DT[dtype], 0, tb, batch, m, n, k, 0.75, _p(ad), k, m * k, _p(wd),
-                   k if tb else n, 0 if share else n * k, 0.5, _p(bd), 0, 1, 0, _p(d), n,
+        _capi.call("sph_gemm_ex", DT[dtype], 0, tb, batch, m, n, k, 0.75, _p(ad) + eb, lda, 0 if share == 2 else m * lda,
+                   _p(wd) + eb, ldb, 0 if share == 1 else W.shape[1] * ldb, 0.5, _p(bd), 0, 1, 0, _p(d), n,
                    (m + 1) * n, epi, _p(ws) if w_n else None, w_n, _stream())
         _sync()
         assert_close_fp(d[:, :m], want, out_dtype=dtype, what="unaligned gemm", **tol)
         assert bool((d[:, m] == 7.0).all()), "rows past M written"
+        assert bool((ws[w_n:] == 255).all()), "bytes past the workspace written"
+        ws.fill_(255)
 
 
-@pytest.mark.parametrize("m,n,k,pad", [(9, 512, 4096, 0), (24, 1000, 520, 8), (100, 513, 512, 0),
-                                       (333, 1280, 1024, 0), (1100, 1280, 2048, 8),
-                                       (2, 64, 40, 0)])
+@pytest.mark.parametrize("m,n,k,pad,route", [
+    (9, 512, 4096, 0, ("ring", 0, 8)), (24, 1000, 520, 8, ("ring", 0, 1)),
+    (100, 513, 512, 0, ("ring", 0, 1)), (333, 1280, 1024, 0, ("ring", 1, 1)),
+    (1100, 1280, 2048, 8, ("ring", 3, 1)), (2, 64, 40, 0, ("ring", 0, 1)),
+    # every tile of the ring kernel, without and with K slices
+    (103, 2078, 8, 8, ("ring", 1, 1)), (49, 1361, 1728, 0, ("ring", 1, 5)),
+    (1398, 371, 8, 0, ("ring", 2, 1)), (36, 1408, 2304, 8, ("ring", 2, 8)),
+    (633, 1664, 40, 0, ("ring", 3, 1)), (67, 1433, 2328, 8, ("ring", 3, 8)),
+    (1160, 2560, 40, 0, ("ring", 4, 1)), (1813, 330, 4360, 0, ("ring", 4, 5)),
+    (429, 2553, 8, 8, ("ring", 5, 1)), (143, 2992, 6784, 0, ("ring", 5, 5)),
+    # ragged rows of the direct-load kernel's tiles
+    (1190, 5376, 64, 0, ("direct", -1, 1)), (1617, 4224, 64, 8, ("direct", -1, 1)),
+    (2157, 512, 5504, 0, ("direct", -1, 7)), (1539, 640, 6336, 8, ("direct", -1, 7))])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_gemm_swiglu_any_rows(m, n, k, pad, dtype):
-    # the row counts, widths and depths that sph_gemm_swiglu refuses
+def test_gemm_swiglu_any_rows(m, n, k, pad, route, dtype):
+    # the row counts, widths and depths that sph_gemm_swiglu refuses (route:
+    # kernel, ring configuration and K slices with the workspace)
     _log(f"gemm swiglu any {m}x{n}x{k} pad={pad} {dtype}")
     X = uniform((m, k), k=54, dtype=dtype)
     W = (uniform((2 * n, k), k=55) * 0.05).to(dtype)
@@ -865,34 +945,40 @@ def test_gemm_swiglu_any_rows(m, n, k, pad, dtype):
     xf, wf = X.float().numpy(), W.float().numpy()
     want = O.silu(O.gemm(xf, wf[:n].T)) * O.gemm(xf, wf[n:].T)
     tol = dict(rtol=1e-2, atol=1e-2) if dtype == torch.float16 else dict(rtol=2e-2, atol=2e-2)
+    plan = gemm_plan(1, m, n, k, 1, lda=k + pad, ldb=k + pad, swiglu=True)
+    assert (plan[0], plan[4], plan[2]) == route
     nws = _capi.lib().sph_gemm_swiglu_workspace_bytes(m, n, k)
-    ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)
-    for w_n in (0, nws):
+    ws = torch.full((nws + 4096,), 255, dtype=torch.uint8, device=DEV)
+    for w_n in (0, nws) if nws else (0,):
         d = torch.full((m + 1, n + pad), 7.0, dtype=dtype, device=DEV)
         _capi.call("sph_gemm_swiglu_any", DT[dtype], m, n, k, _p(xd), k + pad, _p(wd), k + pad,
                    _p(d), n + pad, _p(ws) if w_n else None, w_n, _stream())
         _sync()
         assert_close_fp(d[:m, :n], want, out_dtype=dtype, what=f"swiglu any {dtype}", **tol)
         assert bool((d[m] == 7.0).all()) and bool((d[:, n:] == 7.0).all()), "outside D written"
+        assert bool((ws[w_n:] == 255).all()), "bytes past the workspace written"
 
 
-@pytest.mark.parametrize("m,n,k,tb,epi,dtype", [
-    (2048, 4096, 12800, True, 0, torch.float16),   # 128 tiles, 2 K slices (c4 down shape)
-    (1024, 4096, 8192, False, 3, torch.bfloat16),  # row-major B, bf16: 64 tiles, 4 slices
-    (768, 512, 2048, False, 2, torch.float16),     # 6 tiles, 8 K slices
-    (512, 1024, 12800, True, 0, torch.float16),    # 8 tiles, 200 K tiles in 8 slices
-    (256, 256, 2048, True, 3, torch.float16),      # one tile
-    (2048, 10240, 2048, True, 0, torch.float16),   # 320 tiles: a full round, then 64 in 4 slices
-    (2048, 10240, 2048, False, 2, torch.bfloat16)])
-def test_gemm_splitk_tail(m, n, k, tb, epi, dtype):
-    # sph_gemm_ex with a workspace: the partial last round of 256 x 256
-    # tiles runs as K slices plus a reduce (alpha, beta*C with a bias row,
-    # activation applied there); against the oracle and the call without a
-    # workspace
+@pytest.mark.parametrize("m,n,k,tb,epi,dtype,route", [
+    # 256 x 256 tiles of the direct-load kernel: the last round in K slices
+    (2048, 4096, 12800, True, 0, torch.float16, ("direct", 2)),   # 128 tiles (c4 down shape)
+    (1024, 4096, 8192, False, 3, torch.bfloat16, ("direct", 4)),  # row-major B, bf16: 64 tiles
+    (1280, 1792, 4608, True, 2, torch.float16, ("direct", 7)),    # 35 tiles, 72 K tiles
+    (2048, 10240, 2048, True, 0, torch.float16, ("direct", 4)),   # 320 tiles: a full round, then 64
+    (2048, 10240, 2048, False, 2, torch.bfloat16, ("direct", 4)),
+    # few such tiles: K slices of the ring kernel
+    (768, 512, 2048, False, 2, torch.float16, ("ring", 4)),
+    (512, 1024, 12800, True, 0, torch.float16, ("ring", 8)),
+    (256, 256, 2048, True, 3, torch.float16, ("ring", 8))])
+def test_gemm_splitk_tail(m, n, k, tb, epi, dtype, route):
+    # sph_gemm_ex with a workspace: tiles run as K slices plus a reduce (alpha,
+    # beta*C with a bias row, activation applied there); against the oracle and
+    # the call without a workspace
     _log(f"gemm split-K tail {m}x{n}x{k} tb={tb} epi={epi} {dtype}")
     lib = _capi.lib()
-    nws = lib.sph_gemm_workspace_bytes(1, m, n, k)
-    assert nws > 0, "shape should take a split"
+    nws = lib.sph_gemm_workspace_bytes_ex(0, int(tb), 1, m, n, k, k, k if tb else n)
+    plan = gemm_plan(1, m, n, k, int(tb))
+    assert (plan[0], plan[2]) == route and nws > 0
     X = uniform((m, k), k=61).to(dtype)
     W = (uniform((n, k) if tb else (k, n), k=62) * 0.05).to(dtype)
     bias = uniform((n,), k=63).to(dtype)
@@ -1159,8 +1245,8 @@ def test_attention_causal_mask_matches_causal_positions():
     ("lowest", 2, 140, 72, 0), ("lowest", 1, 200, 320, 0)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
-    # row counts off the 128-row block: the oracle's rows, the same bits as
-    # the padded call's, and nothing written past the last row
+    # row counts off the 128-row block: the oracle's rows, the same bits as a
+    # call on rows padded to whole blocks, and nothing written past the last row
     _log(f"attention ragged {kind} b={b} mq={mq} sk={sk} {dtype}")
     q = randn((b, mq, 128), k=58, dtype=dtype)
     k = randn((b, sk, 128), k=59, dtype=dtype)
@@ -1197,6 +1283,24 @@ def test_attention_ragged_rows(kind, b, mq, sk, causal_q, dtype):
         _sync()
         assert_close_fp(o[:, :mq], want, out_dtype=dtype, what="ragged attention", **tol)
         assert bool((o[:, mq] == 7.0).all()), "rows past mq written"
+        mw = (mq + 127) // 128 * 128
+        qw = torch.zeros(b, mw, 128, dtype=dtype, device=DEV)
+        qw[:, :mq] = qd
+        mkw, ldw, smw = None, ldm, sm
+        if mask is not None:
+            mkw = md
+            if ldm:  # (one row for all needs no padding)
+                mkw = torch.zeros(*md.shape[:-2], mw, sk, dtype=dtype, device=DEV)
+                mkw[..., :mq, :] = md
+                smw = mw * sk if md.dim() == 3 else 0
+        ow = torch.empty(b, mw, 128, dtype=dtype, device=DEV)
+        nww = _capi.lib().sph_attention_workspace_bytes(b, mw, sk, smw) if w_n else 0
+        ww = torch.full((max(nww, 16),), 255, dtype=torch.uint8, device=DEV)
+        _capi.call("sph_attention_fwd", DT[dtype], b, mw, sk, 128, _p(qw), 128, mw * 128, _p(kd), 128,
+                   sk * 128, _p(vd), 128, sk * 128, _p(mkw), ldw, smw, cq, sk - cq if cq else 0,
+                   scale, _p(ow), 128, mw * 128, _p(ww) if nww else None, nww, _stream())
+        _sync()
+        assert torch.equal(ow[:, :mq], o[:, :mq]), "padded rows change the result"
     # sph_attention_fwd keeps refusing these rows
     rc = _capi.lib().sph_attention_fwd(DT[dtype], b, mq, sk, 128, _p(qd), 128, mq * 128, _p(kd), 128,
                                        sk * 128, _p(vd), 128, sk * 128, None, 0, 0, 0, 0,

@@ -1621,6 +1621,7 @@ extern "C" int sph_gemm_plan(int trans_a, int trans_b, int64_t batch, int64_t m,
   plan[2] = ring ? c.ring.bn : dl_ ? c.dl.kind : 0;
   plan[3] = ring ? c.ring.splits : dl_ ? c.dl.split.splits : 1;
   plan[4] = (c.pack.a ? 1 : 0) + (c.pack.b ? 2 : 0);
+  plan[5] = ring ? c.ring.cfg : -1;
   return SPH_OK;
 }
 
