@@ -147,7 +147,8 @@ __global__ void __launch_bounds__((dl::Cfg<BN_, WTN_>::NT)) gemm_dl_kernel(const
   // Buffer ranges: exactly the bytes this tile's rows (columns) span, so the
   // rows of a last, partial tile that lie past M or N read zeros (and are
   // not stored).
-  const int64_t arows = min(static_cast<int64_t>(BM), p.m - m0), brows = min(static_cast<int64_t>(BN), (B_KCONT ? p.n : p.nb) - n0);
+  const int64_t arows = min(static_cast<int64_t>(BM), p.m - m0);
+  const int64_t brows = min(static_cast<int64_t>(BN), (B_KCONT ? p.n : p.nb) - n0);
   const i32x4 ra = buffer_rsrc(A + m0 * lda, static_cast<uint32_t>(((arows - 1) * lda + p.k) * 2));
   // (SwiGLU: from gate row n0 to up row n + n0 + 127)
   const i32x4 rb = SWIGLU

@@ -17,7 +17,9 @@
 //     instead of the second launch would need device-scope releases, each an
 //     L2 write-back on this 8-XCD part.
 //   * The MFMAs take B as the first operand: a lane then holds 4 consecutive
-//     output columns of one row and stores them without staging.
+//     output columns of one row.  K slices store those as they lie; unsplit
+//     products pass 16 rows at a time through LDS, so that stores cover whole
+//     tile rows.
 #include <algorithm>
 
 #include "gemm_ring.h"
@@ -80,12 +82,7 @@ struct Cfg {
 // Waits until at most `tiles` K tiles of L loads each are still in flight.
 template <int ST, int L>
 __device__ inline void wait_tiles(int tiles) {
-  if constexpr (ST >= 6) {
-    if (tiles >= 4) return wait_vmcnt<4 * L>();
-  }
-  if constexpr (ST >= 5) {
-    if (tiles >= 3) return wait_vmcnt<3 * L>();
-  }
+  static_assert(ST <= 4, "at most two tiles in flight behind the one awaited");
   if constexpr (ST >= 4) {
     if (tiles >= 2) return wait_vmcnt<2 * L>();
   }
@@ -413,8 +410,8 @@ double hot_us(int cfg, int64_t wgs, int64_t k) {
 }  // namespace
 
 // Time of a plan: ~2 us of launch and, per round of workgroups, ~4 us of first
-// bytes and output plus the K columns of the fullest CU, but no less than the operands' time from HBM (~5.2
-// TB/s); a K split adds the reduce launch (~2 us) and its partial sums'
+// bytes and output plus the K columns of the fullest CU, but no less than the
+// operands' time from HBM (~5.2 TB/s); a K split adds the reduce launch (~2 us) and its partial sums'
 // write and read (~6 TB/s, mostly from the caches).  At least 256 K columns
 // a slice and at most 8 slices: past that the partial sums cost more than
 // the shorter slices save (24 x 4096 x 4096: 4 slices 11.5 us, 8 12.4).

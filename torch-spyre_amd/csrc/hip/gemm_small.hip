@@ -40,13 +40,14 @@ __device__ inline u32x4 norm_chunk(u32x4 x, u32x4 w, float& ss) {
 // so short rows such as attention keys do not idle most of the workgroup)
 // and a workgroup holds 256/TPR groups.  Workgroups loop over row blocks
 // (grid capped near the number of resident workgroups), so long matrices do
-// not end in a partial wave of workgroups.  A (at most 8 x K, read by every
+// not end in a partial wave of workgroups.  A (at most 16 x K, read by every
 // workgroup) comes through the caches.  fp16 uses v_dot2_f32_f16, bf16
 // v_dot2_f32_bf16 (two products summed into an fp32 accumulator; subnormals
 // kept).  With bf16 widened into fp32 FMAs the vector ALUs set the time: 4 x
 // 6144 x 4096 15.3 us against 13.0, 8 x 49155 x 4096 112 against 83, gate / up of
-// 8 x 12800 x 4096 59.7 against 47.3, the same error against 64 bits.  Partial sums are reduced within the group by butterflies
-// and, for groups wider than a wave, through LDS.
+// 8 x 12800 x 4096 59.7 against 47.3, the same error against 64 bits.  Partial
+// sums are reduced within the group by butterflies and, for groups wider than a
+// wave, through LDS.
 // ---------------------------------------------------------------------------
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
