@@ -516,7 +516,7 @@ def test_gemm_whole_tile_epilogue_and_batch(tb):
 
 @pytest.mark.parametrize("batch,m,n,k,pad,epi,dtype", [
     (1, 2048, 6144, 4096, 0, 0, torch.float16),     # c4 QKV: 256 tiles of 256 x 192
-    (1, 4096, 6144, 320, 8, 2, torch.float16),      # 512 tiles, padded rows, GELU
+    (1, 4096, 6144, 1024, 8, 2, torch.float16),     # 512 tiles, padded rows, GELU
     (1, 2048, 6144, 1216, 0, 3, torch.bfloat16),    # bf16, SiLU, 19 K tiles
     (2, 1024, 6144, 256, 0, 0, torch.float16)])     # batched: 2 x 128 tiles
 def test_gemm_192_wide_tiles(batch, m, n, k, pad, epi, dtype):
@@ -557,7 +557,7 @@ def test_gemm_192_wide_tiles(batch, m, n, k, pad, epi, dtype):
     (1, 2048, 4096, 4096, 1, 0, 0, torch.float16),   # c4 O (no workspace): 256 tiles of 256 x 128
     (1, 2048, 4096, 4096, 0, 0, 3, torch.bfloat16),  # row-major B, bf16, SiLU
     (4, 1024, 2048, 1024, 1, 8, 2, torch.float16),   # batched, padded rows, GELU
-    (3, 768, 1152, 64, 1, 8, 3, torch.bfloat16),     # batched, one K tile, bf16
+    (3, 768, 2176, 64, 1, 8, 3, torch.bfloat16),     # batched, one K tile, bf16
     (1, 768, 1408, 64, 0, 8, 0, torch.float16)])     # N % 256 != 0, row-major B, one K tile
 def test_gemm_128_wide_tiles(batch, m, n, k, tb, pad, epi, dtype):
     # shapes whose 256-wide tiles leave most CUs idle and that have no
@@ -790,7 +790,7 @@ def test_gemm_swiglu(m, n, k, pad, route, dtype):
     (1, 200, 4100, 4096, 1, 8, 0, torch.float16, ("ring", 3)),   # N % 128 != 0 through the reduce
     (1, 193, 512, 96, 1, 0, 0, torch.bfloat16, ("ring", 1)),
     (3, 300, 136, 776, 0, 0, 0, torch.float16, ("ring", 1)),     # batched, ragged M, N and K
-    (32, 300, 392, 384, 0, 0, 0, torch.float16, ("staged", 1)),  # batched short K, uneven round
+    (32, 300, 392, 128, 0, 0, 0, torch.float16, ("staged", 1)),  # batched short K, uneven round
     (32, 300, 392, 712, 0, 0, 0, torch.bfloat16, ("ring", 1)),   # the same past it
     (8, 512, 1280, 64, 0, 8, 3, torch.float16, ("direct", 1)),   # whole 256-row tiles of such a round
     (1, 2100, 4104, 576, 1, 0, 3, torch.float16, ("staged", 1)),

@@ -1178,14 +1178,16 @@ inline void launch_pack(const GemmArgs& p, const GemmArgs& q, int64_t batch, boo
 // Time of the register-staged kernel on aligned operands in the caches, K up to
 // ~1500 (us; fitted with the ring kernel's hot_us): per round of 512 tiles of 128
 // x 128, or of 256 x 256 tiles where those give every CU one, or one round of
-// 64 x 64 tiles.
+// 64 x 64 tiles.  Output rows off 16 bytes cost more.
 inline double staged_us(const GemmArgs& p, int64_t batch, bool b_kcont) {
   const double k = static_cast<double>(p.k) * 1e-3;
   const int64_t t256 = ceil_div(p.m, 256) * ceil_div(p.n, 256) * batch;
   const int64_t t128 = ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
-  if (t256 >= kNumCUs) return static_cast<double>(ceil_div(t256, kNumCUs)) * (11.5 + 36.0 * k);
+  const bool odd = p.n % 8 != 0;
+  if (t256 >= kNumCUs) return static_cast<double>(ceil_div(t256, kNumCUs)) * ((odd ? 17.0 : 12.7) + 36.0 * k);
   if (t128 >= 128) {
-    const double one = b_kcont ? 6.3 + 14.6 * k : 6.7 + 19.7 * k, two = b_kcont ? 7.3 + 19.0 * k : 7.4 + 25.6 * k;
+    const double one = (b_kcont ? 6.3 + 14.6 * k : 6.7 + 19.7 * k) + (odd ? 0.5 : 0.0);
+    const double two = (b_kcont ? 7.3 + 19.0 * k : 7.4 + 25.6 * k) + (odd ? 1.4 : 0.0);
     const int64_t rest = t128 % (2 * kNumCUs);
     return static_cast<double>(t128 / (2 * kNumCUs)) * two + (rest > kNumCUs ? two : rest > 0 ? one : 0.0);
   }
@@ -1194,13 +1196,18 @@ inline double staged_us(const GemmArgs& p, int64_t batch, bool b_kcont) {
 }
 
 // Short K where the ring kernel's epilogue or tiles cost more than its loads
-// save (fp16, K-contiguous B, ring beside register-staged: 10 x 250 x 1024 x 32
-// 12.3 / 7.0 us, 24 x 552 x 512 x 128 13.3 / 11.3, 4 x 1608 x 608 x 224 16.5 /
-// 13.1; row-major 10 x 1571 x 328 x 128 13.1 / 11.2).  Past the K of both fits the
-// ring kernel is ahead (bmm of 250 to 500 tiles: K 1024 even, 2048 5 % ahead).
+// save; by a margin where 256 x 256 tiles fill the CUs, whose times spread most.
+// Of the 1180 products of the fits, 41 take more than 5 % longer than on the
+// other kernel (336 with the ring kernel for all).  fp16, ring beside
+// register-staged: K-contiguous B 10 x 250 x 1024 x 32 12.3 / 7.0 us, 24 x 552 x
+// 512 x 128 13.3 / 11.3, 4 x 1608 x 608 x 224 16.5 / 13.1; row-major 10 x 1571 x
+// 328 x 128 13.1 / 11.2.  Past the K of both fits the ring kernel is ahead (bmm of
+// 250 to 500 tiles: K 1024 even, 2048 5 % ahead).
 constexpr int64_t kStagedMaxK = 1536;
 inline bool staged_leads(const GemmArgs& p, int64_t batch, bool b_kcont, const GemmRoute& r) {
-  return r.ring && r.rp.splits == 1 && p.k <= kStagedMaxK && staged_us(p, batch, b_kcont) < r.rp.hot_us;
+  if (!r.ring || r.rp.splits != 1 || p.k > kStagedMaxK) return false;
+  const bool large = ceil_div(p.m, 256) * ceil_div(p.n, 256) * batch >= kNumCUs;
+  return staged_us(p, batch, b_kcont) < (large ? 0.85 : 0.97) * r.rp.hot_us;
 }
 
 // 9 to 16 rows times few columns with a long K that the ring kernel does not

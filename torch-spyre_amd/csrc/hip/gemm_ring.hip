@@ -388,15 +388,15 @@ constexpr int64_t kCUs = 256;
 // Unsplit products of K up to ~1500 with operands in the caches: us per round of
 // workgroups, fixed and per 1000 K columns, with one, two or three workgroups
 // on the CUs, in the order of kRing (128 x 128 tiles on 4 waves, third: one on
-// the CUs behind a full round).  Fitted to 880 products (both layouts of B,
+// the CUs behind a full round).  Fitted to 1180 products (both layouts of B,
 // 40 to 3000 rows and 40 to 6000 columns in batches of 1 to 64, K 8 to 3072).
 // What the plan's model leaves out is the second workgroup's epilogue (128 x
 // 128 tiles, 480 of them, K 32: 11.5 us against 7.0 for 160 at K 64) and the 192
 // x 128 tile's (160, K 32: 12.3 us).
 constexpr double kHot[kRingCfgs][3][2] = {
     {{1.5, 4.0}, {1.6, 6.0}, {2.2, 8.0}}, {{2.4, 5.5}, {3.0, 9.0}, {}},
-    {{4.0, 7.6}, {5.2, 12.0}, {}},        {{4.6, 10.8}, {}, {}},
-    {{4.6, 11.0}, {9.0, 19.5}, {7.1, 11.0}}, {{11.0, 18.5}, {12.3, 34.0}, {}}};
+    {{4.0, 7.6}, {4.3, 12.0}, {}},        {{4.3, 10.8}, {}, {}},
+    {{4.2, 11.0}, {8.5, 17.2}, {8.3, 11.0}}, {{12.5, 18.5}, {12.5, 34.3}, {}}};
 double hot_us(int cfg, int64_t wgs, int64_t k) {
   const int64_t slots = kCUs * kRing[cfg].per_cu, rest = wgs % slots;
   const double kk = static_cast<double>(k) * 1e-3;
