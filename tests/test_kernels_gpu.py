@@ -1328,6 +1328,7 @@ def test_attention_finite_mask_values(kind, b, mq, sk, scale):
     if kind == "levels":
         mask[:, :, 30:] = -1e9          # later keys
         mask[:, :, :30] = f.min         # padding: rows with no visible key
+        mask[:, ::8, 30:] = f.min / 2   # (a level between the two)
         mask[:, 1::2, 5:9] = 0.0        # every other row sees some
     elif kind == "lowest":
         mask[:, :, :13] = f.min
@@ -1336,8 +1337,9 @@ def test_attention_finite_mask_values(kind, b, mq, sk, scale):
         mask[:, ::2, 11:17] = f.max
         mask[:, :, 40:] = f.min
     mask = mask.to(dtype)
-    want = O.attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), scale,
-                       mask=mask.float().numpy())
+    with np.errstate(over="ignore"):  # (lowest - largest)
+        want = O.attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), scale,
+                           mask=mask.float().numpy())
     qd, kd, vd, md = q.to(DEV), k.to(DEV), v.to(DEV), mask.to(DEV)
     nws = _capi.lib().sph_attention_workspace_bytes(b, mq, sk, mq * sk)
     ws = torch.full((max(nws, 16),), 255, dtype=torch.uint8, device=DEV)

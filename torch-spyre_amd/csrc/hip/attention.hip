@@ -526,11 +526,12 @@ attn_fwd_kernel(const AttnArgs p) {
     block_max();
     // Finite bf16 masks whose quotient overflows (the type's lowest value, with
     // which masks are often filled) became infinite.  Where that matters, in a
-    // row with no visible key yet or with a positive one, they become fp32's
-    // lowest (largest) value, beside which every score vanishes: rows with
-    // nothing else get uniform weights, as softmax over equal values does, and
-    // smaller masks (a causal fill of -1e9) keep their rank above.  (Clamped per
-    // element instead, blocks full of mask values took 6 % longer.)
+    // row with no visible key yet or with a positive one, they become the last
+    // quarter of fp32's range in their own order, where every score vanishes:
+    // rows with nothing else get uniform weights over the largest of them, as
+    // softmax does, and smaller masks (a causal fill of -1e9) keep their rank
+    // above.  (Clamped per element instead, blocks full of mask values took 6 %
+    // longer.)
     if constexpr (HUGE_MASK) {
       const bool huge = min(near2[0], near2[1]) < p.huge_n;
       const bool redo = mb == INFINITY || (mb == -INFINITY && !(r_ref >= -p.far_raw));
@@ -546,7 +547,7 @@ attn_fwd_kernel(const AttnArgs p) {
             if (!keep || fabsf(s[t][r]) != INFINITY) continue;
             const float v = Num<T>::to_f(mp[kx]);
             if (fabsf(v) < INFINITY && fabsf(v * p.inv_scale) == INFINITY)
-              s[t][r] = copysignf(3.402823466e38f, v);
+              s[t][r] = copysignf(fmaf(0.25f, fabsf(v), 2.55e38f), v);
           }
         block_max();
       }
