@@ -662,8 +662,9 @@ def test_gemm_bf16_and_unaligned_ld():
                                    (13, 33, 8), (16, 520, 136)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_gemm_small_m_weight_layout(m, n, k, dtype):
-    # decode-step shapes: x[M,K] @ W[N,K]^T, both K-contiguous (streaming
-    # small-M kernel), including K tails (k % 2048 != 0) and odd N
+    # decode-step shapes: x[M,K] @ W[N,K]^T, both K-contiguous (small-M and
+    # streaming kernels; 13 rows of one K chunk on the register-staged kernel, 16
+    # on the ring kernel), including K tails (k % 2048 != 0) and odd N
     _log(f"gemm small-M {m}x{n}x{k} {dtype}")
     X = uniform((m, k), k=11, dtype=dtype)
     W = (uniform((n, k), k=12) * 0.05).to(dtype)

@@ -174,8 +174,8 @@ __device__ inline float rounded_product(float a, float b) {
 constexpr uint8_t MB_ZERO = 0, MB_MIXED = 1, MB_NEGINF = 2;
 
 // One workgroup per (mask batch, row block, key block): class the block's
-// 128 x 64 mask values (rows past mq and keys past sk ignored).  The classes are read off the
-// 16-bit patterns (fp16 and bf16 alike: zero is +-0, -inf is one pattern), two
+// 128 x 64 mask values (rows past mq and keys past sk ignored).  The classes are
+// read off the 16-bit patterns (fp16 and bf16 alike: zero is +-0, -inf is one pattern), two
 // values per 32-bit word, and the workgroup's verdicts meet in one LDS word
 // per wave behind a single barrier.
 template <typename T>
@@ -822,7 +822,9 @@ extern "C" int sph_attention_fwd(sph_dtype dtype, int64_t batch, int64_t mq, int
                                  int64_t stride_m, int64_t causal_q, int64_t causal_off,
                                  float scale, void* o, int64_t ldo, int64_t stride_o,
                                  void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
-  return attention_run(false, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v, ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo, stride_o, workspace, workspace_bytes, stream);
+  return attention_run(false, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v,
+                       ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo,
+                       stride_o, workspace, workspace_bytes, stream);
 }
 
 extern "C" int sph_attention_fwd_rows(sph_dtype dtype, int64_t batch, int64_t mq, int64_t sk,
@@ -832,7 +834,9 @@ extern "C" int sph_attention_fwd_rows(sph_dtype dtype, int64_t batch, int64_t mq
                                  int64_t stride_m, int64_t causal_q, int64_t causal_off,
                                  float scale, void* o, int64_t ldo, int64_t stride_o,
                                  void* workspace, int64_t workspace_bytes, sph_stream_t stream) {
-  return attention_run(true, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v, ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo, stride_o, workspace, workspace_bytes, stream);
+  return attention_run(true, dtype, batch, mq, sk, head_dim, q, ldq, stride_q, k, ldk, stride_k, v,
+                       ldv, stride_v, mask, ldm, stride_m, causal_q, causal_off, scale, o, ldo,
+                       stride_o, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------
